@@ -254,13 +254,14 @@ class _Pinned:
 
 
 def _numbering(model):
-    """caller -> internal node numbers."""
+    """caller -> internal node numbers, and the same for the fields' entries."""
     perm = np.zeros(model.mesh.nb_nodes, dtype=np.int64)
     model.ctx.check(akx.lib.akx_node_numbering(model.ctx.h,
                                                perm.ctypes.data_as(ctypes.c_void_p)))
     inv = np.empty_like(perm)
     inv[perm] = np.arange(perm.size)
-    return torch.from_numpy(inv).cuda()
+    inv = torch.from_numpy(inv).cuda()
+    return inv, inv[:, None] * model.dim + torch.arange(model.dim, device="cuda")
 
 
 def _model(case, inp):
@@ -303,12 +304,12 @@ def _prepare_step(case, seed):
     model = _model(case, inp)
     if case["layout"] >= 0:
         model.set_launch(256, 256, 1, 1, case["layout"], 0)
-    inv = _numbering(model)
+    inv, entries = _numbering(model)
     start = {}
     for name, f in (("displacement", inp["u"]), ("velocity", inp["v"])):
         start[name] = torch.empty_like(_view(model, name))
         start[name][inv] = torch.from_numpy(np.ascontiguousarray(f)).cuda()
-    state = dict(case=case, model=model, inv=inv, start=start, damage=None,
+    state = dict(case=case, model=model, entries=entries, start=start, damage=None,
                  fields={n: _view(model, n) for n in ("displacement", "velocity", "acceleration")})
     if inp["Yd"] is not None:
         state["damage"] = _Pinned(*model.field_layout("damage"))
@@ -329,7 +330,7 @@ def _run_step(state):
     step = model.solve_step_graph if case["graph"] else model.solve_step
     for _ in range(case["steps"] // case["per_call"]):
         step(case["per_call"], precision)
-    out = {n: t.index_select(0, state["inv"]) for n, t in f.items()}
+    out = {n: t.take(state["entries"]) for n, t in f.items()}
     if state["damage"] is not None:
         model.wait(model.get_async("damage", state["damage"]))
         out["damage"] = state["damage"].tensor
