@@ -74,8 +74,10 @@ void free_derived(akx_ctx* c) {
   dfree(c->tab64_d);
   dfree(c->node_inv_d); dfree(c->elem_inv_d);
   dfree(c->fel_off); dfree(c->fel); dfree(c->flslot); dfree(c->fch_off); dfree(c->fcbase);
+  dfree(c->fblk); dfree(c->fhalo_off); dfree(c->fhalo); dfree(c->fsrec); dfree(c->fsmat);
   dfree(c->u_alt); dfree(c->pcoef); dfree(c->frec);
   c->fused_ok = false;
+  c->fused_default = false;
   c->patch_ok = false;
   dfree(c->slots); dfree(c->elem_mat_d); dfree(c->mats_d); dfree(c->damage); dfree(c->Yd);
   // one entry per material: sized by the material count at its first use
@@ -284,9 +286,13 @@ void to_internal_points(const akx_ctx* c, const T* src, T* dst, int comp) {
 
 // Step fused over node blocks (slot layout 6): one launch per step, no force
 // slots; stateless laws of a single kind on elements of up to 4 nodes, FP64
-// or mixed.
-bool uses_fused(const akx_ctx* c, int /*precision*/) {
-  return c->node_ordered == 6 && c->fused_ok && c->groups.size() == 1 && !c->groups[0].filter &&
+// or mixed.  The FP64 path takes it by default (fused_default): it gives the
+// slots' bits.
+bool uses_fused(const akx_ctx* c, int precision) {
+  const bool asked = c->layout_set ? c->node_ordered == 6
+                                   : precision == AKX_FP64 && c->fused_default;
+  return asked && c->fused_ok && (precision == AKX_MIXED || c->fsrec) &&
+         c->groups.size() == 1 && !c->groups[0].filter &&
          !(c->sur.enabled && c->groups[0].kind == AKX_MATERIAL_NEOHOOKEAN_DAMAGE);
 }
 
@@ -327,6 +333,7 @@ ElemArgs elem_args(akx_ctx* c, const KindGroup& g, int precision) {
   A.xcd_remap = c->xcd_remap;
   A.recompute = c->mixed_recompute;
   A.X = c->X;
+  A.safe_division = c->safe_division;
   A.slot_pos = !c->node_ordered ? nullptr : precision == AKX_MIXED ? c->slot2_pos : c->slot_pos;
   A.patch = (precision == AKX_MIXED && c->node_ordered >= 2 && c->patch_ok && !g.filter) ? 1 : 0;
   A.partials = (A.patch && uses_partials(c, precision)) ? (c->node_ordered == 3 ? 1 : 2) : 0;
@@ -595,29 +602,100 @@ int build_fused(akx_ctx* c, const std::vector<uint32_t>& order, const std::vecto
   if (n > 4 || int64_t(FUSED_CH) * n > 0xFFFF) return AKX_OK;
   std::vector<uint32_t> rank(E);  // assembly rank of each internal element
   for (int64_t r = 0; r < E; ++r) rank[c->elem_inv[order[r]]] = uint32_t(r);
-  const int64_t nblk = (N + FUSED_NB - 1) / FUSED_NB;
-  std::vector<uint32_t> el_off(nblk + 1, 0), ch_off(nblk + 1, 0), el;
-  std::vector<uint16_t> lslot, cbase;
-  std::vector<uint32_t> L;
-  std::vector<uint32_t> cnt, run;
-  for (int64_t b = 0; b < nblk; ++b) {
-    const int64_t n0 = b * FUSED_NB, n1 = std::min<int64_t>(N, n0 + FUSED_NB);
+  std::vector<uint32_t> conn(size_t(E) * n);  // internal, element-major
+  for (int64_t e = 0; e < E; ++e) {
+    const uint32_t* src = &c->hconn[size_t(c->elem_perm[e]) * n];
+    for (int a = 0; a < n; ++a) conn[size_t(e) * n + a] = c->node_inv[src[a]];
+  }
+  std::vector<uint32_t> erank(slot.size());  // of the CSR entries: element rank, local node
+  std::vector<uint8_t> local(slot.size());
+  for (size_t p = 0; p < slot.size(); ++p) {
+    const uint32_t e = slot[p] / uint32_t(n);
+    erank[p] = rank[e];
+    local[p] = uint8_t(slot[p] - e * uint32_t(n));
+  }
+  const bool several = c->mats.size() > 1;
+  std::vector<uint32_t> blk{0}, el_off, ch_off, halo_off, el, halo;
+  std::vector<uint16_t> lslot, cbase, smat;
+  std::vector<uint4> srec;
+  std::vector<uint32_t> L;      // ranks of the block's elements
+  std::vector<uint32_t> cnt, run, places;
+  std::vector<uint32_t> at(E);  // by rank: place in the current block's list
+  // block-local number of a node, valid for the list that stamped it
+  std::vector<uint32_t> loc(N), seen(N, 0);
+  uint32_t stamp = 0;
+  size_t lds_max = 0;
+  // Elements (by rank) of the nodes [n0, n1), where each node's run of each
+  // chunk starts, and the LDS the block takes with its nodes staged.
+  auto list = [&](int64_t n0, int64_t n1) -> size_t {
     L.clear();
-    for (int64_t k = n0; k < n1; ++k)
-      for (uint32_t p = off[k]; p < off[k + 1]; ++p) L.push_back(slot[p] / n);
-    std::sort(L.begin(), L.end(), [&](uint32_t x, uint32_t y) { return rank[x] < rank[y]; });
+    L.assign(erank.begin() + off[n0], erank.begin() + off[n1]);
+    std::sort(L.begin(), L.end());
     L.erase(std::unique(L.begin(), L.end()), L.end());
+    for (size_t j = 0; j < L.size(); ++j) at[L[j]] = uint32_t(j);
     const size_t nch = (L.size() + FUSED_CH - 1) / FUSED_CH;
-    auto pos = [&](uint32_t ei) {  // index of ei in L (sorted by rank)
-      return size_t(std::lower_bound(L.begin(), L.end(), ei,
-                                     [&](uint32_t x, uint32_t y) { return rank[x] < rank[y]; }) -
-                    L.begin());
-    };
     cnt.assign(nch * FUSED_NB, 0);
+    places.clear();  // of the nodes' entries, in CSR order
     for (int64_t k = n0; k < n1; ++k)
-      for (uint32_t p = off[k]; p < off[k + 1]; ++p)
-        cnt[(pos(slot[p] / n) / FUSED_CH) * FUSED_NB + size_t(k - n0)]++;
-    const size_t cb0 = cbase.size();
+      for (uint32_t p = off[k]; p < off[k + 1]; ++p) {
+        const uint32_t j = at[erank[p]];
+        places.push_back(j);
+        cnt[(j / FUSED_CH) * FUSED_NB + size_t(k - n0)]++;
+      }
+    size_t slots = 0;
+    for (size_t ch = 0; ch < nch; ++ch) {
+      size_t acc = 0;
+      for (int k = 0; k < FUSED_NB; ++k) acc += cnt[ch * FUSED_NB + k];
+      slots = std::max(slots, acc);
+    }
+    // block-local node numbers: the block's own, then the others in the order
+    // its elements meet them
+    ++stamp;
+    uint32_t others = 0;
+    for (uint32_t r : L) {
+      const uint32_t* v = &conn[size_t(c->elem_inv[order[r]]) * n];
+      for (int a = 0; a < n; ++a)
+        if (seen[v[a]] != stamp) {
+          seen[v[a]] = stamp;
+          const bool own = int64_t(v[a]) >= n0 && int64_t(v[a]) < n1;
+          loc[v[a]] = own ? uint32_t(v[a] - n0) : uint32_t(n1 - n0) + others++;
+        }
+    }
+    return ((size_t(n1 - n0) + others) * 2 + slots) * size_t(d) * 8;
+  };
+  // Small meshes take smaller blocks: a block's chunks follow one another, so
+  // that few large blocks leave most of the chip idle for the longest time
+  // (bar of 4,000 triangles: 7.1 us per step in 9 blocks of 256 nodes, 4.4 in
+  // 34 of 64).
+  const int64_t most = std::min<int64_t>(FUSED_NB, std::max<int64_t>(64, (N / 512 + 63) / 64 * 64));
+  bool staged = true;
+  int64_t next = most;  // what the last block took and a little more
+  for (int64_t n0 = 0; n0 < N;) {
+    int64_t n1 = std::min(N, n0 + next);
+    size_t lds = list(n0, n1);
+    while (staged && lds > FUSED_STAGED_LDS && n1 - n0 > FUSED_NB_MIN) {
+      // fewer nodes, by the LDS they take too much
+      const int64_t fit = int64_t(double(n1 - n0) * FUSED_STAGED_LDS / double(lds)) / 8 * 8;
+      n1 = n0 + std::max<int64_t>(FUSED_NB_MIN, std::min(fit, n1 - n0 - 8));
+      lds = list(n0, n1);
+    }
+    if (staged && lds > FUSED_STAGED_LDS) {
+      // no block small enough: start again without staging
+      staged = false;
+      n0 = 0;
+      next = most;
+      blk.assign(1, 0);
+      el_off.clear(); ch_off.clear(); halo_off.clear(); el.clear(); halo.clear();
+      lslot.clear(); cbase.clear(); smat.clear(); srec.clear();
+      continue;
+    }
+    next = std::min(most, n1 - n0 + 16);
+    lds_max = std::max(lds_max, lds);
+    blk.push_back(uint32_t(n1));
+    el_off.push_back(uint32_t(el.size()));
+    ch_off.push_back(uint32_t(cbase.size() / (FUSED_NB + 1)));
+    halo_off.push_back(uint32_t(halo.size()));
+    const size_t nch = cnt.size() / FUSED_NB, cb0 = cbase.size(), l0 = lslot.size();
     for (size_t ch = 0; ch < nch; ++ch) {
       uint32_t acc = 0;
       for (int k = 0; k < FUSED_NB; ++k) {
@@ -626,22 +704,41 @@ int build_fused(akx_ctx* c, const std::vector<uint32_t>& order, const std::vecto
       }
       cbase.push_back(uint16_t(acc));
     }
-    const size_t l0 = lslot.size();
     lslot.resize(l0 + L.size() * n, 0xFFFF);
     // each node's entries in CSR (assembly) order fill its run of each chunk
     run.assign(nch * FUSED_NB, 0);
+    size_t at_entry = 0;
     for (int64_t k = n0; k < n1; ++k)
       for (uint32_t p = off[k]; p < off[k + 1]; ++p) {
-        const uint32_t ei = slot[p] / n, a = slot[p] % n;
-        const size_t j = pos(ei), ch = j / FUSED_CH, kl = size_t(k - n0);
-        const uint32_t at = cbase[cb0 + ch * (FUSED_NB + 1) + kl] + run[ch * FUSED_NB + kl]++;
-        lslot[l0 + j * n + a] = uint16_t(at);
+        const size_t j = places[at_entry++], ch = j / FUSED_CH, kl = size_t(k - n0);
+        const uint32_t to = cbase[cb0 + ch * (FUSED_NB + 1) + kl] + run[ch * FUSED_NB + kl]++;
+        lslot[l0 + j * n + local[p]] = uint16_t(to);
       }
-    el.insert(el.end(), L.begin(), L.end());
-    el_off[b + 1] = uint32_t(el.size());
-    ch_off[b + 1] = ch_off[b] + uint32_t(nch);
+    const size_t h0 = halo.size();
+    for (size_t j = 0; j < L.size(); ++j) {
+      const uint32_t e = order[L[j]], ei = c->elem_inv[e];
+      el.push_back(ei);
+      if (!staged) continue;
+      uint32_t w[4] = {0, 0, 0, 0};
+      for (int a = 0; a < n; ++a) {
+        const uint32_t v = conn[size_t(ei) * n + a];
+        // the halo nodes' numbers ascend in the order they are met
+        if (loc[v] == uint32_t(n1 - n0) + uint32_t(halo.size() - h0)) halo.push_back(v);
+        w[a] = loc[v] | uint32_t(lslot[l0 + j * n + a]) << 16;
+      }
+      if (n == 3) w[3] = uint32_t(c->elem_mat[e]);
+      else if (several) smat.push_back(uint16_t(c->elem_mat[e]));
+      srec.push_back(make_uint4(w[0], w[1], w[2], w[3]));
+    }
+    n0 = n1;
   }
+  const int64_t nblk = int64_t(blk.size()) - 1;
+  el_off.push_back(uint32_t(el.size()));
+  ch_off.push_back(uint32_t(cbase.size() / (FUSED_NB + 1)));
+  halo_off.push_back(uint32_t(halo.size()));
   if (el.size() >= (size_t(1) << 32)) return AKX_OK;
+  HIP_TRY(c, dalloc(&c->fblk, blk.size()));
+  HIP_TRY(c, hipMemcpy(c->fblk, blk.data(), blk.size() * 4, hipMemcpyHostToDevice));
   HIP_TRY(c, dalloc(&c->fel_off, el_off.size()));
   HIP_TRY(c, dalloc(&c->fel, el.size()));
   HIP_TRY(c, dalloc(&c->flslot, lslot.size()));
@@ -655,7 +752,29 @@ int build_fused(akx_ctx* c, const std::vector<uint32_t>& order, const std::vecto
   HIP_TRY(c, hipMemcpy(c->fcbase, cbase.data(), cbase.size() * 2, hipMemcpyHostToDevice));
   c->fused_blocks = nblk;
   c->fused_elements = int64_t(el.size());
-  c->fused_lds = FUSED_CH * n * d * 8;
+  c->fused_lds = FUSED_CH * n * d * 4;  // the mixed step's FP32 contributions
+  if (staged) {
+    HIP_TRY(c, dalloc(&c->fhalo_off, halo_off.size()));
+    HIP_TRY(c, dalloc(&c->fhalo, halo.size()));
+    HIP_TRY(c, dalloc(&c->fsrec, srec.size()));
+    HIP_TRY(c, hipMemcpy(c->fhalo_off, halo_off.data(), halo_off.size() * 4, hipMemcpyHostToDevice));
+    if (!halo.empty())
+      HIP_TRY(c, hipMemcpy(c->fhalo, halo.data(), halo.size() * 4, hipMemcpyHostToDevice));
+    HIP_TRY(c, hipMemcpy(c->fsrec, srec.data(), srec.size() * 16, hipMemcpyHostToDevice));
+    if (!smat.empty()) {
+      HIP_TRY(c, dalloc(&c->fsmat, smat.size()));
+      HIP_TRY(c, hipMemcpy(c->fsmat, smat.data(), smat.size() * 2, hipMemcpyHostToDevice));
+    }
+    c->fused_staged_lds = int(lds_max);
+    // Against slots on layout 0 (us per step, slots / fused): 4,000 triangles
+    // 8.9 / 4.4, 1.6 M 62 / 31; 6,000 tetrahedra 17 / 9.0, 1.3 M 128 / 51,
+    // neo-Hookean 131 / 86, with a shuffled numbering kept (4 evaluations per
+    // element) 267 / 124.  A quadrangle's four points are dear to repeat:
+    // 800,000 take 52 / 44 at 1.19 evaluations per element, a shuffled
+    // 240,000 45 / 56 at 4, hence the line between them at the ratio where
+    // the former would break even.
+    c->fused_default = c->Q == 1 || double(el.size()) <= 1.4 * double(E);
+  }
   c->fused_ok = true;
   return AKX_OK;
 }
@@ -1055,8 +1174,8 @@ int akx_init(akx_ctx* c) {
   HIP_TRY(c, dalloc(&c->B64, bq)); HIP_TRY(c, dalloc(&c->B32, bq));
   HIP_TRY(c, dalloc(&c->J64, jq)); HIP_TRY(c, dalloc(&c->J32, jq));
   HIP_TRY(c, hipMalloc(&c->slots, std::max<size_t>(1, size_t(E) * dn) * sizeof(double)));
-  HIP_TRY(c, dalloc(&c->flag, 1));
-  HIP_TRY(c, hipMemset(c->flag, 0, sizeof(int)));
+  HIP_TRY(c, dalloc(&c->flag, 2));
+  HIP_TRY(c, hipMemset(c->flag, 0, 2 * sizeof(int)));
   c->partial_blocks = 4096;
   HIP_TRY(c, dalloc(&c->partial, size_t(c->partial_blocks)));
   HIP_TRY(c, dalloc(&c->scalar, 4));
@@ -1068,11 +1187,12 @@ int akx_init(akx_ctx* c) {
   HIP_TRY(c, dalloc(&c->tab64_d, 1));
   HIP_TRY(c, hipMemcpy(c->tab64_d, &tab, sizeof(ElemTables), hipMemcpyHostToDevice));
   HIP_TRY(c, launch_precompute(c->et, c->stream, E, N, c->X, c->conn_soa, tab, c->B64, c->J64,
-                               c->B32, c->J32, c->flag));
-  int bad = 0;
-  HIP_TRY(c, hipMemcpyAsync(&bad, c->flag, sizeof(int), hipMemcpyDeviceToHost, c->stream));
+                               c->B32, c->J32, c->flag, c->flag + 1));
+  int bad[2] = {0, 0};
+  HIP_TRY(c, hipMemcpyAsync(bad, c->flag, sizeof bad, hipMemcpyDeviceToHost, c->stream));
   HIP_TRY(c, hipStreamSynchronize(c->stream));
-  if (bad)
+  c->safe_division = !bad[1];
+  if (bad[0])
     return fail(c, AKX_ERR_JACOBIAN,
                 "Negative jacobian computed, possible problem in the element node ordering");
   HIP_TRY(c, launch_mass(c->et, c->stream, N, E, c->mass_off, c->mass_slot, tab, c->J64,
@@ -1411,7 +1531,9 @@ int enqueue_steps(akx_ctx* c, int nsteps, int precision, bool timing) {
   {
     NodeArgs A = node_args(c, NODE_PREDICT | (nsteps == 1 ? NODE_SAVE_PREV : 0) | position,
                            precision);
-    if (position) {
+    // an odd number of fused FP64 steps starts from the other buffer too, so
+    // that the displacement ends in c->u
+    if (position || (uses_fused(c, precision) && (nsteps & 1))) {
       A.u_out = c->u_alt;
       std::swap(ucur, uprev);
     }
@@ -1441,9 +1563,14 @@ int enqueue_steps(akx_ctx* c, int nsteps, int precision, bool timing) {
       // coordinates gathered through element ids (0): the same forces bit
       // for bit
       F.rec = c->mixed_recompute ? c->frec : nullptr;
+      F.blk = c->fblk;
+      F.halo_off = c->fhalo_off;
+      F.halo = c->fhalo;
+      F.srec = c->fsrec;
+      F.smat = c->fsmat;
       F.nblk = c->fused_blocks;
-      HIP_TRY(c, launch_fused(c->et, g.kind, precision, c->mixed_recompute != 0, c->has_fext,
-                              c->stream, EA, NA, F, c->fused_lds));
+      HIP_TRY(c, launch_fused(c->et, g.kind, precision, c->has_fext, c->stream, EA, NA, F,
+                              precision == AKX_MIXED ? c->fused_lds : c->fused_staged_lds));
       if (timing) {
         HIP_TRY(c, hipEventRecord(c->pool[2 * s - 1], c->stream));
         HIP_TRY(c, hipEventRecord(c->pool[2 * s], c->stream));
@@ -1518,7 +1645,7 @@ int akx_solve_step_graph(akx_ctx* c, int nsteps, int precision) {
   akx_ctx::GraphKey k;
   k.nsteps = nsteps; k.precision = precision;
   k.eb = c->elem_block; k.nb = c->node_block; k.x = c->xcd_remap; k.rc = c->mixed_recompute;
-  k.lay = c->node_ordered; k.stage = c->node_stage;
+  k.lay = c->layout_set ? c->node_ordered : -1; k.stage = c->node_stage;
   k.fext = c->has_fext; k.bc = c->has_bc_inc; k.dt = c->dt;
   for (int i = 0; i < 3; ++i) k.bc_inc[i] = c->bc_inc[i];
   k.dt_node = c->dt_node;
@@ -1689,6 +1816,8 @@ int akx_query(akx_ctx* c, const char* key, double* value) {
   else if (k == "patch_available") *value = c->patch_ok ? 1. : 0.;
   else if (k == "patch_packed") *value = (c->patch_ok && c->lcr) ? 1. : 0.;
   else if (k == "fused_available") *value = c->fused_ok ? 1. : 0.;
+  else if (k == "fused_blocks") *value = double(c->fused_ok ? c->fused_blocks : 0);
+  else if (k == "fused_staged_lds") *value = double(c->fsrec ? c->fused_staged_lds : 0);
   else if (k == "fused_records") *value = c->frec ? 1. : 0.;
   else if (k == "fused_elements") *value = double(c->fused_ok ? c->fused_elements : 0);
   else if (k == "element_block") *value = c->elem_block;
@@ -1887,6 +2016,7 @@ int akx_autotune(akx_ctx* c, int precision, int nsteps, int* chosen, double* bes
   float best_t = std::numeric_limits<float>::max();
   const bool was_timing = c->timing;
   c->timing = false;
+  c->layout_set = true;  // each candidate names its layout, and so does the choice
   // candidates: slot layout x node staging x table/recompute x XCD mapping x block sizes
   struct Shape { int eb, nb, x, rcmp, lay, stage; };
   std::vector<Shape> cand;
@@ -1905,11 +2035,11 @@ int akx_autotune(akx_ctx* c, int precision, int nsteps, int* chosen, double* bes
               cand.push_back(Shape{eb, nb, x, rcmp, lay, stage});
             }
           }
-  // the fused step (layout 6) has its own block shapes; on the mixed path it
-  // rebuilds B, from per-evaluation records (mixed_recompute 1, triangles)
+  // the fused step (layout 6) has its own block shapes and rebuilds B; on the
+  // mixed path from per-evaluation records (mixed_recompute 1, triangles)
   // or from coordinates gathered through element ids (0)
   if (c->fused_ok)
-    for (int rcmp = (precision == AKX_MIXED && !c->frec ? 1 : 0); rcmp < 2; ++rcmp)
+    for (int rcmp = (precision == AKX_MIXED && c->frec ? 0 : 1); rcmp < 2; ++rcmp)
       for (int x = 0; x < 2; ++x) cand.push_back(Shape{256, 256, x, rcmp, 6, 0});
   for (const Shape& sh : cand) {
           const int eb = sh.eb, nb = sh.nb, x = sh.x, lay = sh.lay;
@@ -1956,7 +2086,10 @@ int akx_set_launch(akx_ctx* c, int element_block, int node_block, int xcd_remap,
   if (node_block) c->node_block = node_block;
   if (xcd_remap >= 0) c->xcd_remap = xcd_remap ? 1 : 0;
   if (mixed_recompute >= 0) c->mixed_recompute = mixed_recompute ? 1 : 0;
-  if (slot_layout >= 0) c->node_ordered = slot_layout;
+  if (slot_layout >= 0) {
+    c->node_ordered = slot_layout;
+    c->layout_set = true;
+  }
   if (node_stage >= 0) c->node_stage = node_stage ? 1 : 0;
   return AKX_OK;
 }

@@ -101,6 +101,35 @@ __device__ __forceinline__ void matrixt_matrix(const double* A, const double* B,
     }
 }
 
+// The same sums, in the same order, for the force path: each starts at its
+// first product instead of at +0, one FP64 add less per entry.  Only the sign
+// of a zero entry can differ, and the nodes' force sums, which start at +0,
+// do not see it.
+template <int im, int in, int ik>
+__device__ __forceinline__ void force_product(const double* A, const double* B, double* C) {
+#pragma unroll
+  for (int j = 0; j < in; ++j)
+#pragma unroll
+    for (int i = 0; i < im; ++i) {
+      double s = A[i] * B[j * ik];
+#pragma unroll
+      for (int l = 1; l < ik; ++l) s += A[i + l * im] * B[l + j * ik];
+      C[i + j * im] = s;
+    }
+}
+template <int im, int in, int ik>
+__device__ __forceinline__ void force_productt(const double* A, const double* B, double* C) {
+#pragma unroll
+  for (int j = 0; j < in; ++j)
+#pragma unroll
+    for (int i = 0; i < im; ++i) {
+      double s = A[i] * B[j];
+#pragma unroll
+      for (int l = 1; l < ik; ++l) s += A[i + l * im] * B[j + l * in];
+      C[i + j * im] = s;
+    }
+}
+
 template <typename T> __device__ __forceinline__ T det2(const T* m) { return m[0] * m[3] - m[1] * m[2]; }
 template <typename T> __device__ __forceinline__ T det3(const T* m) {
   return m[0] * (m[4] * m[8] - m[7] * m[5]) - m[3] * (m[1] * m[8] - m[7] * m[2]) +
@@ -127,6 +156,71 @@ template <int d, typename T> __device__ __forceinline__ void invn(const T* m, T*
   }
 }
 
+// Quotients by one divisor: 1/b refined once from the hardware's estimate (two
+// Newton steps), then per quotient q = a y and the remainder step
+// q + (a - b q) y, which rounds like the division (Markstein, IBM J. Res. Dev.
+// 34, 1990) as long as nothing on the way leaves the normal range -- the
+// caller knows: |b| in 2^+-SAFE_DIVISOR, a zero or in 2^+-SAFE_NUMERATOR.
+// Three operations a quotient instead of the compiler's eleven, which carry
+// scalings for the extremes.
+constexpr int SAFE_DIVISOR = 300, SAFE_NUMERATOR = 600;
+struct Divisor {
+  double b, y;
+  __device__ __forceinline__ explicit Divisor(double d) : b(d) {
+    y = __builtin_amdgcn_rcp(b);
+    y = __builtin_fma(y, __builtin_fma(-b, y, 1.), y);
+    y = __builtin_fma(y, __builtin_fma(-b, y, 1.), y);
+  }
+  __device__ __forceinline__ double operator()(double a) const {
+    const double q = a * y;
+    return __builtin_fma(__builtin_fma(-b, q, a), y, q);
+  }
+};
+__host__ __device__ inline bool safe_magnitude(double x, int e) {
+  const double m = x < 0 ? -x : x;
+  return m >= __builtin_ldexp(1., -e) && m <= __builtin_ldexp(1., e);
+}
+
+// Adjugate (invn's numerators, column-major) and determinant.  det3's
+// cofactors are the adjugate's first column (one of them with the opposite
+// sign, exactly), so the determinant costs five operations more, with det3's
+// bits.
+template <int d>
+__device__ __forceinline__ double adjugate(const double* m, double* r) {
+  if constexpr (d == 2) {
+    r[0] = m[3]; r[1] = -m[1]; r[2] = -m[2]; r[3] = m[0];
+    return det2(m);
+  } else {
+    r[0] = m[4] * m[8] - m[7] * m[5];
+    r[1] = m[2] * m[7] - m[8] * m[1];
+    r[2] = m[1] * m[5] - m[4] * m[2];
+    r[3] = m[5] * m[6] - m[8] * m[3];
+    r[4] = m[0] * m[8] - m[6] * m[2];
+    r[5] = m[2] * m[3] - m[5] * m[0];
+    r[6] = m[3] * m[7] - m[6] * m[4];
+    r[7] = m[1] * m[6] - m[7] * m[0];
+    r[8] = m[0] * m[4] - m[3] * m[1];
+    return m[0] * r[0] + m[3] * r[1] + m[6] * r[2];
+  }
+}
+
+// Inverse (invn) and determinant for the force path; `safe`: every numerator
+// and determinant of the mesh is in Divisor's range (k_precompute looks).
+template <int d>
+__device__ __forceinline__ double inv_det(const double* m, bool safe, double* r) {
+  double n[d * d];
+  const double dd = adjugate<d>(m, n);
+  if (safe) {
+    const Divisor by(dd);
+#pragma unroll
+    for (int k = 0; k < d * d; ++k) r[k] = by(n[k]);
+  } else {
+#pragma unroll
+    for (int k = 0; k < d * d; ++k) r[k] = n[k] / dd;
+  }
+  return dd;
+}
+
 // MaterialElastic::computeStressOnQuad (material_elastic_inline_impl.hh:41-55)
 template <int d>
 __device__ __forceinline__ void elastic_stress_ref(const MatParams& m, const double* G, double* S) {
@@ -139,6 +233,25 @@ __device__ __forceinline__ void elastic_stress_ref(const MatParams& m, const dou
     for (int j = 0; j < d; ++j) {
       double v = (i == j) ? m.lambda * trace : 0.;
       S[i + j * d] = v + m.mu * (G[i + j * d] + G[j + i * d]);
+    }
+}
+
+// The same stress for the force path (see force_product): the off-diagonal
+// entries once each -- G_ij + G_ji and G_ji + G_ij round alike -- and without
+// their leading + 0.
+template <int d>
+__device__ __forceinline__ void elastic_stress_force(const MatParams& m, const double* G,
+                                                     double* S) {
+  double trace = G[0];
+#pragma unroll
+  for (int i = 1; i < d; ++i) trace += G[i + i * d];
+#pragma unroll
+  for (int i = 0; i < d; ++i)
+#pragma unroll
+    for (int j = 0; j <= i; ++j) {
+      const double v = m.mu * (G[i + j * d] + G[j + i * d]);
+      if (i == j) S[i + i * d] = m.lambda * trace + v;
+      else S[i + j * d] = S[j + i * d] = v;
     }
 }
 
@@ -200,8 +313,9 @@ __device__ __forceinline__ void nh_damage_stress_ref(const MatParams& m, const d
 // (material.cc:689-706), VoigtHelper::transferBMatrixToSymVoigtBMatrix
 // (aka_voigthelper_tmpl.hh:104-143), transferBMatrixToBL2 (:177-226), Voigt
 // order xx, yy, zz, yz, xz, xy (aka_voigthelper.cc:52-61).  The entries of the
-// dense 6 x 3n matrices are formed exactly as the reference forms them, then
-// contracted with S in the order of Math::matrixt_matrix.
+// dense 6 x 3n matrices are formed as the reference forms them, then contracted
+// with S in the order of Math::matrixt_matrix; additions of an exact zero are
+// left out (see force_product).
 template <int d, int n>
 __device__ __forceinline__ void finite_residual_ref(const double* B, const double* G,
                                                     const double* S, double* r) {
@@ -217,35 +331,29 @@ __device__ __forceinline__ void finite_residual_ref(const double* B, const doubl
 #pragma unroll
         for (int I = 0; I < 3; ++I) {
           double bl2 = Gm(k, I) * Bm(I, a);
-          bt[I] = (k == I) ? Bm(I, a) + bl2 : 0. + bl2;
+          bt[I] = (k == I) ? Bm(I, a) + bl2 : bl2;
         }
         // I = 3 (yz): sym (k=1: dndz, k=2: dndy); BL2 += G(k,1) B(2,a); += G(k,2) B(1,a)
         {
-          double bl2 = 0.;
-          bl2 += Gm(k, 1) * Bm(2, a);
+          double bl2 = Gm(k, 1) * Bm(2, a);
           bl2 += Gm(k, 2) * Bm(1, a);
-          double sym = (k == 1) ? Bm(2, a) : (k == 2) ? Bm(1, a) : 0.;
-          bt[3] = sym + bl2;
+          bt[3] = (k == 1) ? Bm(2, a) + bl2 : (k == 2) ? Bm(1, a) + bl2 : bl2;
         }
         // I = 4 (xz): sym (k=0: dndz, k=2: dndx); BL2 += G(k,0) B(2,a); += G(k,2) B(0,a)
         {
-          double bl2 = 0.;
-          bl2 += Gm(k, 0) * Bm(2, a);
+          double bl2 = Gm(k, 0) * Bm(2, a);
           bl2 += Gm(k, 2) * Bm(0, a);
-          double sym = (k == 0) ? Bm(2, a) : (k == 2) ? Bm(0, a) : 0.;
-          bt[4] = sym + bl2;
+          bt[4] = (k == 0) ? Bm(2, a) + bl2 : (k == 2) ? Bm(0, a) + bl2 : bl2;
         }
         // I = 5 (xy): sym (k=0: dndy, k=1: dndx); BL2 += G(k,0) B(1,a); += G(k,1) B(0,a)
         {
-          double bl2 = 0.;
-          bl2 += Gm(k, 0) * Bm(1, a);
+          double bl2 = Gm(k, 0) * Bm(1, a);
           bl2 += Gm(k, 1) * Bm(0, a);
-          double sym = (k == 0) ? Bm(1, a) : (k == 1) ? Bm(0, a) : 0.;
-          bt[5] = sym + bl2;
+          bt[5] = (k == 0) ? Bm(1, a) + bl2 : (k == 1) ? Bm(0, a) + bl2 : bl2;
         }
-        double s = 0.;
+        double s = bt[0] * Sv[0];
 #pragma unroll
-        for (int I = 0; I < 6; ++I) s += bt[I] * Sv[I];
+        for (int I = 1; I < 6; ++I) s += bt[I] * Sv[I];
         r[3 * a + k] = s;
       }
   } else {
@@ -258,16 +366,15 @@ __device__ __forceinline__ void finite_residual_ref(const double* B, const doubl
 #pragma unroll
         for (int I = 0; I < 2; ++I) {
           double bl2 = Gm(k, I) * Bm(I, a);
-          bt[I] = (k == I) ? Bm(I, a) + bl2 : 0. + bl2;
+          bt[I] = (k == I) ? Bm(I, a) + bl2 : bl2;
         }
-        double bl2 = 0.;
-        bl2 += Gm(k, 0) * Bm(1, a);
+        double bl2 = Gm(k, 0) * Bm(1, a);
         bl2 += Gm(k, 1) * Bm(0, a);
         double sym = (k == 0) ? Bm(1, a) : Bm(0, a);
         bt[2] = sym + bl2;
-        double s = 0.;
+        double s = bt[0] * Sv[0];
 #pragma unroll
-        for (int I = 0; I < 3; ++I) s += bt[I] * Sv[I];
+        for (int I = 1; I < 3; ++I) s += bt[I] * Sv[I];
         r[2 * a + k] = s;
       }
   }

@@ -45,6 +45,7 @@ struct ElemArgs {
   int xcd_remap;
   int recompute;             // mixed path: rebuild B, det(J) w from X
   const double* X;           // (N, d) reference coordinates
+  bool safe_division;        // the Jacobians suit Divisor (k_precompute)
   const uint32_t* slot_pos;  // [a][E] CSR position of (e, a); nullptr = element-ordered slots
   // LDS-patch variant of the mixed kernel (k_element_patch)
   int patch;                 // 1: use it
@@ -102,11 +103,12 @@ struct NodeArgs {
   int partials;           // slots are per-patch partial sums, 1 FP64, 2 FP32 (csr_off/csr_slot: node -> entries)
 };
 
-// Fused FP64 step over node blocks (stateless laws, slot layout 6): block b
-// owns nodes [b * FUSED_NB, (b + 1) * FUSED_NB) and recomputes the elements
+// Fused step over node blocks (stateless laws, slot layout 6): block b owns
+// the nodes [blk[b], blk[b + 1]), at most FUSED_NB, and recomputes the elements
 // around them in chunks of FUSED_CH, in the reference's assembly order.
 constexpr int FUSED_NB = 256, FUSED_CH = 256;
 struct FusedArgs {
+  const uint32_t* blk;     // [nblk + 1] first node of each block
   const uint32_t* el_off;  // [nblk + 1] offsets into el
   const uint32_t* el;      // internal element ids of each block, assembly order
   const uint16_t* lslot;   // [j * n + a] LDS slot of (element j, node a); 0xFFFF: not a block node
@@ -118,8 +120,22 @@ struct FusedArgs {
   // gathers instead): rec[2 j] = the element's coordinate differences
   // x_a - x_0, a = 1, 2 (4 FP32); rec[2 j + 1] = fused_record_ids(...)
   const uint4* rec;
+  // FP64 path, nodes staged in LDS: the nodes beyond its own that a block's
+  // elements touch, and per evaluation one word per node, block-local number (own nodes first, then the halo) |
+  // LDS slot << 16 (0xFFFF: not a block node); the fourth word of a triangle
+  // is its material, larger elements have it in smat (several materials)
+  const uint32_t* halo_off;  // [nblk + 1] offsets into halo
+  const uint32_t* halo;
+  const uint4* srec;
+  const uint16_t* smat;
   int64_t nblk;
 };
+// LDS a staged block of the fused FP64 step may take: four blocks of 256
+// threads per CU (160 KB).  A block owns as many nodes as fit, at least
+// FUSED_NB_MIN (a mesh that needs more LDS even so, for a node in thousands of
+// elements, runs on slots).
+constexpr size_t FUSED_STAGED_LDS = 40 * 1024 - 512;
+constexpr int64_t FUSED_NB_MIN = 32;
 
 // Second word of a fused triangle record: the three node ids in the low 23
 // bits of x, y, z; LDS slots 0 and 1 in w (16 bits each, 0xFFFF: not a block
@@ -179,15 +195,15 @@ hipError_t launch_sur_mlp(hipStream_t s, const void* img, const float* imgb, boo
 // Launchers (akx_kernels.hip).  All enqueue on `stream` and return the launch status.
 hipError_t launch_precompute(int et, hipStream_t s, int64_t E, int64_t N, const double* X,
                              const uint32_t* conn_soa, const ElemTables& tab, double* B64,
-                             double* J64, float* B32, float* J32, int* bad_jacobian);
+                             double* J64, float* B32, float* J32, int* bad_jacobian,
+                             int* unsafe_division);
 hipError_t launch_mass(int et, hipStream_t s, int64_t N, int64_t E, const uint32_t* off,
                        const uint32_t* slot, const ElemTables& tab, const double* J64,
                        const uint16_t* elem_mat, const MatParams* mats, double* mass);
 hipError_t launch_element(int et, int kind, int precision, hipStream_t s, const ElemArgs& A,
                           int block);
-hipError_t launch_fused(int et, int kind, int precision, bool recompute, bool has_fext,
-                        hipStream_t s, const ElemArgs& EA, const NodeArgs& NA, const FusedArgs& F,
-                        int lds);
+hipError_t launch_fused(int et, int kind, int precision, bool has_fext, hipStream_t s,
+                        const ElemArgs& EA, const NodeArgs& NA, const FusedArgs& F, int lds);
 hipError_t launch_node(int d, int precision, bool has_fext, hipStream_t s, const NodeArgs& A,
                        int block);
 hipError_t launch_fused_records(hipStream_t s, int64_t J, int64_t E, const uint32_t* el,
@@ -355,7 +371,8 @@ struct akx_ctx {
   double* gradu = nullptr;
   double* stress = nullptr;
   double* work = nullptr;  // N*d scratch (current position)
-  int* flag = nullptr;
+  int* flag = nullptr;       // negative Jacobian, Jacobian out of Divisor's range
+  bool safe_division = false;
 
   bool has_fext = false;
   bool has_bc_inc = false;
@@ -366,6 +383,10 @@ struct akx_ctx {
 
   int elem_block = 256, node_block = 256, xcd_remap = 1, mixed_recompute = 1;
   int node_ordered = 0;             // slot layout (see store_slots)
+  // set by akx_set_launch or the autotuner; until then the FP64 path takes the
+  // fused step wherever it applies (the same bits as the element-ordered slots
+  // of layout 0, the mixed path's default)
+  bool layout_set = false;
   int node_stage = 1;               // node kernel copies its slot range to LDS when it fits
   uint32_t span_max[4] = {0, 0, 0, 0};  // largest slot range of a node block of 64, 128, 192, 256
   uint32_t* slot_pos = nullptr;     // [a][E] CSR position of (e, a)
@@ -386,6 +407,13 @@ struct akx_ctx {
   int64_t fused_blocks = 0, fused_elements = 0;
   uint32_t *fel_off = nullptr, *fel = nullptr, *fch_off = nullptr;
   uint16_t *flslot = nullptr, *fcbase = nullptr;
+  // its FP64 form: halo nodes and element records (nullptr: too many nodes);
+  // fused_default: the FP64 path takes it when no layout is set
+  bool fused_default = false;
+  int fused_staged_lds = 0;
+  uint32_t *fblk = nullptr, *fhalo_off = nullptr, *fhalo = nullptr;
+  uint4* fsrec = nullptr;
+  uint16_t* fsmat = nullptr;
   double* u_alt = nullptr;  // second displacement buffer (position form, fused step)
   double* pcoef = nullptr;  // position form: dt^2 / M per node
   uint4* frec = nullptr;     // per-evaluation records of the fused mixed step (triangles)

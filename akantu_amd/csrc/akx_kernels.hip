@@ -35,6 +35,42 @@ __device__ __forceinline__ double point_shapes_ref(const ElemTables& tab, int q,
   return detn<d>(J) * tab.w[q];
 }
 
+// The same for the force path: the values of point_shapes_ref up to the sign of
+// zeros (see force_product).  On simplices dN/dxi holds only -1, 0 and 1 (node
+// 0 is the vertex the natural coordinates start from), whose products are
+// exact, so the Jacobian is a difference per entry and B a copy of its inverse
+// (node 0: minus the row's sum, in the order of the product).
+template <int ET>
+__device__ __forceinline__ double point_shapes_force(const ElemTables& tab, bool safe, int q,
+                                                     const double* xe, double* B) {
+  using T = Elem<ET>;
+  constexpr int d = T::d, n = T::n;
+  double J[d * d], Ji[d * d];
+  if constexpr (n == d + 1) {
+#pragma unroll
+    for (int j = 0; j < d; ++j)
+#pragma unroll
+      for (int i = 0; i < d; ++i) J[i + j * d] = xe[j + (i + 1) * d] - xe[j];
+  } else {
+    force_productt<d, d, n>(tab.dnds[q], xe, J);
+  }
+  const double det = inv_det<d>(J, safe, Ji);
+  if constexpr (n == d + 1) {
+#pragma unroll
+    for (int i = 0; i < d; ++i) {
+      double s = -Ji[i];
+#pragma unroll
+      for (int l = 1; l < d; ++l) s -= Ji[i + l * d];
+      B[i] = s;
+#pragma unroll
+      for (int a = 1; a < n; ++a) B[i + a * d] = Ji[i + (a - 1) * d];
+    }
+  } else {
+    force_product<d, n, d>(Ji, tab.dnds[q], B);
+  }
+  return det * tab.w[q];
+}
+
 // ===========================================================================
 // precompute: B = J^{-1} dN/dxi and det(J) w
 //   ShapeLagrange::computeShapeDerivativesOnIntegrationPoints
@@ -47,7 +83,7 @@ __global__ void __launch_bounds__(256) k_precompute(int64_t E, const double* __r
                                                     const uint32_t* __restrict__ conn, ElemTables tab,
                                                     double* __restrict__ B64, double* __restrict__ J64,
                                                     float* __restrict__ B32, float* __restrict__ J32,
-                                                    int* bad) {
+                                                    int* bad, int* unsafe) {
   using T = Elem<ET>;
   constexpr int d = T::d, n = T::n, Q = T::Q, dn = d * n;
   const int64_t e = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -71,6 +107,14 @@ __global__ void __launch_bounds__(256) k_precompute(int64_t E, const double* __r
     J64[int64_t(q) * E + e] = jw;
     J32[int64_t(q) * E + e] = float(jw);
     if (jw < 0) *bad = 1;
+    // whether the force path may divide by its Jacobians with Divisor
+    double J[d * d], num[d * d];
+    matrix_matrixt<d, d, n>(tab.dnds[q], xe, J);
+    bool safe = safe_magnitude(adjugate<d>(J, num), SAFE_DIVISOR);
+#pragma unroll
+    for (int k = 0; k < d * d; ++k)
+      safe = safe && (num[k] == 0. || safe_magnitude(num[k], SAFE_NUMERATOR));
+    if (!safe) *unsafe = 1;
   }
 }
 
@@ -174,23 +218,25 @@ __device__ __forceinline__ void element_forces_fp64(const ElemArgs& A, int64_t e
   const double* __restrict__ Jt = static_cast<const double*>(A.J);
 #pragma unroll
   for (int k = 0; k < dn; ++k) fe[k] = 0.;
-#pragma unroll
+  // rolled: unrolled, the four points of a quadrangle took 141 registers
+#pragma unroll 1
   for (int q = 0; q < Q; ++q) {
     double Bq[dn];
-    double jq_rc = 0.;
+    double jq;
     if constexpr (RECOMPUTE) {
-      jq_rc = point_shapes_ref<ET>(*A.tab64, q, xe, Bq);
+      jq = point_shapes_force<ET>(*A.tab64, A.safe_division, q, xe, Bq);
     } else {
 #pragma unroll
       for (int k = 0; k < dn; ++k) Bq[k] = Bt[(int64_t(q) * dn + k) * E + e];
+      jq = Jt[int64_t(q) * E + e];
     }
     double G[d * d], S[d * d], R[dn];
     // grad u = u_e B^T (shape_functions_inline_impl.hh:388, Matrix::mul<false, true>)
-    matrix_matrixt<d, d, n>(ue, Bq, G);
+    force_productt<d, d, n>(ue, Bq, G);
     if constexpr (KIND == ELASTIC) {
-      elastic_stress_ref<d>(m, G, S);
+      elastic_stress_force<d>(m, G, S);
       // B^T sigma computed as sigma B (shape_lagrange_inline_impl.hh:421)
-      matrix_matrix<d, n, d>(S, Bq, R);
+      force_product<d, n, d>(S, Bq, R);
     } else {
       if constexpr (KIND == NEOHOOKEAN) {
         neohookean_stress_ref<d>(m, G, S);
@@ -203,9 +249,8 @@ __device__ __forceinline__ void element_forces_fp64(const ElemArgs& A, int64_t e
       finite_residual_ref<d, n>(Bq, G, S, R);
     }
     // IntegratorGauss::integrate (integrator_gauss_inline_impl.hh:446-452)
-    const double jq = RECOMPUTE ? jq_rc : Jt[int64_t(q) * E + e];
 #pragma unroll
-    for (int k = 0; k < dn; ++k) fe[k] += R[k] * jq;
+    for (int k = 0; k < dn; ++k) fe[k] = Q == 1 ? R[k] * jq : fe[k] + R[k] * jq;
   }
 }
 
@@ -1636,68 +1681,121 @@ __global__ void __launch_bounds__(256) k_node(NodeArgs A) {
 //   computed by every block they touch; no force slot goes through HBM.
 //   u is read from NodeArgs::u and written to FusedArgs::u_out: other blocks
 //   still read the old displacements while this one updates its nodes.
+//   The block first copies u and X of its own nodes and of the others its
+//   elements touch into LDS, and an element is one 16-byte record of
+//   block-local node numbers and force slots: gathered from global memory,
+//   the 2 d n doubles of every element were 64 scattered 8-byte reads per load
+//   instruction and set the step's time.
+//   Bound: FP64 instructions and LDS about equally.  Cube of 6 M tetrahedra,
+//   per step: 288 us gathering, 205 staged, 183 with the quotients by one
+//   divisor (Divisor; 170 in a graph), where two blocks more per CU matter as
+//   much as fewer repeated elements: 240 us with 54 KB of LDS a block (9.8 M
+//   evaluations), 183 with 40 KB (10.3 M), 199 with 32 KB (11.2 M).
 // ===========================================================================
-template <int ET, int KIND, bool RECOMPUTE, bool HAS_FEXT>
+template <int ET, int KIND, bool HAS_FEXT>
 __global__ void __launch_bounds__(256) k_step_fused(ElemArgs EA, NodeArgs NA, FusedArgs F) {
   static_assert(KIND != NH_DAMAGE, "the fused step recomputes elements: stateless laws only");
   static_assert(FUSED_NB <= 256 && FUSED_CH == 256, "one node and one element per thread of 256");
   using T = Elem<ET>;
   constexpr int d = T::d, n = T::n, dn = d * n;
   extern __shared__ __align__(16) unsigned char smem[];
-  double* s_f = reinterpret_cast<double*>(smem);  // FUSED_CH * n contributions, d each
   const int64_t b = logical_block(NA.xcd_remap);
   if (b >= F.nblk) return;  // uniform over the block
   const int t = threadIdx.x;
-  const int64_t n0 = b * FUSED_NB;
-  const int cnt = int(min<int64_t>(FUSED_NB, NA.N - n0));
+  const int64_t n0 = F.blk[b];
+  const int cnt = int(F.blk[b + 1] - n0);
   const bool owner = t < cnt;
   const int64_t node = n0 + t;
-  const int64_t E = EA.E;
   const double* __restrict__ u_in = NA.u;
   double f[d];
 #pragma unroll
   for (int i = 0; i < d; ++i) f[i] = 0.;
   const uint32_t j0 = F.el_off[b], j1 = F.el_off[b + 1];
   const uint32_t c0 = F.ch_off[b];
+  // the first elements' records travel with the nodes
+  uint4 rec = make_uint4(0, 0, 0, 0);
+  if (j0 + uint32_t(t) < j1) rec = F.srec[j0 + uint32_t(t)];
+  const uint32_t h0 = F.halo_off[b];
+  const int total = cnt + int(F.halo_off[b + 1] - h0);
+  // u and X of the staged nodes, 2 d doubles each, then the contributions of
+  // a chunk, d each
+  double* s_n = reinterpret_cast<double*>(smem);
+  double* s_f = s_n + size_t(total) * 2 * d;
+  for (int k = t; k < total; k += 256) {
+    const int64_t nd = k < cnt ? n0 + k : int64_t(F.halo[h0 + uint32_t(k - cnt)]);
+    double v[2 * d];
+#pragma unroll
+    for (int i = 0; i < d; ++i) {
+      v[i] = u_in[nd * d + i];
+      v[d + i] = EA.X[nd * d + i];
+    }
+    double2* dst = reinterpret_cast<double2*>(s_n + size_t(k) * 2 * d);
+#pragma unroll
+    for (int i = 0; i < d; ++i) dst[i] = make_double2(v[2 * i], v[2 * i + 1]);
+  }
+  __syncthreads();
   uint32_t c = 0;
   for (uint32_t jc = j0; jc < j1; jc += FUSED_CH, ++c) {
     const uint32_t j = jc + uint32_t(t);
+    // where the node's run of this chunk lies, needed after the barrier
+    int q0 = 0, q1 = 0;
+    if (owner) {
+      const uint16_t* cb = F.cbase + size_t(c0 + c) * (FUSED_NB + 1);
+      q0 = cb[t];
+      q1 = cb[t + 1];
+    }
     if (j < j1) {
-      const int64_t e = F.el[j];
-      const MatParams m = EA.mats[EA.elem_mat ? EA.elem_mat[e] : 0];
-      double ue[dn];
-      double xe[RECOMPUTE ? dn : 1];
+      double ue[dn], xe[dn];
+      uint32_t ls[n];
+      int mat = 0;
+      const uint32_t w[4] = {rec.x, rec.y, rec.z, rec.w};
+      // triangles carry their material in the fourth word
+      if (n == 3) mat = int(rec.w);
+      else if (EA.elem_mat) mat = F.smat[j];
+      if (j + FUSED_CH < j1) rec = F.srec[j + FUSED_CH];
 #pragma unroll
       for (int a = 0; a < n; ++a) {
-        const int64_t nd = EA.conn[a * E + e];
+        ls[a] = w[a] >> 16;
+        const double2* src = reinterpret_cast<const double2*>(s_n + (w[a] & 0xFFFFu) * (2 * d));
+        double v[2 * d];
 #pragma unroll
         for (int i = 0; i < d; ++i) {
-          ue[i + a * d] = u_in[nd * d + i];
-          if constexpr (RECOMPUTE) xe[i + a * d] = EA.X[nd * d + i];
+          const double2 p = src[i];
+          v[2 * i] = p.x;
+          v[2 * i + 1] = p.y;
+        }
+#pragma unroll
+        for (int i = 0; i < d; ++i) {
+          ue[i + a * d] = v[i];
+          xe[i + a * d] = v[d + i];
         }
       }
+      const MatParams m = EA.mats[mat];
       double fe[dn];
-      element_forces_fp64<ET, KIND, RECOMPUTE>(EA, e, m, ue, xe, fe);
+      element_forces_fp64<ET, KIND, true>(EA, 0, m, ue, xe, fe);
 #pragma unroll
-      for (int a = 0; a < n; ++a) {
-        const uint32_t ls = F.lslot[size_t(j) * n + a];
-        if (ls != 0xFFFFu)
+      for (int a = 0; a < n; ++a)
+        if (ls[a] != 0xFFFFu)
 #pragma unroll
-          for (int i = 0; i < d; ++i) s_f[ls * d + i] = fe[i + a * d];
-      }
+          for (int i = 0; i < d; ++i) s_f[ls[a] * d + i] = fe[i + a * d];
     }
     __syncthreads();
     if (owner) {
       // this chunk's run of the node, in assembly order (the node kernel's
-      // sum: f += -1 * contribution)
-      const uint16_t* cb = F.cbase + size_t(c0 + c) * (FUSED_NB + 1);
-      const int q0 = cb[t], q1 = cb[t + 1];
-      for (int q = q0; q < q1; ++q)
+      // sum f += -1 * contribution), four entries read before they are added
+      int q = q0;
+      for (; q + 4 <= q1; q += 4) {
+        double x[4 * d];
 #pragma unroll
-        for (int i = 0; i < d; ++i) {
-          const double x = -1. * s_f[q * d + i];
-          f[i] += x;
-        }
+        for (int k = 0; k < 4 * d; ++k) x[k] = s_f[q * d + k];
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+#pragma unroll
+          for (int i = 0; i < d; ++i) f[i] -= x[k * d + i];
+      }
+      for (; q < q1; ++q)
+#pragma unroll
+        for (int i = 0; i < d; ++i) f[i] -= s_f[q * d + i];
     }
     __syncthreads();
   }
@@ -1707,7 +1805,7 @@ __global__ void __launch_bounds__(256) k_step_fused(ElemArgs EA, NodeArgs NA, Fu
   uint8_t bl[d];
 #pragma unroll
   for (int i = 0; i < d; ++i) {
-    u[i] = u_in[node * d + i];
+    u[i] = s_n[t * 2 * d + i];
     v[i] = NA.v[node * d + i];
     acc[i] = NA.a[node * d + i];
     bl[i] = NA.blocked[node * d + i];
@@ -2062,10 +2160,10 @@ static inline unsigned grid_for(int64_t n, int block) {
 
 hipError_t launch_precompute(int et, hipStream_t s, int64_t E, int64_t, const double* X,
                              const uint32_t* conn, const ElemTables& tab, double* B64, double* J64,
-                             float* B32, float* J32, int* bad) {
+                             float* B32, float* J32, int* bad, int* unsafe) {
   clear_error();
   if (E == 0) return hipSuccess;
-#define F(ET) k_precompute<ET><<<grid_for(E, 256), 256, 0, s>>>(E, X, conn, tab, B64, J64, B32, J32, bad)
+#define F(ET) k_precompute<ET><<<grid_for(E, 256), 256, 0, s>>>(E, X, conn, tab, B64, J64, B32, J32, bad, unsafe)
   AKX_ET_SWITCH(et, F)
 #undef F
   return hipGetLastError();
@@ -2201,8 +2299,8 @@ __global__ void __launch_bounds__(256) k_step_fused_mixed(ElemArgs EA, NodeArgs 
   const int64_t b = logical_block(NA.xcd_remap);
   if (b >= F.nblk) return;  // uniform over the block
   const int t = threadIdx.x;
-  const int64_t n0 = b * FUSED_NB;
-  const int cnt = int(min<int64_t>(FUSED_NB, NA.N - n0));
+  const int64_t n0 = F.blk[b];
+  const int cnt = int(F.blk[b + 1] - n0);
   const bool owner = t < cnt;
   const int64_t node = n0 + t;
   const int64_t E = EA.E;
@@ -2385,17 +2483,11 @@ hipError_t launch_fused_geometry(int et, hipStream_t s, int64_t E, const double*
 }
 
 template <int ET, int KIND>
-static hipError_t launch_fused_et(bool recompute, bool has_fext, hipStream_t s,
-                                  const ElemArgs& EA, const NodeArgs& NA, const FusedArgs& F,
-                                  int lds) {
+static hipError_t launch_fused_et(bool has_fext, hipStream_t s, const ElemArgs& EA,
+                                  const NodeArgs& NA, const FusedArgs& F, int lds) {
   const unsigned g = unsigned(F.nblk);
-  if (recompute) {
-    if (has_fext) k_step_fused<ET, KIND, true, true><<<g, 256, lds, s>>>(EA, NA, F);
-    else k_step_fused<ET, KIND, true, false><<<g, 256, lds, s>>>(EA, NA, F);
-  } else {
-    if (has_fext) k_step_fused<ET, KIND, false, true><<<g, 256, lds, s>>>(EA, NA, F);
-    else k_step_fused<ET, KIND, false, false><<<g, 256, lds, s>>>(EA, NA, F);
-  }
+  if (has_fext) k_step_fused<ET, KIND, true><<<g, 256, lds, s>>>(EA, NA, F);
+  else k_step_fused<ET, KIND, false><<<g, 256, lds, s>>>(EA, NA, F);
   return hipGetLastError();
 }
 
@@ -2415,17 +2507,15 @@ static hipError_t launch_fused_mixed_et(bool has_fext, hipStream_t s, const Elem
   return hipGetLastError();
 }
 
-hipError_t launch_fused(int et, int kind, int precision, bool recompute, bool has_fext,
-                        hipStream_t s, const ElemArgs& EA, const NodeArgs& NA, const FusedArgs& F,
-                        int lds) {
+hipError_t launch_fused(int et, int kind, int precision, bool has_fext, hipStream_t s,
+                        const ElemArgs& EA, const NodeArgs& NA, const FusedArgs& F, int lds) {
   clear_error();
   if (F.nblk == 0) return hipSuccess;
   if (kind != ELASTIC && kind != NEOHOOKEAN) return hipErrorInvalidValue;
   if (precision == 1) {
-    // FP32 contributions: half the LDS of the FP64 step
 #define M_(ET)                                                                            \
-  return kind == ELASTIC ? launch_fused_mixed_et<ET, ELASTIC>(has_fext, s, EA, NA, F, lds / 2) \
-                         : launch_fused_mixed_et<ET, NEOHOOKEAN>(has_fext, s, EA, NA, F, lds / 2);
+  return kind == ELASTIC ? launch_fused_mixed_et<ET, ELASTIC>(has_fext, s, EA, NA, F, lds) \
+                         : launch_fused_mixed_et<ET, NEOHOOKEAN>(has_fext, s, EA, NA, F, lds);
     switch (et) {
     case TRI3: M_(TRI3);
     case QUAD4: M_(QUAD4);
@@ -2436,8 +2526,8 @@ hipError_t launch_fused(int et, int kind, int precision, bool recompute, bool ha
   }
   // elements of up to 4 nodes (the host builds no fused tables for others)
 #define F_(ET)                                                                       \
-  return kind == ELASTIC ? launch_fused_et<ET, ELASTIC>(recompute, has_fext, s, EA, NA, F, lds) \
-                         : launch_fused_et<ET, NEOHOOKEAN>(recompute, has_fext, s, EA, NA, F, lds);
+  return kind == ELASTIC ? launch_fused_et<ET, ELASTIC>(has_fext, s, EA, NA, F, lds) \
+                         : launch_fused_et<ET, NEOHOOKEAN>(has_fext, s, EA, NA, F, lds);
   switch (et) {
   case TRI3: F_(TRI3);
   case QUAD4: F_(QUAD4);

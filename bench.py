@@ -109,15 +109,18 @@ def algorithmic_bytes(E, N, n, Q, d, pe, has_fext=False, tables=True, node_order
     return elem, node
 
 
-def fused_bytes(E, N, n, d, evaluations, nblk, node_block=256, chunk=256):
+def fused_bytes(E, N, n, d, evaluations, nblk, node_block=256, chunk=256, staged=False):
     """Compulsory HBM bytes of one fused FP64 step (slot layout 6): the blocks'
     element lists (4 bytes per evaluation) and LDS slots (2 bytes per node of
     an evaluation), the per-chunk run tables, connectivity and coordinates
     once, u read and written (two buffers), v and a read and written, lumped
-    mass and blocked flags."""
+    mass and blocked flags.  staged: one 16-byte record per evaluation in
+    place of list, slots and connectivity (the halo lists, 4 bytes per node of
+    another block, not counted)."""
     chunks = evaluations / chunk + nblk
-    return (evaluations * (4 + 2 * n) + chunks * (node_block + 1) * 2 + (nblk + 1) * 8
-            + E * n * 4 + N * d * 8 + 2 * N * d * 8 + 4 * N * d * 8 + N * 8 + N * d)
+    elements = evaluations * 16 if staged else evaluations * (4 + 2 * n) + E * n * 4
+    return (elements + chunks * (node_block + 1) * 2 + (nblk + 1) * 8
+            + N * d * 8 + 2 * N * d * 8 + 4 * N * d * 8 + N * 8 + N * d)
 
 
 def fused_mixed_bytes(E, N, n, d, evaluations, nblk, dt_per_node=False, node_block=256,
@@ -396,7 +399,9 @@ def bench_cube(args, akx):
                                    tables=not shapes["fp64"]["mixed_recompute"],
                                    node_ordered=bool(shapes["fp64"]["slot_layout"]))
     if shapes["fp64"]["slot_layout"] == 6 and model.query("fused_available") == 1:
-        eb64 = fused_bytes(E, N, n, d, model.query("fused_elements"), (N + 255) // 256)
+        eb64 = fused_bytes(E, N, n, d, model.query("fused_elements"),
+                           model.query("fused_blocks"),
+                           staged=model.query("fused_staged_lds") > 0)
         nb64 = 0
     copy_gbs = copy_bandwidth()
     log("device copy ceiling: %s GB/s" % (None if copy_gbs is None else round(copy_gbs, 1)))
@@ -635,10 +640,11 @@ def bench_ensemble(args, akx):
         return ("void akx::k_element_patch<0, 0>(akx::ElemArgs)" if patch else
                 "void akx::k_element_mixed<0, 0, %s>(akx::ElemArgs)" % ("true" if rc else "false"))
     fused = model.query("fused_available") == 1
-    nblk = (N + 255) // 256
+    nblk = model.query("fused_blocks")
     step64 = None
     if fused and shapes["fp64"]["slot_layout"] == 6:
-        step64 = fused_bytes(E, N, n, d, model.query("fused_elements"), nblk) + N * 8
+        step64 = N * 8 + fused_bytes(E, N, n, d, model.query("fused_elements"), nblk,
+                                     staged=model.query("fused_staged_lds") > 0)
     if fused and shapes["mixed"]["slot_layout"] == 6:
         # one kernel per step: its roofline is the step's
         records = (shapes["mixed"]["mixed_recompute"] == 1 and

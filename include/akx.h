@@ -233,7 +233,8 @@ int akx_last_step_timing(akx_ctx* ctx, double* element_ms, double* node_ms);
  * path), or no slots at all (6: one fused launch per step over node blocks
  * that recompute the elements around their nodes, on either path; stateless
  * laws of one kind on elements of up to 4 nodes -- elsewhere the FP64 path
- * runs 6 as node-ordered slots and the mixed path as 5), and whether the node
+ * runs 6 as node-ordered slots and the mixed path as 5; until a layout is set
+ * or autotuned, the FP64 path takes 6 where it applies), and whether the node
  * kernel copies its block's contiguous slot range to LDS first (node_stage
  * 1/0) (-1 keeps).  On the FP64 path none of these changes a result bit; on
  * the mixed path layouts 0/1, 2, 3 and 4/5 differ in rounding only
@@ -253,7 +254,9 @@ int akx_set_launch(akx_ctx* ctx, int element_block, int node_block, int xcd_rema
  *   "patch_nodes_total" (sum over LDS patches of their distinct nodes),
  *   "patch_max_nodes", "patch_available" (1/0), "patch_packed" (1/0: 16-bit
  *   patch-local node | rank words), "fused_available" (1/0: slot layout 6),
- *   "fused_elements" (element evaluations of one fused step),
+ *   "fused_elements" (element evaluations of one fused step), "fused_blocks",
+ *   "fused_staged_lds" (LDS bytes of a block of the fused FP64 step, 0: nodes
+ *   not staged),
  *   "fused_records" (1/0: per-evaluation records of the mixed fused step),
  *   "element_block", "node_block", "xcd_remap", "mixed_recompute", "slot_layout". */
 int akx_query(akx_ctx* ctx, const char* key, double* value);
