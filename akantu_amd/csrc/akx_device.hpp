@@ -61,6 +61,15 @@ __device__ __forceinline__ int64_t logical_block(int remap) {
   return (x < r) ? x * (q + 1) + l : r * (q + 1) + (x - r) * q + l;
 }
 
+// Block barrier for data exchanged through LDS only: __syncthreads would also
+// wait for every global load and store in flight (prefetches, results on their
+// way out), which no other thread of the block reads.
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 // ---------------------------------------------------------------------------
 // reference-order FP64 helpers (column-major)
 // ---------------------------------------------------------------------------

@@ -292,14 +292,10 @@ struct Surrogate {
   int64_t nsamples = 0;
   // batch buffers
   int bcap = 0;
-  __bf16 *X0 = nullptr, *X0T = nullptr, *dY = nullptr, *dYT = nullptr;
   float *Tb = nullptr, *Yb = nullptr, *loss_part = nullptr;
-  __bf16* H[5] = {};
-  __bf16* HT[5] = {};
+  __bf16* act[5] = {};  // inputs of each layer, by 16-point groups
+  __bf16* err[5] = {};  // errors at each layer's output, the same way
   float* part[5] = {};
-  float* Zt[4] = {};
-  __bf16* dZ[4] = {};
-  __bf16* dZT[4] = {};
   float *io_x = nullptr, *io_y = nullptr;
   int64_t io_cap = 0;
   // per-point inputs / outputs of the element step (8 floats per point)
@@ -314,7 +310,9 @@ struct Surrogate {
   hipError_t ensure_io(int64_t n);
   hipError_t ensure_points(int64_t n);
   hipError_t refresh(hipStream_t s);
-  hipError_t pass(hipStream_t s, int B, bool grad_only, float lr);
+  hipError_t run_pass(hipStream_t s, const float* x, const float* t, int64_t n, int B,
+                      uint64_t seed, int64_t iter, bool backward, bool outputs);
+  hipError_t apply(hipStream_t s, int B, bool grad_only, float lr);
   hipError_t batch_loss(hipStream_t s, int B, double* loss);
   hipError_t generate(hipStream_t s, int64_t paths, int steps, double inc_std, double yd_scale,
                       double yd_shape, uint64_t seed);

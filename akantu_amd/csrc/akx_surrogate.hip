@@ -134,86 +134,206 @@ __global__ void __launch_bounds__(256) k_sur_gen(int64_t paths, int steps, doubl
 }
 
 // ---------------------------------------------------------------------------
-// minibatch assembly: row b of the batch is sample idx(b) (drawn with
-// replacement) or, for an explicit batch, sample b
-__global__ void __launch_bounds__(256) k_sur_batch(const float* __restrict__ X,
-                                                   const float* __restrict__ T, int64_t n,
-                                                   int B, uint64_t seed, int64_t iter,
-                                                   int draw, __bf16* X0, __bf16* X0T,
-                                                   float* Tb) {
-  const int b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= B) return;
-  const int64_t idx = draw ? int64_t(mix64(seed ^ mix64(uint64_t(iter) * B + b)) % uint64_t(n)) : b;
-  float x[7];
-  for (int k = 0; k < 7; ++k) x[k] = X[idx * 7 + k];
-  for (int k = 0; k < K0; ++k) {
-    float v = 0.f;
-    if (k < NIN) v = x[k];
-    else if (k < 2 * NIN) v = x[k - NIN] - from_bf16(to_bf16(x[k - NIN]));
-    const __bf16 bv = to_bf16(v);
-    X0[int64_t(b) * K0 + k] = bv;
-    X0T[int64_t(k) * B + b] = bv;
-  }
-  for (int k = 0; k < 7; ++k) Tb[int64_t(b) * 8 + k] = T[idx * 7 + k];
-  Tb[int64_t(b) * 8 + 7] = 0.f;
+// Training pass.  Three launches per minibatch: k_sur_pass (draw, forward,
+// output error, backward through the layers), k_sur_weight_gradients (every
+// layer's split-K products) and k_sur_update.  16-bit operands live in memory
+// as MFMA fragments, so that every operand load is one contiguous kilobyte per
+// wave:
+//   weights, rows x K:      frag(row, k, K / 16), both orientations
+//   activations and errors: [16-point group][feature][point], K = points
+__host__ __device__ constexpr int frag(int row, int k, int ksteps) {
+  return (((row >> 5) * ksteps + (k >> 4)) * 64 + ((k >> 3) & 1) * 32 + (row & 31)) * 8 + (k & 7);
 }
+// features stored per 16-point group: the inputs (7 + 7 residuals + 2 zeros),
+// the hidden layers, and the output errors (7 + 1 zero)
+__host__ __device__ constexpr int act_rows(int layer) { return layer == 0 ? K0 : HID; }
+__host__ __device__ constexpr int err_rows(int layer) { return layer == 4 ? 8 : HID; }
 
-// forward layer: Z^T = W H^T + b over a 32 x 32 tile per wave.
-//   Hin  [B x KIN] bf16 (row = point), W [NP x KIN] bf16, rows >= nout zero
-//   ACT:  Zt [nout x B] fp32, Hout [B x nout], HoutT [nout x B] bf16 (activation)
-//   !ACT: Y [B x 8] fp32
-template <int KIN, int NP, bool ACT>
-__global__ void __launch_bounds__(256) k_sur_fwd(const __bf16* __restrict__ Hin,
-                                                 const __bf16* __restrict__ W,
-                                                 const float* __restrict__ bias, int nout, int B,
-                                                 float* Zt, __bf16* Hout, __bf16* HoutT,
-                                                 float* Y) {
-  const int64_t wave = (int64_t(blockIdx.x) * blockDim.x + threadIdx.x) >> 6;
-  constexpr int MB = NP / 32;
-  if (wave >= int64_t(MB) * (B / 32)) return;  // uniform over the wave
-  const int mb = int(wave % MB), jb = int(wave / MB);
-  const int lane = threadIdx.x & 63, i = lane & 31, h = lane >> 5;
-  f32x16 acc = f32x16{};
+struct PassArgs {
+  const float *X, *T;       // samples: n x 7 inputs and targets
+  int64_t n;
+  int B;                    // batch (a multiple of 32)
+  uint64_t seed;
+  int64_t iter;
+  int draw;                 // samples drawn with replacement, else sample b
+  const __bf16* W[5];       // weights, fragments
+  const __bf16* WT[5];      // transposed weights (layers 1 to 4)
+  const float* params;      // biases
+  __bf16* act[5];           // inputs of layer l (l = 0: the samples), point groups
+  __bf16* err[5];           // errors at the output of layer l
+  float *Y, *T8;            // outputs and targets, B x 8 (nullptr: not written)
+  int backward;
+};
+
+// One block of 4 waves per 32 points; wave mb owns features 32 mb .. 32 mb + 31
+// of every layer.  A layer's result tile becomes the next layer's operand
+// through LDS (rows of 128 + 8: 16-byte reads without bank conflicts); the
+// pre-activations stay in registers for the way back, whose tiles have the
+// same shape.  Products, roundings and their order are those of one 32 x 32
+// tile per wave and layer, so the pass is bound by the chain of its layers
+// (LDS exchange, barrier, 8 MFMAs), not by rates: 12 us at a batch of 8,192,
+// and 7 more for the 17 MB of activations and errors the weight gradients
+// read.  As one launch per layer and direction, with every intermediate
+// written twice (row-major and transposed), such a minibatch took 205 us of
+// kernels in 21 launches, now 32 in three.  One wave per SIMD with all its
+// registers: capped at two (spilling) it was slower at every batch (8,192: 48
+// against 35 us per minibatch, 65,536: 222 against 161).
+__global__ void __launch_bounds__(256) k_sur_pass(PassArgs A) {
+  constexpr int HS = HID + 8, XS = 24, TS = 40;
+  __shared__ __align__(16) __bf16 s_h[2][32][HS];
+  __shared__ __align__(16) __bf16 s_x[32][XS];      // inputs, later output errors
+  __shared__ __align__(16) __bf16 s_t[4][32][TS];   // a wave's tile, transposed
+  __shared__ __align__(16) float s_b[4 * HID + 8];
+  __shared__ float s_T[32][8];
+  const int64_t tile = blockIdx.x;
+  const int mb = threadIdx.x >> 6, lane = threadIdx.x & 63, i = lane & 31, h = lane >> 5;
+  constexpr int OFF_B[5] = {OFF_B0, OFF_B1, OFF_B2, OFF_B3, OFF_B4};
+  // the weights of the layer after the current one, loaded a layer ahead
+  bf16x8 w[8], wn[8];
+  auto fetch = [&](const __bf16* W, int ksteps, bf16x8 (&dst)[8]) {
 #pragma unroll
-  for (int t = 0; t < KIN / 16; ++t) {
-    const bf16x8 a = *reinterpret_cast<const bf16x8*>(W + (32 * mb + i) * KIN + 16 * t + 8 * h);
-    const bf16x8 b =
-        *reinterpret_cast<const bf16x8*>(Hin + int64_t(32 * jb + i) * KIN + 16 * t + 8 * h);
-    acc = mfma(a, b, acc);
-  }
-  const int64_t c = 32 * jb + i;
+    for (int t = 0; t < 8; ++t)
+      if (t < ksteps)
+        dst[t] = *reinterpret_cast<const bf16x8*>(W + ((mb * ksteps + t) * 64 + lane) * 8);
+  };
+  fetch(A.W[0], 1, w);
+  fetch(A.W[1], 8, wn);
+  if (threadIdx.x < 32) {
+    const int64_t b = tile * 32 + threadIdx.x;
+    const int64_t idx =
+        A.draw ? int64_t(mix64(A.seed ^ mix64(uint64_t(A.iter) * A.B + b)) % uint64_t(A.n)) : b;
+    float x[NIN];
 #pragma unroll
-  for (int v = 0; v < 16; ++v) {
-    const int r = 32 * mb + crow(v, h);
-    if (r >= nout) continue;
-    const float z = acc[v] + bias[r];
-    if constexpr (ACT) {
-      Zt[int64_t(r) * B + c] = z;
-      const __bf16 hv = to_bf16(act(z));
-      Hout[c * nout + r] = hv;
-      HoutT[int64_t(r) * B + c] = hv;
-    } else {
-      Y[c * 8 + r] = z;
+    for (int k = 0; k < NIN; ++k) x[k] = A.X[idx * NIN + k];
+#pragma unroll
+    for (int k = 0; k < K0; ++k) {
+      float v = 0.f;
+      if (k < NIN) v = x[k];
+      else if (k < 2 * NIN) v = x[k - NIN] - from_bf16(to_bf16(x[k - NIN]));
+      const __bf16 bv = to_bf16(v);
+      s_x[threadIdx.x][k] = bv;
+      if (A.backward)
+        A.act[0][((b >> 4) * K0 + k) * 16 + (b & 15)] = bv;
+    }
+#pragma unroll
+    for (int k = 0; k < NOUT; ++k) s_T[threadIdx.x][k] = A.T[idx * NOUT + k];
+    s_T[threadIdx.x][7] = 0.f;
+  } else {
+    for (int k = int(threadIdx.x) - 32; k < 4 * HID + NOUT; k += 224) {
+      const int l = k >> 7;
+      s_b[k] = A.params[OFF_B[l] + (k - l * HID)];
     }
   }
+  lds_barrier();
+  // a wave's tile of 16-bit values v[16] (register r: feature 32 mb +
+  // crow(r, h), point i): to s_h[buf] for the next layer and, transposed
+  // through LDS, to memory for the weight gradients
+  auto emit = [&](const __bf16 (&v)[16], int buf, __bf16* out, int rows) {
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+      *reinterpret_cast<bf16x4*>(&s_h[buf][i][32 * mb + crow(4 * g, h)]) =
+          bf16x4{v[4 * g], v[4 * g + 1], v[4 * g + 2], v[4 * g + 3]};
+    }
+    if (A.backward) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) s_t[mb][crow(r, h)][i] = v[r];
+    }
+    lds_barrier();
+    if (A.backward) {
+#pragma unroll
+      for (int g = 0; g < 2; ++g) {
+        const int row = lane >> 1, half = lane & 1;
+        const bf16x8 u = *reinterpret_cast<const bf16x8*>(&s_t[mb][row][16 * g + 8 * half]);
+        *reinterpret_cast<bf16x8*>(out + ((tile * 2 + g) * rows + 32 * mb + row) * 16 + 8 * half) =
+            u;
+      }
+    }
+  };
+  auto product = [&](const bf16x8 (&a)[8], int buf) {
+    f32x16 acc = f32x16{};
+#pragma unroll
+    for (int t = 0; t < 8; ++t)
+      acc = mfma(a[t], *reinterpret_cast<const bf16x8*>(&s_h[buf][i][16 * t + 8 * h]), acc);
+    return acc;
+  };
+  f32x16 z[4];
+#pragma unroll
+  for (int l = 0; l < 4; ++l) {
+    f32x16 acc;
+    if (l == 0) acc = mfma(w[0], *reinterpret_cast<const bf16x8*>(&s_x[i][8 * h]), f32x16{});
+    else acc = product(w, (l - 1) & 1);
+    __bf16 v[16];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      z[l][r] = acc[r] + s_b[l * HID + 32 * mb + crow(r, h)];
+      v[r] = to_bf16(act(z[l][r]));
+    }
+#pragma unroll
+    for (int t = 0; t < 8; ++t) w[t] = wn[t];
+    if (l < 2) fetch(A.W[l + 2], 8, wn);
+    else if (l == 2) {
+      // the output layer's 32 rows are one tile, wave 0's
+#pragma unroll
+      for (int t = 0; t < 8; ++t)
+        wn[t] = *reinterpret_cast<const bf16x8*>(A.W[4] + (t * 64 + lane) * 8);
+    } else if (A.backward) {
+      fetch(A.WT[4], 1, wn);
+    }
+    emit(v, l & 1, A.act[l + 1], HID);
+  }
+  // outputs, and their errors 2 (Y - T) / (7 B) in place of the inputs
+  if (mb == 0) {
+    const f32x16 acc = product(w, 1);
+    const int64_t b = tile * 32 + i;
+    const float sc = 2.f / (7.f * float(A.B));
+    __bf16 g[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int k = 4 * h + r;
+      const float t = s_T[i][k];
+      const float y = k < NOUT ? acc[r] + s_b[4 * HID + k] : 0.f;
+      if (A.Y) {
+        A.Y[b * 8 + k] = y;
+        A.T8[b * 8 + k] = t;
+      }
+      g[r] = to_bf16(k < NOUT ? sc * (y - t) : 0.f);
+      s_x[i][k] = g[r];
+      s_x[i][8 + k] = to_bf16(0.f);
+      if (A.backward) A.err[4][((b >> 4) * 8 + k) * 16 + (b & 15)] = g[r];
+    }
+  }
+  if (!A.backward) return;
+  lds_barrier();
+  bf16x8 wb[8];
+  fetch(A.WT[3], 8, wb);
+#pragma unroll
+  for (int l = 3; l >= 0; --l) {
+    // error at the output of layer l: W_{l+1}^T err_{l+1}, times a'(z_l)
+    f32x16 acc;
+    if (l == 3) acc = mfma(wn[0], *reinterpret_cast<const bf16x8*>(&s_x[i][8 * h]), f32x16{});
+    else acc = product(w, (l + 1) & 1);
+    __bf16 v[16];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) v[r] = to_bf16(acc[r] * act_grad(z[l][r]));
+#pragma unroll
+    for (int t = 0; t < 8; ++t) w[t] = wb[t];
+    if (l >= 2) fetch(A.WT[l - 1], 8, wb);
+    emit(v, l & 1, A.err[l], HID);
+  }
 }
 
-// output error: dY = 2 (Y - T) / (7 B) (bf16, both layouts), loss partial sums
+// loss partial sums per 256 points
 __global__ void __launch_bounds__(256) k_sur_loss(const float* __restrict__ Y,
                                                   const float* __restrict__ T, int B,
-                                                  __bf16* dY, __bf16* dYT, float* partial) {
+                                                  float* partial) {
   const int b = blockIdx.x * blockDim.x + threadIdx.x;
   float l = 0.f;
-  if (b < B) {
-    const float sc = 2.f / (7.f * float(B));
+  if (b < B)
     for (int k = 0; k < 7; ++k) {
       const float diff = Y[int64_t(b) * 8 + k] - T[int64_t(b) * 8 + k];
       l += diff * diff;
-      const __bf16 g = to_bf16(sc * diff);
-      dY[int64_t(b) * 16 + k] = g;
-      dYT[int64_t(k) * B + b] = g;
     }
-  }
   __shared__ float sh[4];
   for (int o = 32; o > 0; o >>= 1) l += __shfl_down(l, o, 64);
   if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = l;
@@ -221,101 +341,131 @@ __global__ void __launch_bounds__(256) k_sur_loss(const float* __restrict__ Y,
   if (threadIdx.x == 0) partial[blockIdx.x] = (sh[0] + sh[1]) + (sh[2] + sh[3]);
 }
 
-// backward through a layer's weights and the previous activation:
-//   dH^T = W^T dZ^T (tile rows: input features 0..127, columns: points),
-//   dZprev = dH * a'(Zprev), stored bf16 in both layouts.
-//   WT [128 x KC] bf16, dZ [B x KC] bf16, Zt_prev [128 x B] fp32
-template <int KC>
-__global__ void __launch_bounds__(256) k_sur_bwd_data(const __bf16* __restrict__ WT,
-                                                      const __bf16* __restrict__ dZ,
-                                                      const float* __restrict__ Zt_prev, int B,
-                                                      __bf16* dZp, __bf16* dZpT) {
-  const int64_t wave = (int64_t(blockIdx.x) * blockDim.x + threadIdx.x) >> 6;
-  if (wave >= int64_t(4) * (B / 32)) return;
-  const int mb = int(wave % 4), jb = int(wave / 4);
-  const int lane = threadIdx.x & 63, i = lane & 31, h = lane >> 5;
-  f32x16 acc = f32x16{};
-#pragma unroll
-  for (int t = 0; t < KC / 16; ++t) {
-    const bf16x8 a = *reinterpret_cast<const bf16x8*>(WT + (32 * mb + i) * KC + 16 * t + 8 * h);
-    const bf16x8 b =
-        *reinterpret_cast<const bf16x8*>(dZ + int64_t(32 * jb + i) * KC + 16 * t + 8 * h);
-    acc = mfma(a, b, acc);
-  }
-  const int64_t c = 32 * jb + i;
-#pragma unroll
-  for (int v = 0; v < 16; ++v) {
-    const int r = 32 * mb + crow(v, h);
-    const float z = Zt_prev[int64_t(r) * B + c];
-    const __bf16 g = to_bf16(acc[v] * act_grad(z));
-    dZp[c * HID + r] = g;
-    dZpT[int64_t(r) * B + c] = g;
-  }
+// Weight and bias gradients of every layer, split over batch chunks, one wave
+// per 32 x 32 tile and chunk:
+//   partial[c][n][k]    = sum_{b in chunk c} err[n][b] act[k][b]   (k < act_rows)
+//   partial[c][n][rows] = sum_{b in chunk c} err[n][b]             (bias)
+// The points of a chunk are one chain of MFMAs (64 in chunks of 1,024), so the
+// loads of the next group of 8 steps are in flight while the current one
+// multiplies: bound by the operands' way from the L2.  The chunk is the fastest
+// index of the waves, so that with 8 chunks each XCD reads one chunk only (9.6
+// -> 9.0 us at a batch of 8,192, and the layers' separate launches before:
+// 17 to 19.5 us each, 93 together).
+struct WeightGradArgs {
+  const __bf16* act[5];
+  const __bf16* err[5];
+  float* partial[5];
+  int first[6];  // first wave of each layer
+  int chunk, nch;
+};
+__host__ __device__ constexpr int grad_tiles(int layer) {
+  return ((layer == 4 ? 32 : HID) / 32) * ((act_rows(layer) + 1 + 31) / 32);
 }
 
-// weight and bias gradients, split over batch chunks:
-//   partial[c][n][k] = sum_{b in chunk c} dZ^T[n][b] H^T[k][b]   (k < KC)
-//   partial[c][n][KC] = sum_{b in chunk c} dZ^T[n][b]            (bias)
-template <int NP, int KC>
-__global__ void __launch_bounds__(256) k_sur_bwd_weight(const __bf16* __restrict__ dZT, int nout,
-                                                        const __bf16* __restrict__ HT, int B,
-                                                        int chunk, float* partial) {
-  constexpr int MB = NP / 32, KB = (KC + 1 + 31) / 32;
-  const int64_t wave = (int64_t(blockIdx.x) * blockDim.x + threadIdx.x) >> 6;
-  const int nch = B / chunk;
-  if (wave >= int64_t(MB) * KB * nch) return;
-  const int mb = int(wave % MB), kb = int((wave / MB) % KB), ch = int(wave / (MB * KB));
-  const int lane = threadIdx.x & 63, i = lane & 31, h = lane >> 5;
+template <int L>
+__device__ __forceinline__ void weight_gradient_tile(const WeightGradArgs& A, int wave, int lane) {
+  constexpr int MB = (L == 4 ? 32 : HID) / 32, KR = act_rows(L), ER = err_rows(L);
+  constexpr int nout = L == 4 ? NOUT : HID, STEP = 8;
+  const int ch = wave % A.nch, mb = (wave / A.nch) % MB, kb = wave / (A.nch * MB);
+  const int i = lane & 31, h = lane >> 5;
   const int n_a = 32 * mb + i, k_b = 32 * kb + i;
-  const int64_t b0 = int64_t(ch) * chunk;
+  const int64_t g0 = int64_t(ch) * (A.chunk / 16);
+  const bf16x8 zero = bf16x8{};
   bf16x8 one;
 #pragma unroll
   for (int s = 0; s < 8; ++s) one[s] = to_bf16(1.f);
-  const bf16x8 zero = bf16x8{};
+  const bool has_a = n_a < ER, has_b = k_b < KR;
+  const bf16x8 fill = k_b == KR ? one : zero;
+  const __bf16* pa = A.err[L] + (g0 * ER + (has_a ? n_a : 0)) * 16 + 8 * h;
+  const __bf16* pb = A.act[L] + (g0 * KR + (has_b ? k_b : 0)) * 16 + 8 * h;
+  bf16x8 a[STEP], b[STEP], an[STEP], bn[STEP];
+  auto load = [&](int t, bf16x8 (&x)[STEP], bf16x8 (&y)[STEP]) {
+#pragma unroll
+    for (int s = 0; s < STEP; ++s) {
+      x[s] = has_a ? *reinterpret_cast<const bf16x8*>(pa + int64_t(t + s) * ER * 16) : zero;
+      y[s] = has_b ? *reinterpret_cast<const bf16x8*>(pb + int64_t(t + s) * KR * 16) : fill;
+    }
+  };
+  const int steps = A.chunk / 16;  // 16 or 64
   f32x16 acc = f32x16{};
-  for (int t = 0; t < chunk / 16; ++t) {
-    const int64_t bb = b0 + 16 * t + 8 * h;
-    const bf16x8 a = n_a < nout ? *reinterpret_cast<const bf16x8*>(dZT + int64_t(n_a) * B + bb) : zero;
-    const bf16x8 b = k_b < KC ? *reinterpret_cast<const bf16x8*>(HT + int64_t(k_b) * B + bb)
-                              : (k_b == KC ? one : zero);
-    acc = mfma(a, b, acc);
+  load(0, a, b);
+  for (int t = 0; t < steps; t += STEP) {
+    if (t + STEP < steps) load(t + STEP, an, bn);
+#pragma unroll
+    for (int s = 0; s < STEP; ++s) acc = mfma(a[s], b[s], acc);
+#pragma unroll
+    for (int s = 0; s < STEP; ++s) {
+      a[s] = an[s];
+      b[s] = bn[s];
+    }
   }
 #pragma unroll
   for (int v = 0; v < 16; ++v) {
     const int n = 32 * mb + crow(v, h);
-    if (n < nout && k_b <= KC) partial[(int64_t(ch) * nout + n) * (KC + 1) + k_b] = acc[v];
+    if (n < nout && k_b <= KR) A.partial[L][(int64_t(ch) * nout + n) * (KR + 1) + k_b] = acc[v];
   }
+}
+
+__global__ void __launch_bounds__(64) k_sur_weight_gradients(WeightGradArgs A) {
+  const int wave = blockIdx.x, lane = threadIdx.x;
+  // the layer is uniform over the wave
+  if (wave < A.first[1]) weight_gradient_tile<0>(A, wave, lane);
+  else if (wave < A.first[2]) weight_gradient_tile<1>(A, wave - A.first[1], lane);
+  else if (wave < A.first[3]) weight_gradient_tile<2>(A, wave - A.first[2], lane);
+  else if (wave < A.first[4]) weight_gradient_tile<3>(A, wave - A.first[3], lane);
+  else if (wave < A.first[5]) weight_gradient_tile<4>(A, wave - A.first[4], lane);
 }
 
 struct LayerDesc {
   int nout, nin, kc;     // kc: partial columns before the bias column (16 for layer 0)
   int off_w, off_b;
   const float* partial;  // [nch][nout][kc + 1]
-  __bf16* Wbf;           // forward weights [np][kbf]
-  int kbf;
-  __bf16* WT;            // backward weights [nin][ktp] (nullptr for layer 0)
-  int ktp;
+  __bf16* W;             // fragments of the weights and, layers 1 to 4, of their transpose
+  __bf16* WT;
+  int first;             // first thread of the layer
+};
+struct UpdateArgs {
+  LayerDesc layer[5];
+  int threads;
 };
 
-// gradient of every parameter of one layer from the chunk partials (fixed
-// order); then either an Adam step on the FP32 master copy (refreshing the
-// BF16 copies) or a plain copy of the gradient to `grad_out`
-__global__ void __launch_bounds__(256) k_sur_update(LayerDesc L, int nch, float* params,
+// gradient of every parameter from the chunk partials (fixed order); then
+// either an Adam step on the FP32 master copy (refreshing the BF16 copies) or
+// a plain copy of the gradient to `grad_out`
+__global__ void __launch_bounds__(256) k_sur_update(UpdateArgs U, int nch, float* params,
                                                     float* m1, float* m2, float lr, float beta1,
                                                     float beta2, float eps, float bc1, float bc2,
                                                     float* grad_out) {
-  const int idx = blockIdx.x * blockDim.x + threadIdx.x;
+  const int at = blockIdx.x * blockDim.x + threadIdx.x;
+  if (at >= U.threads) return;
+  int l = 0;
+#pragma unroll
+  for (int k = 1; k < 5; ++k)
+    if (at >= U.layer[k].first) l = k;
+  const LayerDesc L = U.layer[l];
+  const int idx = at - L.first;
   const int nw = L.nout * L.nin;
-  if (idx >= nw + L.nout) return;
   const bool is_w = idx < nw;
   const int n = is_w ? idx / L.nin : idx - nw;
   const int k = is_w ? idx % L.nin : L.kc;
   const int cols = L.kc + 1;
+  // layer 0: x_hi and x_lo share the weight, added after each chunk's x_hi
+  const bool pair = is_w && L.kc == K0;
   float g = 0.f;
-  for (int c = 0; c < nch; ++c) {
-    const float* P = L.partial + (int64_t(c) * L.nout + n) * cols;
-    g += P[k];
-    if (is_w && L.kc == K0) g += P[k + NIN];  // layer 0: x_hi and x_lo share the weight
+  for (int c = 0; c < nch; c += 4) {
+    float p[4], q[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float* P = L.partial + (int64_t(min(c + j, nch - 1)) * L.nout + n) * cols;
+      p[j] = P[k];
+      q[j] = pair ? P[k + NIN] : 0.f;
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (c + j < nch) {
+        g += p[j];
+        if (pair) g += q[j];
+      }
   }
   const int p = is_w ? L.off_w + idx : L.off_b + n;
   if (grad_out) {
@@ -330,14 +480,15 @@ __global__ void __launch_bounds__(256) k_sur_update(LayerDesc L, int nch, float*
   params[p] = w;
   if (is_w) {
     const __bf16 wb = to_bf16(w);
-    L.Wbf[n * L.kbf + k] = wb;
-    if (L.kc == K0) L.Wbf[n * L.kbf + k + NIN] = wb;
-    if (L.WT) L.WT[k * L.ktp + n] = wb;
+    const int ks = l == 0 ? 1 : 8;
+    L.W[frag(n, k, ks)] = wb;
+    if (l == 0) L.W[frag(n, k + NIN, ks)] = wb;
+    else L.WT[frag(k, n, l == 4 ? 1 : 8)] = wb;
   }
 }
 
-// BF16 copies of the master weights (forward layout, transposed layout) and
-// the permuted inference image, FP16 or (bf16 != 0) BF16
+// BF16 copies of the master weights (fragments, both orientations) and the
+// permuted inference image, FP16 or (bf16 != 0) BF16
 __global__ void __launch_bounds__(256) k_sur_refresh(const float* __restrict__ P, __bf16* W0,
                                                      __bf16* W1, __bf16* W2, __bf16* W3,
                                                      __bf16* W4, __bf16* T1, __bf16* T2,
@@ -348,20 +499,21 @@ __global__ void __launch_bounds__(256) k_sur_refresh(const float* __restrict__ P
   if (idx < HID * K0) {
     const int n = idx / K0, k = idx % K0;
     const float w = k < NIN ? P[OFF_W0 + n * NIN + k] : k < 2 * NIN ? P[OFF_W0 + n * NIN + k - NIN] : 0.f;
-    W0[idx] = to_bf16(w);
+    W0[frag(n, k, 1)] = to_bf16(w);
   }
   if (idx < HID * HID) {
     const int n = idx / HID, k = idx % HID;
     const __bf16 a = to_bf16(P[OFF_W1 + idx]), b = to_bf16(P[OFF_W2 + idx]),
                  c = to_bf16(P[OFF_W3 + idx]);
-    W1[idx] = a; W2[idx] = b; W3[idx] = c;
-    T1[k * HID + n] = a; T2[k * HID + n] = b; T3[k * HID + n] = c;
+    const int f = frag(n, k, 8), ft = frag(k, n, 8);
+    W1[f] = a; W2[f] = b; W3[f] = c;
+    T1[ft] = a; T2[ft] = b; T3[ft] = c;
   }
   if (idx < 32 * HID) {
     const int n = idx / HID, k = idx % HID;
     const __bf16 w = to_bf16(n < NOUT ? P[OFF_W4 + n * HID + k] : 0.f);
-    W4[idx] = w;
-    if (n < 16) T4[k * 16 + n] = w;
+    W4[frag(n, k, 8)] = w;
+    if (n < 16) T4[frag(k, n, 1)] = w;
   }
   // permuted image: one thread per (vector, slot)
   if (idx < PW_SIZE * 8) {
@@ -470,18 +622,14 @@ void dfree_p(T*& p) {
   p = nullptr;
 }
 
-inline unsigned blocks_for_waves(int64_t waves) { return unsigned((waves + 3) / 4); }
-
 }  // namespace
 
 // ---------------------------------------------------------------------------
 Surrogate::~Surrogate() { release(); }
 
 void Surrogate::release_batch() {
-  dfree_p(X0); dfree_p(X0T); dfree_p(Tb); dfree_p(Yb); dfree_p(dY); dfree_p(dYT);
-  dfree_p(loss_part);
-  for (int l = 0; l < 5; ++l) { dfree_p(H[l]); dfree_p(HT[l]); dfree_p(part[l]); }
-  for (int l = 0; l < 4; ++l) { dfree_p(Zt[l]); dfree_p(dZ[l]); dfree_p(dZT[l]); }
+  dfree_p(Tb); dfree_p(Yb); dfree_p(loss_part);
+  for (int l = 0; l < 5; ++l) { dfree_p(act[l]); dfree_p(err[l]); dfree_p(part[l]); }
   bcap = 0;
 }
 
@@ -549,80 +697,87 @@ hipError_t Surrogate::ensure_batch(int B) {
   release_batch();
   hipError_t e;
   const size_t b = size_t(B);
-  if ((e = dalloc_n(&X0, b * K0)) || (e = dalloc_n(&X0T, b * K0)) || (e = dalloc_n(&Tb, b * 8)) ||
-      (e = dalloc_n(&Yb, b * 8)) || (e = dalloc_n(&dY, b * 16)) || (e = dalloc_n(&dYT, b * NOUT)) ||
+  if ((e = dalloc_n(&Tb, b * 8)) || (e = dalloc_n(&Yb, b * 8)) ||
       (e = dalloc_n(&loss_part, (b + 255) / 256)))
     return e;
-  for (int l = 1; l < 5; ++l)
-    if ((e = dalloc_n(&H[l], b * HID)) || (e = dalloc_n(&HT[l], b * HID))) return e;
-  for (int l = 0; l < 4; ++l)
-    if ((e = dalloc_n(&Zt[l], b * HID)) || (e = dalloc_n(&dZ[l], b * HID)) ||
-        (e = dalloc_n(&dZT[l], b * HID)))
-      return e;
   // chunk partials: at most B / 256 chunks of [nout][kc + 1]
   const size_t nch = b / 256;
-  const int kc[5] = {K0, HID, HID, HID, HID}, no[5] = {HID, HID, HID, HID, NOUT};
   for (int l = 0; l < 5; ++l)
-    if ((e = dalloc_n(&part[l], nch * no[l] * (kc[l] + 1)))) return e;
-  if ((e = hipMemset(dY, 0, b * 16 * 2))) return e;  // columns 7..15 stay zero
+    if ((e = dalloc_n(&act[l], b * act_rows(l))) || (e = dalloc_n(&err[l], b * err_rows(l))) ||
+        (e = dalloc_n(&part[l], nch * (l == 4 ? NOUT : HID) * (act_rows(l) + 1))))
+      return e;
   bcap = B;
   return hipSuccess;
 }
 
-// one forward + backward pass over the current batch; then either an Adam
-// step (grad_only = false) or the gradient into `grad` (grad_only = true)
-hipError_t Surrogate::pass(hipStream_t s, int B, bool grad_only, float lr) {
+// k_sur_pass on a batch of B samples of (x, t): drawn for iteration `iter`
+// (iter >= 0) or the first B
+hipError_t Surrogate::run_pass(hipStream_t s, const float* x, const float* t, int64_t n, int B,
+                               uint64_t seed, int64_t iter, bool backward, bool outputs) {
+  PassArgs A;
+  A.X = x;
+  A.T = t;
+  A.n = n;
+  A.B = B;
+  A.seed = seed;
+  A.iter = iter < 0 ? 0 : iter;
+  A.draw = iter >= 0;
+  for (int l = 0; l < 5; ++l) {
+    A.W[l] = Wbf[l];
+    A.WT[l] = WT[l];
+    A.act[l] = act[l];
+    A.err[l] = err[l];
+  }
+  A.params = params;
+  A.Y = outputs ? Yb : nullptr;
+  A.T8 = Tb;
+  A.backward = backward;
+  k_sur_pass<<<unsigned(B / 32), 256, 0, s>>>(A);
+  return hipGetLastError();
+}
+
+// parameter gradients of the batch that k_sur_pass went back through; then
+// either an Adam step (grad_only = false) or the gradient into `grad`
+// (grad_only = true)
+hipError_t Surrogate::apply(hipStream_t s, int B, bool grad_only, float lr) {
   const int chunk = (B % 1024 == 0) ? 1024 : 256;
   const int nch = B / chunk;
-  const int64_t jbs = B / 32;
-  k_sur_fwd<K0, HID, true><<<blocks_for_waves(4 * jbs), 256, 0, s>>>(
-      X0, Wbf[0], params + OFF_B0, HID, B, Zt[0], H[1], HT[1], nullptr);
-  k_sur_fwd<HID, HID, true><<<blocks_for_waves(4 * jbs), 256, 0, s>>>(
-      H[1], Wbf[1], params + OFF_B1, HID, B, Zt[1], H[2], HT[2], nullptr);
-  k_sur_fwd<HID, HID, true><<<blocks_for_waves(4 * jbs), 256, 0, s>>>(
-      H[2], Wbf[2], params + OFF_B2, HID, B, Zt[2], H[3], HT[3], nullptr);
-  k_sur_fwd<HID, HID, true><<<blocks_for_waves(4 * jbs), 256, 0, s>>>(
-      H[3], Wbf[3], params + OFF_B3, HID, B, Zt[3], H[4], HT[4], nullptr);
-  k_sur_fwd<HID, 32, false><<<blocks_for_waves(jbs), 256, 0, s>>>(
-      H[4], Wbf[4], params + OFF_B4, NOUT, B, nullptr, nullptr, nullptr, Yb);
-  k_sur_loss<<<(B + 255) / 256, 256, 0, s>>>(Yb, Tb, B, dY, dYT, loss_part);
-  // layer 4
-  k_sur_bwd_weight<32, HID><<<blocks_for_waves(int64_t(1) * 5 * nch), 256, 0, s>>>(
-      dYT, NOUT, HT[4], B, chunk, part[4]);
-  k_sur_bwd_data<16><<<blocks_for_waves(4 * jbs), 256, 0, s>>>(WT[4], dY, Zt[3], B, dZ[3], dZT[3]);
-  // layers 3, 2, 1
-  for (int l = 3; l >= 1; --l) {
-    k_sur_bwd_weight<HID, HID><<<blocks_for_waves(int64_t(4) * 5 * nch), 256, 0, s>>>(
-        dZT[l], HID, HT[l], B, chunk, part[l]);
-    k_sur_bwd_data<HID><<<blocks_for_waves(4 * jbs), 256, 0, s>>>(WT[l], dZ[l], Zt[l - 1], B,
-                                                                  dZ[l - 1], dZT[l - 1]);
+  WeightGradArgs G;
+  G.chunk = chunk;
+  G.nch = nch;
+  G.first[0] = 0;
+  for (int l = 0; l < 5; ++l) {
+    G.act[l] = act[l];
+    G.err[l] = err[l];
+    G.partial[l] = part[l];
+    G.first[l + 1] = G.first[l] + grad_tiles(l) * nch;
   }
-  // layer 0 (inputs X0^T, 16 columns)
-  k_sur_bwd_weight<HID, K0><<<blocks_for_waves(int64_t(4) * 1 * nch), 256, 0, s>>>(
-      dZT[0], HID, X0T, B, chunk, part[0]);
+  k_sur_weight_gradients<<<unsigned(G.first[5]), 64, 0, s>>>(G);
   hipError_t e = hipGetLastError();
   if (e) return e;
-  const int nin[5] = {NIN, HID, HID, HID, HID}, nout[5] = {HID, HID, HID, HID, NOUT};
-  const int kc[5] = {K0, HID, HID, HID, HID};
   const int offw[5] = {OFF_W0, OFF_W1, OFF_W2, OFF_W3, OFF_W4};
   const int offb[5] = {OFF_B0, OFF_B1, OFF_B2, OFF_B3, OFF_B4};
   const float b1 = 0.9f, b2 = 0.999f;
   if (!grad_only) ++step;
   const float bc1 = 1.f - std::pow(b1, float(std::max<int64_t>(step, 1)));
   const float bc2 = 1.f - std::pow(b2, float(std::max<int64_t>(step, 1)));
+  UpdateArgs U;
+  U.threads = 0;
   for (int l = 0; l < 5; ++l) {
-    LayerDesc L;
-    L.nout = nout[l]; L.nin = nin[l]; L.kc = kc[l];
-    L.off_w = offw[l]; L.off_b = offb[l];
+    LayerDesc& L = U.layer[l];
+    L.nout = l == 4 ? NOUT : HID;
+    L.nin = l == 0 ? NIN : HID;
+    L.kc = act_rows(l);
+    L.off_w = offw[l];
+    L.off_b = offb[l];
     L.partial = part[l];
-    L.Wbf = Wbf[l];
-    L.kbf = l == 0 ? K0 : HID;
-    L.WT = l == 0 ? nullptr : WT[l];
-    L.ktp = l == 4 ? 16 : HID;
-    const int cnt = L.nout * L.nin + L.nout;
-    k_sur_update<<<(cnt + 255) / 256, 256, 0, s>>>(L, nch, params, m1, m2, lr, b1, b2, 1e-8f, bc1,
-                                                   bc2, grad_only ? grad : nullptr);
+    L.W = Wbf[l];
+    L.WT = WT[l];
+    L.first = U.threads;
+    U.threads += L.nout * L.nin + L.nout;
   }
+  k_sur_update<<<(U.threads + 255) / 256, 256, 0, s>>>(U, nch, params, m1, m2, lr, b1, b2, 1e-8f,
+                                                       bc1, bc2, grad_only ? grad : nullptr);
   return hipGetLastError();
 }
 
@@ -654,29 +809,23 @@ hipError_t Surrogate::train(hipStream_t s, int iterations, int B, double lr0, ui
     if (it < warm) lr = lr0 * double(it + 1) / warm;
     else lr = lr0 * (0.01 + 0.99 * 0.5 * (1 + std::cos(M_PI * double(it - warm) /
                                                       double(std::max(1, iterations - warm)))));
-    k_sur_batch<<<(B + 255) / 256, 256, 0, s>>>(X, T, nsamples, B, seed, it, 1, X0, X0T, Tb);
-    if ((e = pass(s, B, false, float(lr)))) return e;
+    if ((e = run_pass(s, X, T, nsamples, B, seed, it, true, false)) ||
+        (e = apply(s, B, false, float(lr))))
+      return e;
   }
   if ((e = refresh(s))) return e;
   // loss of the last batch (after the final update, on the same batch)
-  if ((e = batch_loss(s, B, &loss))) return e;
+  if ((e = run_pass(s, X, T, nsamples, B, seed, iterations - 1, false, true)) ||
+      (e = batch_loss(s, B, &loss)))
+    return e;
   if (final_loss) *final_loss = loss;
   return hipSuccess;
 }
 
+// mean squared error of the outputs that the last pass wrote
 hipError_t Surrogate::batch_loss(hipStream_t s, int B, double* loss) {
-  // forward only, reusing the pass kernels' first half
-  const int64_t jbs = B / 32;
-  k_sur_fwd<K0, HID, true><<<blocks_for_waves(4 * jbs), 256, 0, s>>>(
-      X0, Wbf[0], params + OFF_B0, HID, B, Zt[0], H[1], HT[1], nullptr);
-  for (int l = 1; l <= 3; ++l)
-    k_sur_fwd<HID, HID, true><<<blocks_for_waves(4 * jbs), 256, 0, s>>>(
-        H[l], Wbf[l], params + (l == 1 ? OFF_B1 : l == 2 ? OFF_B2 : OFF_B3), HID, B, Zt[l],
-        H[l + 1], HT[l + 1], nullptr);
-  k_sur_fwd<HID, 32, false><<<blocks_for_waves(jbs), 256, 0, s>>>(
-      H[4], Wbf[4], params + OFF_B4, NOUT, B, nullptr, nullptr, nullptr, Yb);
   const int nb = (B + 255) / 256;
-  k_sur_loss<<<nb, 256, 0, s>>>(Yb, Tb, B, dY, dYT, loss_part);
+  k_sur_loss<<<nb, 256, 0, s>>>(Yb, Tb, B, loss_part);
   hipError_t e = hipGetLastError();
   if (e) return e;
   std::vector<float> h(nb);
@@ -699,10 +848,9 @@ hipError_t Surrogate::gradients(hipStream_t s, int64_t n, const float* x_host, c
   if ((e = hipMemcpyAsync(io_x, x_host, size_t(n) * 7 * 4, hipMemcpyHostToDevice, s)) ||
       (e = hipMemcpyAsync(tdev, t_host, size_t(n) * 7 * 4, hipMemcpyHostToDevice, s)))
     return e;
-  k_sur_batch<<<(B + 255) / 256, 256, 0, s>>>(io_x, tdev, n, B, 0, 0, 0, X0, X0T, Tb);
-  if ((e = pass(s, B, true, 0.f))) return e;
+  if ((e = run_pass(s, io_x, tdev, n, B, 0, -1, true, true)) || (e = apply(s, B, true, 0.f)))
+    return e;
   if ((e = hipMemcpyAsync(grad_host, grad, NPARAM * 4, hipMemcpyDeviceToHost, s))) return e;
-  // loss with the same (unchanged) parameters
   return batch_loss(s, B, loss);
 }
 

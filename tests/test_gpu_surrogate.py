@@ -105,6 +105,47 @@ def test_training_gradients_match_reference():
     assert np.linalg.norm(g - ge) / np.linalg.norm(ge) < 5e-2
 
 
+@pytest.mark.parametrize("n", [256, 768, 1024, 3072])
+def test_gradients_over_chunk_shapes(n):
+    """Batches of one and several split-K chunks of 256 and of 1,024 points,
+    against the CPU reference with the same BF16 rounding points."""
+    model = _plate_model()
+    p = ref.init_params(23).astype(np.float32)
+    model.surrogate_params(p)
+    rng = np.random.default_rng(n)
+    x = rng.uniform(-1, 1, size=(n, 7)).astype(np.float32)
+    t = rng.normal(scale=0.3, size=(n, 7)).astype(np.float32)
+    g, loss = model.surrogate_gradients(x, t)
+    lr, gr = ref.loss_and_grad(p.astype(np.float64), x, t, rounded=True)
+    assert abs(loss - lr) <= 1e-3 * lr
+    offs = np.cumsum([0] + [int(np.prod(s)) for _, s in ref.SHAPES])
+    for (name, _), a, b in zip(ref.SHAPES, offs[:-1], offs[1:]):
+        err = np.linalg.norm(g[a:b] - gr[a:b]) / np.linalg.norm(gr[a:b])
+        assert err < 2e-2, (name, err)
+
+
+def _mix64(z):
+    """SplitMix64's finaliser, as the minibatch draw uses it."""
+    m = (1 << 64) - 1
+    z = (z + 0x9E3779B97F4A7C15) & m
+    z = ((z ^ (z >> 30)) * 0xBF58476D1CE4E5B9) & m
+    z = ((z ^ (z >> 27)) * 0x94D049BB133111EB) & m
+    return z ^ (z >> 31)
+
+
+def test_training_loss_is_the_last_batchs():
+    """The loss that training returns is the trained network's on the batch of
+    the last iteration: the forward-only pass, on the same draw."""
+    model = _plate_model()
+    model.surrogate_generate(100, 30, seed=5)
+    x, t = model.surrogate_dataset(0, 3000)
+    iters, batch, seed = 3, 512, 9
+    loss = model.surrogate_train(iters, batch=batch, seed=seed)
+    rows = [_mix64(seed ^ _mix64((iters - 1) * batch + b)) % 3000 for b in range(batch)]
+    _, again = model.surrogate_gradients(x[rows], t[rows])
+    assert loss == again
+
+
 def test_training_set_follows_the_plain_law():
     model = _plate_model()
     model.surrogate_generate(400, 250, seed=3)
