@@ -284,14 +284,23 @@ void to_internal_points(const akx_ctx* c, const T* src, T* dst, int comp) {
     std::memcpy(dst + size_t(e) * per, src + size_t(c->elem_perm[e]) * per, per * sizeof(T));
 }
 
+// The slot layout a launch takes: the one set, else element-ordered slots on
+// the mixed path (another layout would round differently) and, on the FP64
+// path, where all layouts give the same bits, the fused step (fused_default)
+// or node-ordered slots: the node kernel streams them where it would gather
+// element-ordered ones (64,000 neo-Hookean hexahedra: 14.4 -> 10.1 us, 1 M
+// 126 -> 69; the element kernel's scattered stores cost 0 and 38 us of that).
+int layout_of(const akx_ctx* c, int precision) {
+  if (c->layout_set || precision == AKX_MIXED) return c->node_ordered;
+  return c->fused_default ? 6 : 1;
+}
+
 // Step fused over node blocks (slot layout 6): one launch per step, no force
 // slots; stateless laws of a single kind on elements of up to 4 nodes, FP64
 // or mixed.  The FP64 path takes it by default (fused_default): it gives the
 // slots' bits.
 bool uses_fused(const akx_ctx* c, int precision) {
-  const bool asked = c->layout_set ? c->node_ordered == 6
-                                   : precision == AKX_FP64 && c->fused_default;
-  return asked && c->fused_ok && (precision == AKX_MIXED || c->fsrec) &&
+  return layout_of(c, precision) == 6 && c->fused_ok && (precision == AKX_MIXED || c->fsrec) &&
          c->groups.size() == 1 && !c->groups[0].filter &&
          !(c->sur.enabled && c->groups[0].kind == AKX_MATERIAL_NEOHOOKEAN_DAMAGE);
 }
@@ -303,7 +312,8 @@ bool uses_fused(const akx_ctx* c, int precision) {
 // node's place in a node-major list (5); the node kernel sums a node's
 // partials in FP64.  Needs the LDS patches and a single launch group.
 bool uses_partials(const akx_ctx* c, int precision) {
-  return precision == AKX_MIXED && c->node_ordered >= 3 && c->node_ordered <= 6 &&
+  const int lay = layout_of(c, precision);
+  return precision == AKX_MIXED && lay >= 3 && lay <= 6 &&
          !uses_fused(c, precision) &&
          c->patch_ok && c->groups.size() == 1 &&
          !c->groups[0].filter &&
@@ -334,10 +344,11 @@ ElemArgs elem_args(akx_ctx* c, const KindGroup& g, int precision) {
   A.recompute = c->mixed_recompute;
   A.X = c->X;
   A.safe_division = c->safe_division;
-  A.slot_pos = !c->node_ordered ? nullptr : precision == AKX_MIXED ? c->slot2_pos : c->slot_pos;
-  A.patch = (precision == AKX_MIXED && c->node_ordered >= 2 && c->patch_ok && !g.filter) ? 1 : 0;
-  A.partials = (A.patch && uses_partials(c, precision)) ? (c->node_ordered == 3 ? 1 : 2) : 0;
-  A.part_pos = (A.partials && c->node_ordered >= 5) ? c->ppos : nullptr;
+  const int lay = layout_of(c, precision);
+  A.slot_pos = !lay ? nullptr : precision == AKX_MIXED ? c->slot2_pos : c->slot_pos;
+  A.patch = (precision == AKX_MIXED && lay >= 2 && c->patch_ok && !g.filter) ? 1 : 0;
+  A.partials = (A.patch && uses_partials(c, precision)) ? (lay == 3 ? 1 : 2) : 0;
+  A.part_pos = (A.partials && lay >= 5) ? c->ppos : nullptr;
   A.patch_max_nodes = c->patch_max_nodes;
   A.patch_lds = c->patch_lds;
   A.patch_blocks = c->patch_blocks;
@@ -392,19 +403,20 @@ NodeArgs node_args(akx_ctx* c, int mode, int precision) {
   for (int i = 0; i < 3; ++i) A.bc_inc[i] = c->bc_inc[i];
   A.mode = mode;
   A.xcd_remap = c->xcd_remap;
-  A.node_ordered = c->node_ordered;
+  const int lay = layout_of(c, precision);
+  A.node_ordered = lay;
   A.stage_lds = 0;
   A.partials = 0;
   if (uses_partials(c, precision)) {
-    A.partials = c->node_ordered == 3 ? 1 : 2;
+    A.partials = lay == 3 ? 1 : 2;
     // one partial sum per (patch, node): a short gather per node, or a
     // contiguous run per node when the partials are node-ordered
     A.csr_off = c->pcsr_off;
     A.csr_slot = c->pentry;
-    A.node_ordered = c->node_ordered >= 5 ? 1 : 0;
+    A.node_ordered = lay >= 5 ? 1 : 0;
     return A;
   }
-  if (c->node_ordered && c->node_stage) {
+  if (lay && c->node_stage) {
     // static LDS of k_node is at most 4 * 256 * 3 * 8 + 256 * 3 bytes (< 26 KiB)
     const size_t bytes = size_t(c->span_max[c->node_block / 64 - 1]) * c->d *
                          (precision == AKX_FP64 ? 8 : 4);

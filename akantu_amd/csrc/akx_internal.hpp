@@ -381,9 +381,7 @@ struct akx_ctx {
 
   int elem_block = 256, node_block = 256, xcd_remap = 1, mixed_recompute = 1;
   int node_ordered = 0;             // slot layout (see store_slots)
-  // set by akx_set_launch or the autotuner; until then the FP64 path takes the
-  // fused step wherever it applies (the same bits as the element-ordered slots
-  // of layout 0, the mixed path's default)
+  // set by akx_set_launch or the autotuner (until then: layout_of)
   bool layout_set = false;
   int node_stage = 1;               // node kernel copies its slot range to LDS when it fits
   uint32_t span_max[4] = {0, 0, 0, 0};  // largest slot range of a node block of 64, 128, 192, 256

@@ -281,6 +281,123 @@ __global__ void __launch_bounds__(256) k_element_fp64(ElemArgs A) {
 }
 
 // ===========================================================================
+// element kernel, FP64, 8-node hexahedron: one lane per quadrature point
+//   8 lanes hold an element's points (so q = lane % 8), a wave 8 elements.
+//   The lanes fetch one node each and share the element through LDS, as they
+//   do dN/dxi of the points; each evaluates its point in the reference's
+//   order; then the lanes exchange their 24 contributions through LDS, 8 at a
+//   time, and each adds one component over the points q = 0..7, the sum the
+//   thread-per-element form carried from point to point.  LDS traffic stays
+//   within the wave, so the exchange needs no block barrier.
+//   Bound: FP64 instructions (about 1,430 a neo-Hookean point, 624 of them the
+//   residual's): 1 M elements in 355 us, of which the instructions are 290.
+//   One thread per element, looping over its points (409 us there), left a
+//   mesh of 64,000 elements one wave per SIMD (42 us against 33) and took 35
+//   us for 216 elements against 9; B read from the tables would be 200 bytes
+//   a point.
+// ===========================================================================
+// Makes a wave's own LDS writes precede its later reads: LDS operations of one
+// wave execute in order, so this only has to hold the compiler.
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+template <int KIND>
+__global__ void __launch_bounds__(256) k_element_hex8_fp64(ElemArgs A) {
+  constexpr int d = 3, n = 8, dn = 24;
+  // row strides (doubles) keep 16-byte reads of 8 or 16 rows off each other's
+  // banks
+  constexpr int TS = 26, ES = 50, FS = 10;
+  __shared__ __align__(16) double s_tab[8 * TS];     // dN/dxi of point q, weight
+  __shared__ __align__(16) double s_w[4][64 * FS];   // elements, then contributions
+  const int lane = threadIdx.x & 63, q = lane & 7, el = lane >> 3;
+  for (int k = threadIdx.x; k < 8 * 25; k += blockDim.x) {
+    const int r = k / 25, c = k - r * 25;
+    s_tab[r * TS + c] = c < dn ? A.tab64->dnds[r][c] : A.tab64->w[r];
+  }
+  const int64_t first = (logical_block(A.xcd_remap) * blockDim.x + threadIdx.x) >> 3;
+  const bool live = first < A.count;
+  const int64_t t = live ? first : A.count - 1;  // count > 0
+  const int64_t E = A.E;
+  const int64_t e = A.filter ? int64_t(A.filter[t]) : t;
+  double* sw = s_w[threadIdx.x >> 6];
+  {
+    // FEEngine::extractNodalToElementField (fe_engine_inline_impl.hh:104-143)
+    const int64_t node = A.conn[q * E + e];
+    double* to = sw + el * ES + q * 6;
+#pragma unroll
+    for (int i = 0; i < d; ++i) {
+      to[i] = A.u[node * d + i];
+      to[d + i] = A.X[node * d + i];
+    }
+  }
+  const MatParams m = A.mats[A.elem_mat ? A.elem_mat[e] : 0];
+  __syncthreads();
+  const double* se = sw + el * ES;
+  double D[dn], B[dn], R[dn], J[d * d], Ji[d * d], G[d * d], S[d * d];
+  const double w = s_tab[q * TS + dn];
+#pragma unroll
+  for (int k = 0; k < dn; ++k) D[k] = s_tab[q * TS + k];
+  {
+    double xe[dn];
+#pragma unroll
+    for (int a = 0; a < n; ++a)
+#pragma unroll
+      for (int i = 0; i < d; ++i) xe[i + a * d] = se[a * 6 + d + i];
+    force_productt<d, d, n>(D, xe, J);
+  }
+  const double jq = inv_det<d>(J, A.safe_division, Ji) * w;
+  force_product<d, n, d>(Ji, D, B);
+  {
+    // grad u = u_e B^T (shape_functions_inline_impl.hh:388, Matrix::mul<false, true>)
+    double ue[dn];
+#pragma unroll
+    for (int a = 0; a < n; ++a)
+#pragma unroll
+      for (int i = 0; i < d; ++i) ue[i + a * d] = se[a * 6 + i];
+    force_productt<d, d, n>(ue, B, G);
+  }
+  if constexpr (KIND == ELASTIC) {
+    elastic_stress_force<d>(m, G, S);
+    // B^T sigma computed as sigma B (shape_lagrange_inline_impl.hh:421)
+    force_product<d, n, d>(S, B, R);
+  } else {
+    if constexpr (KIND == NEOHOOKEAN) {
+      neohookean_stress_ref<d>(m, G, S);
+    } else {
+      const int64_t eq = e * 8 + q;
+      double dam = A.damage[eq];
+      nh_damage_stress_ref<d>(m, G, S, dam, A.Yd[eq]);
+      if (live) A.damage[eq] = dam;
+    }
+    finite_residual_ref<d, n>(B, G, S, R);
+  }
+  // IntegratorGauss::integrate (integrator_gauss_inline_impl.hh:446-452): lane
+  // (el, c) adds component 8 r + c over the points
+  double* __restrict__ out = static_cast<double*>(A.slots);
+#pragma unroll
+  for (int r = 0; r < 3; ++r) {
+    wave_lds_sync();
+#pragma unroll
+    for (int c = 0; c < 8; ++c) sw[(el * 8 + c) * FS + q] = R[8 * r + c] * jq;
+    wave_lds_sync();
+    double v[8];
+#pragma unroll
+    for (int p = 0; p < 8; ++p) v[p] = sw[lane * FS + p];
+    double f = v[0];
+#pragma unroll
+    for (int p = 1; p < 8; ++p) f += v[p];
+    const int k = 8 * r + q;
+    if (live) {
+      if (A.slot_pos) out[int64_t(A.slot_pos[int64_t(k / d) * E + e]) * d + k % d] = f;
+      else out[e * dn + k] = f;
+    }
+  }
+}
+
+// ===========================================================================
 // element kernel, FP32 element math (mixed precision)
 //   RECOMPUTE = false: B and det(J) w read from the FP32 tables;
 //   RECOMPUTE = true:  both rebuilt per point from the element's coordinates
@@ -2184,6 +2301,19 @@ static hipError_t launch_element_et(int kind, int precision, hipStream_t s, cons
                                     int block) {
   const unsigned g = grid_for(A.count, block);
   if (precision == 0) {
+    if constexpr (ET == HEX8) {
+      // one lane per point; B always rebuilt (the tables' bits); blocks of 256,
+      // which share the points' table (64: 139 against 101 us on 262,000
+      // neo-Hookean hexahedra)
+      const unsigned gq = grid_for(A.count * 8, 256);
+      switch (kind) {
+      case ELASTIC: k_element_hex8_fp64<ELASTIC><<<gq, 256, 0, s>>>(A); break;
+      case NEOHOOKEAN: k_element_hex8_fp64<NEOHOOKEAN><<<gq, 256, 0, s>>>(A); break;
+      case NH_DAMAGE: k_element_hex8_fp64<NH_DAMAGE><<<gq, 256, 0, s>>>(A); break;
+      default: return hipErrorInvalidValue;
+      }
+      return hipGetLastError();
+    } else
     switch (kind) {
     case ELASTIC:
       if (A.recompute) k_element_fp64<ET, ELASTIC, true><<<g, block, 0, s>>>(A);

@@ -234,7 +234,8 @@ int akx_last_step_timing(akx_ctx* ctx, double* element_ms, double* node_ms);
  * that recompute the elements around their nodes, on either path; stateless
  * laws of one kind on elements of up to 4 nodes -- elsewhere the FP64 path
  * runs 6 as node-ordered slots and the mixed path as 5; until a layout is set
- * or autotuned, the FP64 path takes 6 where it applies), and whether the node
+ * or autotuned, the FP64 path takes 6 or 1, the faster one, and the mixed path
+ * 0), and whether the node
  * kernel copies its block's contiguous slot range to LDS first (node_stage
  * 1/0) (-1 keeps).  On the FP64 path none of these changes a result bit; on
  * the mixed path layouts 0/1, 2, 3 and 4/5 differ in rounding only
