@@ -2155,6 +2155,8 @@ FeArgs fe_args(akx_ctx* c, const uint32_t* filt, int64_t count, int nb) {
   A.B = c->B64;
   A.J = c->J64;
   A.tab = make_tables(c->et);
+  A.tab64 = c->tab64_d;
+  A.X = c->X;
   A.nb = nb;
   return A;
 }

@@ -16,11 +16,11 @@
 // Element-indexed inputs and outputs are rows in the order of the element list
 // the caller gave (t), while the element tables are read at the element's
 // internal id (filt[t]).  Nodal arrays are in the internal node numbering.
-// These run once per operator call; they are written for clarity of the
-// reference order, one thread per element (or per element and component).
 #include <hip/hip_runtime.h>
 
 #include <hipcub/hipcub.hpp>
+
+#include <algorithm>
 
 #include "akx_internal.hpp"
 
@@ -32,103 +32,161 @@ __device__ __forceinline__ int64_t elem_of(const FeArgs& A, int64_t t) {
   return A.filt ? int64_t(A.filt[t]) : t;
 }
 
+// The operators that need B or N work one thread per point (rows r = t Q + q of
+// the per-point arrays, so that a wave's rows are contiguous): the points' dN/dxi
+// and N are staged in LDS and B is rebuilt from the coordinates in the
+// precompute's arithmetic (its bits).  The list's elements are in the caller's
+// order, so B read from the tables would be one 8-byte value per cache line
+// and entry, where the coordinates of an element's nodes are a few lines for
+// all of its points.  27,000 hexahedra, 3 components, against one thread per
+// element reading the tables with its operands in scratch memory: gradient
+// 94 -> 21 us, computeBtD 135 -> 26, interpolation 26 -> 10.
+struct PointTables {
+  double dnds[8][24], N[8][8];
+};
+template <int ET>
+__device__ __forceinline__ void stage_points(PointTables& s, const ElemTables* tab) {
+  using T = Elem<ET>;
+  constexpr int d = T::d, n = T::n, Q = T::Q;
+  for (int k = threadIdx.x; k < Q * d * n; k += 256)
+    s.dnds[k / (d * n)][k % (d * n)] = tab->dnds[k / (d * n)][k % (d * n)];
+  for (int k = threadIdx.x; k < Q * n; k += 256) s.N[k / n][k % n] = tab->N[k / n][k % n];
+  __syncthreads();
+}
+
+// B of point q of element e (element_class_tmpl.hh:282-355; k_precompute)
+template <int ET>
+__device__ __forceinline__ void point_b(const FeArgs& A, const double* dnds, int64_t e,
+                                        double* B) {
+  using T = Elem<ET>;
+  constexpr int d = T::d, n = T::n;
+  double xe[d * n], J[d * d], Ji[d * d];
+#pragma unroll
+  for (int a = 0; a < n; ++a) {
+    const int64_t node = A.conn[a * A.E + e];
+#pragma unroll
+    for (int i = 0; i < d; ++i) xe[i + a * d] = A.X[node * d + i];
+  }
+  matrix_matrixt<d, d, n>(dnds, xe, J);
+  invn<d>(J, Ji);
+  matrix_matrix<d, n, d>(Ji, dnds, B);
+}
+
 template <int ET>
 __global__ void __launch_bounds__(256) k_fe_gradient(FeArgs A) {
   using T = Elem<ET>;
-  constexpr int d = T::d, n = T::n, Q = T::Q, dn = d * n;
-  const int64_t t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (t >= A.count) return;
-  const int64_t e = elem_of(A, t), E = A.E;
+  constexpr int d = T::d, n = T::n, Q = T::Q;
+  __shared__ PointTables s_p;
+  stage_points<ET>(s_p, A.tab64);
+  const int64_t r = int64_t(blockIdx.x) * 256 + threadIdx.x;
+  if (r >= A.count * Q) return;
+  const int64_t t = r / Q;
+  const int64_t e = elem_of(A, t);
   const int nb = A.nb;
-  double ue[FE_MAX_DOF * 8];
-  for (int a = 0; a < n; ++a) {
-    const int64_t node = A.conn[a * E + e];
-    for (int i = 0; i < nb; ++i) ue[i + a * nb] = A.in[node * nb + i];
-  }
-  for (int q = 0; q < Q; ++q) {
-    double Bq[dn];
+  double B[d * n];
+  point_b<ET>(A, s_p.dnds[r - t * Q], e, B);
+  int64_t node[n];
 #pragma unroll
-    for (int k = 0; k < dn; ++k) Bq[k] = A.B[(int64_t(q) * dn + k) * E + e];
-    double* o = A.out + (t * Q + q) * nb * d;
-    // nabla_u (nb x d) = u_e (nb x n) * B^T, B (d x n)
-    for (int j = 0; j < d; ++j)
-      for (int i = 0; i < nb; ++i) {
-        double s = 0.;
+  for (int a = 0; a < n; ++a) node[a] = A.conn[a * A.E + e];
+  // nabla_u (nb x d) = u_e (nb x n) * B^T, B (d x n)
+  double* o = A.out + r * nb * d;
+  for (int i = 0; i < nb; ++i) {
+    double u[n];
 #pragma unroll
-        for (int l = 0; l < n; ++l) s += ue[i + l * nb] * Bq[j + l * d];
-        o[i + j * nb] = s;
-      }
+    for (int a = 0; a < n; ++a) u[a] = A.in[node[a] * nb + i];
+#pragma unroll
+    for (int j = 0; j < d; ++j) {
+      double s = 0.;
+#pragma unroll
+      for (int l = 0; l < n; ++l) s += u[l] * B[j + l * d];
+      o[i + j * nb] = s;
+    }
   }
 }
 
+// one thread per value: uq (nb x Q) = u_e (nb x n) * N (n x Q)
 template <int ET>
 __global__ void __launch_bounds__(256) k_fe_interpolate(FeArgs A) {
   using T = Elem<ET>;
   constexpr int n = T::n, Q = T::Q;
-  const int64_t t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (t >= A.count) return;
-  const int64_t e = elem_of(A, t), E = A.E;
+  __shared__ PointTables s_p;
+  stage_points<ET>(s_p, A.tab64);
   const int nb = A.nb;
-  double ue[FE_MAX_DOF * 8];
-  for (int a = 0; a < n; ++a) {
-    const int64_t node = A.conn[a * E + e];
-    for (int i = 0; i < nb; ++i) ue[i + a * nb] = A.in[node * nb + i];
-  }
-  // uq (nb x Q) = u_e (nb x n) * N (n x Q)
-  double* o = A.out + t * Q * nb;
-  for (int q = 0; q < Q; ++q)
-    for (int i = 0; i < nb; ++i) {
-      double s = 0.;
+  const int64_t end = A.count * Q * nb;
+  for (int64_t k = int64_t(blockIdx.x) * 256 + threadIdx.x; k < end;
+       k += int64_t(gridDim.x) * 256) {
+    const int64_t r = k / nb, t = r / Q;
+    const int i = int(k - r * nb), q = int(r - t * Q);
+    const int64_t e = elem_of(A, t);
+    double s = 0.;
 #pragma unroll
-      for (int l = 0; l < n; ++l) s += ue[i + l * nb] * A.tab.N[q][l];
-      o[i + q * nb] = s;
-    }
+    for (int l = 0; l < n; ++l) s += A.in[int64_t(A.conn[l * A.E + e]) * nb + i] * s_p.N[q][l];
+    A.out[k] = s;
+  }
 }
 
-template <int ET>
+// ROWS > 0: rows of D known at compile time, a point's result leaves as one
+// run; 0: any count, row by row
+template <int ET, int ROWS>
 __global__ void __launch_bounds__(256) k_fe_btd(FeArgs A) {
   using T = Elem<ET>;
-  constexpr int d = T::d, n = T::n, Q = T::Q, dn = d * n;
-  const int64_t t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (t >= A.count) return;
-  const int64_t e = elem_of(A, t), E = A.E;
-  const int rows = A.nb;
-  for (int q = 0; q < Q; ++q) {
-    double Bq[dn];
+  constexpr int d = T::d, n = T::n, Q = T::Q;
+  __shared__ PointTables s_p;
+  stage_points<ET>(s_p, A.tab64);
+  const int64_t r = int64_t(blockIdx.x) * 256 + threadIdx.x;
+  if (r >= A.count * Q) return;
+  const int64_t t = r / Q;
+  double B[d * n];
+  point_b<ET>(A, s_p.dnds[r - t * Q], elem_of(A, t), B);
+  const int rows = ROWS ? ROWS : A.nb;
+  const double* D = A.in + r * rows * d;
+  double* o = A.out + r * rows * n;
+  // Bt_D (rows x n) = D (rows x d) * B (d x n)
+  if constexpr (ROWS > 0) {
+    double R[ROWS * n], Dr[ROWS * d];
 #pragma unroll
-    for (int k = 0; k < dn; ++k) Bq[k] = A.B[(int64_t(q) * dn + k) * E + e];
-    const int64_t r = t * Q + q;
-    const double* D = A.in + r * rows * d;
-    double* o = A.out + r * rows * n;
-    // Bt_D (rows x n) = D (rows x d) * B (d x n)
-    for (int j = 0; j < n; ++j)
-      for (int i = 0; i < rows; ++i) {
+    for (int k = 0; k < ROWS * d; ++k) Dr[k] = D[k];
+    matrix_matrix<ROWS, n, d>(Dr, B, R);
+    if constexpr (ROWS * n % 2 == 0) {
+#pragma unroll
+      for (int k = 0; k < ROWS * n / 2; ++k)
+        reinterpret_cast<double2*>(o)[k] = make_double2(R[2 * k], R[2 * k + 1]);
+    } else {
+#pragma unroll
+      for (int k = 0; k < ROWS * n; ++k) o[k] = R[k];
+    }
+  } else {
+    for (int i = 0; i < rows; ++i) {
+      double Di[d];
+#pragma unroll
+      for (int l = 0; l < d; ++l) Di[l] = D[i + l * rows];
+#pragma unroll
+      for (int j = 0; j < n; ++j) {
         double s = 0.;
 #pragma unroll
-        for (int l = 0; l < d; ++l) s += D[i + l * rows] * Bq[l + j * d];
+        for (int l = 0; l < d; ++l) s += Di[l] * B[l + j * d];
         o[i + j * rows] = s;
       }
+    }
   }
 }
 
+// one thread per value: Ntb (nb x n) = b (nb x 1) * N (1 x n)
 template <int ET>
 __global__ void __launch_bounds__(256) k_fe_ntb(FeArgs A) {
   using T = Elem<ET>;
   constexpr int n = T::n, Q = T::Q;
-  const int64_t t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (t >= A.count) return;
+  __shared__ PointTables s_p;
+  stage_points<ET>(s_p, A.tab64);
   const int nb = A.nb;
-  for (int q = 0; q < Q; ++q) {
-    const int64_t r = t * Q + q;
-    const double* b = A.in + r * nb;
-    double* o = A.out + r * nb * n;
-    // Ntb (nb x n) = b (nb x 1) * N (1 x n)
-    for (int j = 0; j < n; ++j)
-      for (int i = 0; i < nb; ++i) {
-        double s = 0.;
-        s += b[i] * A.tab.N[q][j];
-        o[i + j * nb] = s;
-      }
+  const int64_t end = A.count * Q * nb * n;
+  for (int64_t k = int64_t(blockIdx.x) * 256 + threadIdx.x; k < end;
+       k += int64_t(gridDim.x) * 256) {
+    const int64_t r = k / (nb * n);
+    const int c = int(k - r * (nb * n)), j = c / nb, i = c - j * nb, q = int(r % Q);
+    double s = 0.;
+    s += A.in[r * nb + i] * s_p.N[q][j];
+    A.out[k] = s;
   }
 }
 
@@ -350,6 +408,10 @@ __global__ void __launch_bounds__(256) k_mat_gather(int64_t N, int d, int n, int
 
 inline void clear_error() { (void)hipGetLastError(); }
 inline unsigned grid_for(int64_t n) { return unsigned((n + 255) / 256); }
+// for kernels whose threads go on with a stride: within a launch's 2^32 threads
+inline unsigned grid_striding(int64_t n) {
+  return unsigned(std::min<int64_t>((n + 255) / 256, 1 << 20));
+}
 
 #define AKX_FE_SWITCH(et, F)              \
   switch (et) {                           \
@@ -369,22 +431,28 @@ hipError_t launch_fe(int op, int et, hipStream_t s, const FeArgs& A) {
   const int Q = et == QUAD4 ? 4 : et == HEX8 ? 8 : 1;
   switch (op) {
   case FE_GRADIENT:
-#define F(ET) k_fe_gradient<ET><<<grid_for(A.count), 256, 0, s>>>(A)
+#define F(ET) k_fe_gradient<ET><<<grid_for(A.count * Q), 256, 0, s>>>(A)
     AKX_FE_SWITCH(et, F)
 #undef F
     break;
   case FE_INTERPOLATE:
-#define F(ET) k_fe_interpolate<ET><<<grid_for(A.count), 256, 0, s>>>(A)
+#define F(ET) k_fe_interpolate<ET><<<grid_striding(A.count * Q * A.nb), 256, 0, s>>>(A)
     AKX_FE_SWITCH(et, F)
 #undef F
     break;
   case FE_BTD:
-#define F(ET) k_fe_btd<ET><<<grid_for(A.count), 256, 0, s>>>(A)
+#define F(ET)                                                              \
+  switch (A.nb) {                                                          \
+  case 1: k_fe_btd<ET, 1><<<grid_for(A.count * Q), 256, 0, s>>>(A); break; \
+  case 2: k_fe_btd<ET, 2><<<grid_for(A.count * Q), 256, 0, s>>>(A); break; \
+  case 3: k_fe_btd<ET, 3><<<grid_for(A.count * Q), 256, 0, s>>>(A); break; \
+  default: k_fe_btd<ET, 0><<<grid_for(A.count * Q), 256, 0, s>>>(A);       \
+  }
     AKX_FE_SWITCH(et, F)
 #undef F
     break;
   case FE_NTB:
-#define F(ET) k_fe_ntb<ET><<<grid_for(A.count), 256, 0, s>>>(A)
+#define F(ET) k_fe_ntb<ET><<<grid_striding(A.count * Q * A.nb * n), 256, 0, s>>>(A)
     AKX_FE_SWITCH(et, F)
 #undef F
     break;

@@ -248,6 +248,8 @@ struct FeArgs {
   const double* B;        // [(q*dn + k)][E]
   const double* J;        // [q][E]
   ElemTables tab;         // N of the quadrature points
+  const ElemTables* tab64; // the same tables in device memory
+  const double* X;        // (N, d) reference coordinates
   const double* in;       // operand: nodal (internal numbering) or per-element rows
   double* out;            // result rows
   int nb;                 // components of the operand (rows of D for computeBtD)
