@@ -202,7 +202,7 @@ class FEEngine:
     def _op(self, fn, arr, nb, out_cols, elements):
         arr = np.ascontiguousarray(arr, dtype=np.float64)
         p, n, keep = _elements(elements)
-        out = np.zeros((self._count(elements) * self.nb_qp, out_cols))
+        out = np.empty((self._count(elements) * self.nb_qp, out_cols))
         self.ctx.check(fn(self.ctx.h, _ptr(arr), int(nb), p, n, _ptr(out)))
         return out
 
@@ -232,7 +232,7 @@ class FEEngine:
         f = np.ascontiguousarray(f, dtype=np.float64)
         nb = nb_degree_of_freedom or (f.shape[1] if f.ndim == 2 else 1)
         p, n, keep = _elements(elements)
-        out = np.zeros((self._count(elements), nb))
+        out = np.empty((self._count(elements), nb))
         self.ctx.check(lib.akx_fe_integrate(self.ctx.h, _ptr(f), int(nb), p, n, _ptr(out)))
         return out
 
@@ -387,7 +387,7 @@ class SolidMechanicsModel:
     def material_compute_stress(self, mat_id, grad_u):
         """Material::computeStress on the material's points from given gradients."""
         g = np.ascontiguousarray(grad_u, dtype=np.float64)
-        out = np.zeros_like(g)
+        out = np.empty_like(g)
         self.ctx.check(lib.akx_material_compute_stress(self.ctx.h, int(mat_id), _ptr(g),
                                                        _ptr(out)))
         return out
@@ -448,7 +448,7 @@ class SolidMechanicsModel:
 
     def surrogate_infer(self, x):
         x = np.ascontiguousarray(x, dtype=np.float32)
-        y = np.zeros_like(x)
+        y = np.empty_like(x)
         self.ctx.check(lib.akx_surrogate_infer(self.ctx.h, x.shape[0], _ptr(x), _ptr(y)))
         return y
 
@@ -506,7 +506,7 @@ class SolidMechanicsModel:
 
     def get(self, name):
         dtype = np.uint8 if name == "blocked_dofs" else np.float64
-        out = np.zeros(self._shape(name), dtype=dtype)
+        out = np.empty(self._shape(name), dtype=dtype)
         self.ctx.check(lib.akx_field_download(self.ctx.h, FIELDS[name], _ptr(out), out.nbytes))
         if name == "blocked_dofs":
             return out.astype(bool)

@@ -98,6 +98,7 @@ void free_graph(akx_ctx* c) {
 
 void free_mesh_buffers(akx_ctx* c) {
   free_graph(c);
+  c->scratch.release();
   dfree(c->dt_node);
   free_derived(c);
   dfree(c->X); dfree(c->conn_soa);
@@ -791,6 +792,53 @@ int build_fused(akx_ctx* c, const std::vector<uint32_t>& order, const std::vecto
   return AKX_OK;
 }
 
+// caller -> internal numbering on the device, built on first use (nothing for
+// contexts that keep the caller's numbering)
+int device_numbering(akx_ctx* c) {
+  if (!c->reorder) return AKX_OK;
+  if (!c->node_inv_d) {
+    HIP_TRY(c, dalloc(&c->node_inv_d, c->node_inv.size()));
+    HIP_TRY(c, hipMemcpy(c->node_inv_d, c->node_inv.data(), c->node_inv.size() * 4,
+                         hipMemcpyHostToDevice));
+  }
+  if (!c->elem_inv_d && !c->elem_inv.empty()) {
+    HIP_TRY(c, dalloc(&c->elem_inv_d, c->elem_inv.size()));
+    HIP_TRY(c, hipMemcpy(c->elem_inv_d, c->elem_inv.data(), c->elem_inv.size() * 4,
+                         hipMemcpyHostToDevice));
+  }
+  return AKX_OK;
+}
+
+// Rows of `width` doubles between a caller array in its own numbering and a
+// device array in the internal one (inv: caller -> internal, nullptr: equal).
+int upload_numbered(akx_ctx* c, int64_t rows, int width, const uint32_t* inv, const double* host,
+                    double* dev) {
+  const size_t bytes = size_t(rows) * width * 8;
+  if (!inv) {
+    HIP_TRY(c, c->copy.to_device(c->device, c->stream, dev, host, bytes));
+    return AKX_OK;
+  }
+  void* raw = nullptr;
+  HIP_TRY(c, c->scratch.take(bytes, &raw));
+  HIP_TRY(c, c->copy.to_device(c->device, c->stream, raw, host, bytes));
+  HIP_TRY(c, launch_scatter_rows(c->stream, rows, width, inv, static_cast<double*>(raw), dev));
+  return AKX_OK;
+}
+// dw values per row out of rows of sw (sw 1: repeated)
+int download_numbered(akx_ctx* c, int64_t rows, int dw, int sw, const uint32_t* inv,
+                      const double* dev, double* host) {
+  const size_t bytes = size_t(rows) * dw * 8;
+  const void* from = dev;
+  if (inv || dw != sw) {
+    void* raw = nullptr;
+    HIP_TRY(c, c->scratch.take(bytes, &raw));
+    HIP_TRY(c, launch_snapshot(c->stream, rows, dw, sw, inv, dev, raw, 8));
+    from = raw;
+  }
+  HIP_TRY(c, c->copy.to_host(c->device, c->stream, host, from, bytes));
+  return AKX_OK;
+}
+
 int read_blocked(akx_ctx* c, std::vector<uint8_t>& internal) {
   const size_t nd = size_t(c->N) * c->d;
   internal.resize(nd);
@@ -846,6 +894,7 @@ int akx_ctx_destroy(akx_ctx* c) {
   if (!c) return AKX_ERR_ARGUMENT;
   (void)hipSetDevice(c->device);
   if (c->stream) (void)hipStreamSynchronize(c->stream);
+  c->copy.release();
   free_mesh_buffers(c);
   for (auto& e : c->pool) (void)hipEventDestroy(e);
   for (auto& e : c->net_ev)
@@ -1235,9 +1284,12 @@ int akx_field_upload(akx_ctx* c, int field, const void* host, size_t bytes) {
   if (field == AKX_DAMAGE) {
     if (!c->damage) return fail(c, AKX_ERR_STATE, "no damage material");
     if (bytes != size_t(c->E) * c->Q * 8) return fail(c, AKX_ERR_ARGUMENT, "damage: size mismatch");
-    std::vector<double> tmp(size_t(c->E) * c->Q);
-    to_internal_points(c, static_cast<const double*>(host), tmp.data(), 1);
-    HIP_TRY(c, hipMemcpy(c->damage, tmp.data(), bytes, hipMemcpyHostToDevice));
+    if (int rc = device_numbering(c)) return rc;
+    ScratchPool::Use use(c->scratch);
+    if (int rc = upload_numbered(c, c->E, c->Q, c->elem_inv_d, static_cast<const double*>(host),
+                                 c->damage))
+      return rc;
+    HIP_TRY(c, hipStreamSynchronize(c->stream));
     return AKX_OK;
   }
   double* p = nodal_ptr(c, field);
@@ -1246,12 +1298,13 @@ int akx_field_upload(akx_ctx* c, int field, const void* host, size_t bytes) {
   // the internal force is writable as the reference's getInternalForce() is:
   // Material::assembleInternalForces adds into it
   if (bytes != nd * 8) return fail(c, AKX_ERR_ARGUMENT, "size mismatch");
-  std::vector<double> tmp(nd);
-  to_internal_nodal(c, static_cast<const double*>(host), tmp.data());
-  HIP_TRY(c, hipMemcpyAsync(p, tmp.data(), bytes, hipMemcpyHostToDevice, c->stream));
+  if (int rc = device_numbering(c)) return rc;
+  const double* h = static_cast<const double*>(host);
+  ScratchPool::Use use(c->scratch);
+  if (int rc = upload_numbered(c, c->N, c->d, c->node_inv_d, h, p)) return rc;
   if (field == AKX_EXTERNAL_FORCE) {
     c->has_fext = false;
-    for (size_t k = 0; k < nd && !c->has_fext; ++k) c->has_fext = (tmp[k] != 0.);
+    for (size_t k = 0; k < nd && !c->has_fext; ++k) c->has_fext = (h[k] != 0.);
   }
   HIP_TRY(c, hipStreamSynchronize(c->stream));
   return AKX_OK;
@@ -1274,45 +1327,36 @@ int akx_field_download(akx_ctx* c, int field, void* host, size_t bytes) {
   }
   const size_t ne = field_elems(c, field);
   if (bytes != ne * 8) return fail(c, AKX_ERR_ARGUMENT, "size mismatch");
+  double* h = static_cast<double*>(host);
+  if (int rc = device_numbering(c)) return rc;
+  const uint32_t *ninv = c->node_inv_d, *einv = c->elem_inv_d;
+  ScratchPool::Use use(c->scratch);
   if (field == AKX_MASS) {
     if (!c->initialized) return fail(c, AKX_ERR_STATE, "akx_init has not been called");
-    std::vector<double> m(c->N);
-    HIP_TRY(c, hipMemcpyAsync(m.data(), c->mass, c->N * 8, hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(c, hipStreamSynchronize(c->stream));
-    double* h = static_cast<double*>(host);
-    for (int64_t k = 0; k < c->N; ++k)
-      for (int i = 0; i < c->d; ++i) h[size_t(c->node_perm[k]) * c->d + i] = m[k];
-    return AKX_OK;
+    return download_numbered(c, c->N, c->d, 1, ninv, c->mass, h);
   }
-  std::vector<double> tmp(ne);
   if (field == AKX_CURRENT_POSITION) {
     HIP_TRY(c, launch_add(c->stream, int64_t(nd), c->X, c->u, c->work));
-    HIP_TRY(c, hipMemcpyAsync(tmp.data(), c->work, bytes, hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(c, hipStreamSynchronize(c->stream));
-    to_caller_nodal(c, tmp.data(), static_cast<double*>(host));
-    return AKX_OK;
+    return download_numbered(c, c->N, c->d, c->d, ninv, c->work, h);
   }
   if (field == AKX_DAMAGE) {
     if (!c->damage) return fail(c, AKX_ERR_STATE, "no damage material");
-    HIP_TRY(c, hipMemcpyAsync(tmp.data(), c->damage, bytes, hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(c, hipStreamSynchronize(c->stream));
-    to_caller_points(c, tmp.data(), static_cast<double*>(host), 1);
-    return AKX_OK;
+    return download_numbered(c, c->E, c->Q, c->Q, einv, c->damage, h);
   }
   if (field == AKX_SHAPES_DERIVATIVES || field == AKX_JACOBIANS) {
     int rc = check_ready(c);
     if (rc) return rc;
+    std::vector<double> tmp(ne);
     const int comp = field == AKX_JACOBIANS ? 1 : c->d * c->n;
-    HIP_TRY(c, hipMemcpyAsync(tmp.data(), field == AKX_JACOBIANS ? c->J64 : c->B64, bytes,
-                              hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(c, hipStreamSynchronize(c->stream));
+    HIP_TRY(c, c->copy.to_host(c->device, c->stream, tmp.data(),
+                               field == AKX_JACOBIANS ? c->J64 : c->B64, bytes));
     std::vector<double> pts(ne);
     const int64_t E = c->E;
     for (int64_t e = 0; e < E; ++e)
       for (int q = 0; q < c->Q; ++q)
         for (int k = 0; k < comp; ++k)
           pts[(size_t(e) * c->Q + q) * comp + k] = tmp[(size_t(q) * comp + k) * E + e];
-    to_caller_points(c, pts.data(), static_cast<double*>(host), comp);
+    to_caller_points(c, pts.data(), h, comp);
     return AKX_OK;
   }
   if (field == AKX_GRAD_U || field == AKX_STRESS) {
@@ -1326,18 +1370,12 @@ int akx_field_download(akx_ctx* c, int field, void* host, size_t bytes) {
       ElemArgs A = elem_args(c, g, AKX_FP64);
       HIP_TRY(c, launch_point_fields(c->et, g.kind, c->stream, A, c->gradu, c->stress));
     }
-    HIP_TRY(c, hipMemcpyAsync(tmp.data(), field == AKX_GRAD_U ? c->gradu : c->stress, bytes,
-                              hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(c, hipStreamSynchronize(c->stream));
-    to_caller_points(c, tmp.data(), static_cast<double*>(host), c->d * c->d);
-    return AKX_OK;
+    const int w = c->Q * c->d * c->d;
+    return download_numbered(c, c->E, w, w, einv, field == AKX_GRAD_U ? c->gradu : c->stress, h);
   }
   double* p = nodal_ptr(c, field);
   if (!p) return fail(c, AKX_ERR_ARGUMENT, "unknown field");
-  HIP_TRY(c, hipMemcpyAsync(tmp.data(), p, bytes, hipMemcpyDeviceToHost, c->stream));
-  HIP_TRY(c, hipStreamSynchronize(c->stream));
-  to_caller_nodal(c, tmp.data(), static_cast<double*>(host));
-  return AKX_OK;
+  return download_numbered(c, c->N, c->d, c->d, ninv, p, h);
 }
 
 int akx_host_alloc(size_t bytes, void** ptr) {
@@ -1358,17 +1396,7 @@ int akx_field_download_async(akx_ctx* c, int field, void* host, size_t bytes, ui
   if (!c->initialized) return fail(c, AKX_ERR_STATE, "akx_init has not been called");
   if (!host) return fail(c, AKX_ERR_ARGUMENT, "null host pointer");
   (void)hipSetDevice(c->device);
-  // caller -> internal numbering on the device, built on first use
-  if (c->reorder && !c->node_inv_d) {
-    HIP_TRY(c, dalloc(&c->node_inv_d, c->node_inv.size()));
-    HIP_TRY(c, hipMemcpy(c->node_inv_d, c->node_inv.data(), c->node_inv.size() * 4,
-                         hipMemcpyHostToDevice));
-    if (!c->elem_inv.empty()) {
-      HIP_TRY(c, dalloc(&c->elem_inv_d, c->elem_inv.size()));
-      HIP_TRY(c, hipMemcpy(c->elem_inv_d, c->elem_inv.data(), c->elem_inv.size() * 4,
-                           hipMemcpyHostToDevice));
-    }
-  }
+  if (int rc = device_numbering(c)) return rc;
   const uint32_t* ninv = c->reorder ? c->node_inv_d : nullptr;
   const uint32_t* einv = c->reorder ? c->elem_inv_d : nullptr;
   const int d = c->d;
@@ -1739,8 +1767,7 @@ int akx_stable_time_step(akx_ctx* c, double* dt) {
   (void)hipSetDevice(c->device);
   HIP_TRY(c, launch_stable_dt(c->et, c->stream, c->E, c->X, c->u, c->conn_soa, c->elem_mat_d,
                               c->mats_d, c->partial, c->partial_blocks, c->scalar));
-  HIP_TRY(c, hipMemcpyAsync(dt, c->scalar, 8, hipMemcpyDeviceToHost, c->stream));
-  HIP_TRY(c, hipStreamSynchronize(c->stream));
+  HIP_TRY(c, c->copy.to_host(c->device, c->stream, dt, c->scalar, 8));
   return AKX_OK;
 }
 
@@ -1755,8 +1782,7 @@ int akx_energy(akx_ctx* c, int kind, double* value) {
                              c->mats_d, c->damage, nullptr, 0, c->partial, c->partial_blocks,
                              c->scalar));
     double r = 0;
-    HIP_TRY(c, hipMemcpyAsync(&r, c->scalar, 8, hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(c, hipStreamSynchronize(c->stream));
+    HIP_TRY(c, c->copy.to_host(c->device, c->stream, &r, c->scalar, 8));
     *value = kind == AKX_ENERGY_KINETIC ? r * .5 : r * c->dt;
     return AKX_OK;
   }
@@ -1768,8 +1794,7 @@ int akx_energy(akx_ctx* c, int kind, double* value) {
                              c->elem_mat_d, c->mats_d, c->damage, g.filter, g.count, c->partial,
                              c->partial_blocks, c->scalar + 1));
     double r = 0;
-    HIP_TRY(c, hipMemcpyAsync(&r, c->scalar + 1, 8, hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(c, hipStreamSynchronize(c->stream));
+    HIP_TRY(c, c->copy.to_host(c->device, c->stream, &r, c->scalar + 1, 8));
     total += r;
   }
   *value = total;
@@ -1924,7 +1949,7 @@ int akx_surrogate_gradients(akx_ctx* c, int64_t n, const float* x, const float* 
     return fail(c, AKX_ERR_ARGUMENT, "batch must be a positive multiple of 256");
   (void)hipSetDevice(c->device);
   double l = 0;
-  HIP_TRY(c, c->sur.gradients(c->stream, n, x, t, grad, &l));
+  HIP_TRY(c, c->sur.gradients(c->stream, c->device, c->copy, n, x, t, grad, &l));
   if (loss) *loss = l;
   return AKX_OK;
 }
@@ -1932,7 +1957,7 @@ int akx_surrogate_gradients(akx_ctx* c, int64_t n, const float* x, const float* 
 int akx_surrogate_infer(akx_ctx* c, int64_t n, const float* x, float* y) {
   if (!c || (n > 0 && (!x || !y)) || n < 0) return AKX_ERR_ARGUMENT;
   (void)hipSetDevice(c->device);
-  HIP_TRY(c, c->sur.infer(c->stream, n, x, y));
+  HIP_TRY(c, c->sur.infer(c->stream, c->device, c->copy, n, x, y));
   return AKX_OK;
 }
 
@@ -2113,35 +2138,40 @@ int akx_set_launch(akx_ctx* c, int element_block, int node_block, int xcd_remap,
 /* ======================================================================== */
 namespace {
 
-// A device buffer released at the end of an operator call (the calls
-// synchronise before they return).
+// A device buffer of an operator call, from the context's scratch (the calls
+// synchronise before they return and hold a ScratchPool::Use meanwhile).
 struct TempBuf {
   void* p = nullptr;
-  ~TempBuf() {
-    if (p) (void)hipFree(p);
-  }
   template <typename T>
   T* get() { return static_cast<T*>(p); }
 };
 
-hipError_t temp_alloc(TempBuf& b, size_t bytes) {
-  return hipMalloc(&b.p, std::max<size_t>(bytes, 8));
+hipError_t temp_alloc(akx_ctx* c, TempBuf& b, size_t bytes) {
+  return c->scratch.take(std::max<size_t>(bytes, 8), &b.p);
 }
 
 // The caller's element list (nullptr: every element, caller order) as
-// internal ids on the device; returns the row count through *count.
-int fe_element_list(akx_ctx* c, const uint32_t* ids, int64_t nb, TempBuf& dev, int64_t* count) {
+// internal ids on the device (nullptr: 0 .. count - 1); returns the row count
+// through *count.
+int fe_element_list(akx_ctx* c, const uint32_t* ids, int64_t nb, const uint32_t** dev,
+                    int64_t* count) {
   if (ids && nb < 0) return fail(c, AKX_ERR_ARGUMENT, "negative element count");
-  const int64_t cnt = ids ? nb : c->E;
-  std::vector<uint32_t> internal(size_t(std::max<int64_t>(cnt, 0)));
-  for (int64_t t = 0; t < cnt; ++t) {
-    const uint32_t e = ids ? ids[t] : uint32_t(t);
-    if (int64_t(e) >= c->E) return fail(c, AKX_ERR_ARGUMENT, "element id out of range");
-    internal[size_t(t)] = c->elem_inv[e];
+  if (!ids) {
+    if (int rc = device_numbering(c)) return rc;
+    *dev = c->elem_inv_d;
+    *count = c->E;
+    return AKX_OK;
   }
-  HIP_TRY(c, temp_alloc(dev, internal.size() * 4));
-  HIP_TRY(c, hipMemcpy(dev.p, internal.data(), internal.size() * 4, hipMemcpyHostToDevice));
-  *count = cnt;
+  std::vector<uint32_t> internal(static_cast<size_t>(nb));
+  for (int64_t t = 0; t < nb; ++t) {
+    if (int64_t(ids[t]) >= c->E) return fail(c, AKX_ERR_ARGUMENT, "element id out of range");
+    internal[size_t(t)] = c->elem_inv[ids[t]];
+  }
+  TempBuf b;
+  HIP_TRY(c, temp_alloc(c, b, internal.size() * 4));
+  HIP_TRY(c, c->copy.to_device(c->device, c->stream, b.p, internal.data(), internal.size() * 4));
+  *dev = b.get<uint32_t>();
+  *count = nb;
   return AKX_OK;
 }
 
@@ -2163,24 +2193,19 @@ FeArgs fe_args(akx_ctx* c, const uint32_t* filt, int64_t count, int nb) {
 
 // A nodal caller array (N, nb) in the internal node numbering, on the device.
 int upload_nodal(akx_ctx* c, const double* host, int nb, TempBuf& dev) {
-  const size_t N = size_t(c->N);
-  std::vector<double> h(N * nb);
-  for (size_t k = 0; k < N; ++k)
-    for (int i = 0; i < nb; ++i) h[k * nb + i] = host[size_t(c->node_perm[k]) * nb + i];
-  HIP_TRY(c, temp_alloc(dev, h.size() * 8));
-  HIP_TRY(c, hipMemcpy(dev.p, h.data(), h.size() * 8, hipMemcpyHostToDevice));
-  return AKX_OK;
+  if (int rc = device_numbering(c)) return rc;
+  HIP_TRY(c, temp_alloc(c, dev, size_t(c->N) * nb * 8));
+  return upload_numbered(c, c->N, nb, c->node_inv_d, host, dev.get<double>());
 }
 
 int upload_rows(akx_ctx* c, const double* host, size_t n, TempBuf& dev) {
-  HIP_TRY(c, temp_alloc(dev, n * 8));
-  if (n) HIP_TRY(c, hipMemcpy(dev.p, host, n * 8, hipMemcpyHostToDevice));
+  HIP_TRY(c, temp_alloc(c, dev, n * 8));
+  HIP_TRY(c, c->copy.to_device(c->device, c->stream, dev.p, host, n * 8));
   return AKX_OK;
 }
 
 int download_rows(akx_ctx* c, const TempBuf& dev, size_t n, double* host) {
-  HIP_TRY(c, hipStreamSynchronize(c->stream));
-  if (n) HIP_TRY(c, hipMemcpy(host, dev.p, n * 8, hipMemcpyDeviceToHost));
+  HIP_TRY(c, c->copy.to_host(c->device, c->stream, host, dev.p, n * 8));
   return AKX_OK;
 }
 
@@ -2191,14 +2216,16 @@ int fe_op(akx_ctx* c, int op, const double* in, int nb, bool nodal_in, size_t in
   if (rc) return rc;
   if (!in || !out) return fail(c, AKX_ERR_ARGUMENT, "null array");
   (void)hipSetDevice(c->device);
-  TempBuf filt, din, dout;
+  ScratchPool::Use use(c->scratch);
+  const uint32_t* filt = nullptr;
+  TempBuf din, dout;
   int64_t cnt = 0;
-  if ((rc = fe_element_list(c, ids, nb_ids, filt, &cnt))) return rc;
+  if ((rc = fe_element_list(c, ids, nb_ids, &filt, &cnt))) return rc;
   if (nodal_in) rc = upload_nodal(c, in, nb, din);
   else rc = upload_rows(c, in, size_t(cnt) * in_per_elem, din);
   if (rc) return rc;
-  HIP_TRY(c, temp_alloc(dout, size_t(cnt) * out_per_elem * 8));
-  FeArgs A = fe_args(c, filt.get<uint32_t>(), cnt, nb);
+  HIP_TRY(c, temp_alloc(c, dout, size_t(cnt) * out_per_elem * 8));
+  FeArgs A = fe_args(c, filt, cnt, nb);
   A.in = din.get<double>();
   A.out = dout.get<double>();
   HIP_TRY(c, launch_fe(op, c->et, c->stream, A));
@@ -2223,13 +2250,14 @@ std::vector<uint32_t> material_filter(const akx_ctx* c, int mat) {
   return ids;
 }
 
-int material_setup(akx_ctx* c, int mat, TempBuf& filt, int64_t* cnt, MatArgs* M) {
+int material_setup(akx_ctx* c, int mat, const uint32_t** filt, int64_t* cnt, MatArgs* M) {
   int rc = check_ready(c);
   if (rc) return rc;
   if (mat < 0 || mat >= int(c->mats.size())) return fail(c, AKX_ERR_ARGUMENT, "no such material");
   (void)hipSetDevice(c->device);
   const std::vector<uint32_t> ids = material_filter(c, mat);
-  if ((rc = fe_element_list(c, ids.data(), int64_t(ids.size()), filt, cnt))) return rc;
+  if ((rc = fe_element_list(c, ids.data(), int64_t(ids.size()), filt, cnt)))
+    return rc;
   const size_t ne = size_t(c->E) * c->Q * c->d * c->d;
   if (!c->gradu) {
     HIP_TRY(c, dalloc(&c->gradu, ne));
@@ -2305,26 +2333,28 @@ int akx_fe_integrate_scalar(akx_ctx* c, const double* f, const uint32_t* element
   if (rc) return rc;
   if (!f || !value) return fail(c, AKX_ERR_ARGUMENT, "null array");
   (void)hipSetDevice(c->device);
-  TempBuf filt, din, per, tmp, sort, res;
+  ScratchPool::Use use(c->scratch);
+  const uint32_t* filt = nullptr;
+  TempBuf din, per, tmp, sort, res;
   int64_t cnt = 0;
-  if ((rc = fe_element_list(c, elements, nb_elements, filt, &cnt))) return rc;
+  if ((rc = fe_element_list(c, elements, nb_elements, &filt, &cnt))) return rc;
   if (cnt == 0) {
     *value = 0.;
     return AKX_OK;
   }
   if (cnt >= int64_t(1) << 31) return fail(c, AKX_ERR_ARGUMENT, "too many elements");
   if ((rc = upload_rows(c, f, size_t(cnt) * c->Q, din))) return rc;
-  HIP_TRY(c, temp_alloc(per, size_t(cnt) * 8));
-  HIP_TRY(c, temp_alloc(tmp, size_t(cnt) * 8));
-  HIP_TRY(c, temp_alloc(res, 8));
-  FeArgs A = fe_args(c, filt.get<uint32_t>(), cnt, 1);
+  HIP_TRY(c, temp_alloc(c, per, size_t(cnt) * 8));
+  HIP_TRY(c, temp_alloc(c, tmp, size_t(cnt) * 8));
+  HIP_TRY(c, temp_alloc(c, res, 8));
+  FeArgs A = fe_args(c, filt, cnt, 1);
   A.in = din.get<double>();
   A.out = per.get<double>();
   HIP_TRY(c, launch_fe(FE_INTEGRATE, c->et, c->stream, A));
   size_t sort_bytes = 0;
   HIP_TRY(c, launch_reduce_sorted(c->stream, cnt, per.get<double>(), tmp.get<double>(),
                                   res.get<double>(), nullptr, &sort_bytes));
-  HIP_TRY(c, temp_alloc(sort, sort_bytes));
+  HIP_TRY(c, temp_alloc(c, sort, sort_bytes));
   HIP_TRY(c, launch_reduce_sorted(c->stream, cnt, per.get<double>(), tmp.get<double>(),
                                   res.get<double>(), sort.p, &sort_bytes));
   return download_rows(c, res, 1, value);
@@ -2339,26 +2369,20 @@ int akx_fe_assemble_field_lumped(akx_ctx* c, const double* field, int nb_dof, do
   const int64_t E = c->E, N = c->N;
   const int Q = c->Q, n = c->n;
   // the field in internal element order, the lumped vector in internal node order
-  std::vector<double> fi(size_t(E) * Q * nb_dof);
-  for (int64_t e = 0; e < E; ++e)
-    std::memcpy(&fi[size_t(e) * Q * nb_dof], field + size_t(c->elem_perm[e]) * Q * nb_dof,
-                sizeof(double) * Q * nb_dof);
+  if ((rc = device_numbering(c))) return rc;
+  ScratchPool::Use use(c->scratch);
   TempBuf din, integ, dl;
-  if ((rc = upload_rows(c, fi.data(), fi.size(), din))) return rc;
+  HIP_TRY(c, temp_alloc(c, din, size_t(E) * Q * nb_dof * 8));
+  if ((rc = upload_numbered(c, E, Q * nb_dof, c->elem_inv_d, field, din.get<double>()))) return rc;
   if ((rc = upload_nodal(c, lumped, nb_dof, dl))) return rc;
-  HIP_TRY(c, temp_alloc(integ, size_t(E) * n * nb_dof * 8));
+  HIP_TRY(c, temp_alloc(c, integ, size_t(E) * n * nb_dof * 8));
   FeArgs A = fe_args(c, nullptr, E, nb_dof);
   A.in = din.get<double>();
   A.out = integ.get<double>();
   HIP_TRY(c, launch_fe(FE_LUMPED_ELEMENTS, c->et, c->stream, A));
   HIP_TRY(c, launch_fe_lumped_nodes(c->stream, N, nb_dof, n, c->mass_off, c->mass_slot,
                                     integ.get<double>(), dl.get<double>()));
-  std::vector<double> h(size_t(N) * nb_dof);
-  if ((rc = download_rows(c, dl, h.size(), h.data()))) return rc;
-  for (int64_t k = 0; k < N; ++k)
-    for (int i = 0; i < nb_dof; ++i)
-      lumped[size_t(c->node_perm[k]) * nb_dof + i] = h[size_t(k) * nb_dof + i];
-  return AKX_OK;
+  return download_numbered(c, N, nb_dof, nb_dof, c->node_inv_d, dl.get<double>(), lumped);
 }
 
 int akx_material_elements(akx_ctx* c, int mat, int64_t* count, uint32_t* ids) {
@@ -2373,15 +2397,17 @@ int akx_material_elements(akx_ctx* c, int mat, int64_t* count, uint32_t* ids) {
 int akx_material_compute_stress(akx_ctx* c, int mat, const double* grad_u, double* stress) {
   if (!c) return AKX_ERR_ARGUMENT;
   if (!grad_u) return fail(c, AKX_ERR_ARGUMENT, "null gradient");
-  TempBuf filt, din, dout;
+  ScratchPool::Use use(c->scratch);
+  const uint32_t* filt = nullptr;
+  TempBuf din, dout;
   int64_t cnt = 0;
   MatArgs M;
-  int rc = material_setup(c, mat, filt, &cnt, &M);
+  int rc = material_setup(c, mat, &filt, &cnt, &M);
   if (rc) return rc;
   const size_t rows = size_t(cnt) * c->Q * c->d * c->d;
   if ((rc = upload_rows(c, grad_u, rows, din))) return rc;
-  if (stress) HIP_TRY(c, temp_alloc(dout, rows * 8));
-  FeArgs A = fe_args(c, filt.get<uint32_t>(), cnt, c->d * c->d);
+  if (stress) HIP_TRY(c, temp_alloc(c, dout, rows * 8));
+  FeArgs A = fe_args(c, filt, cnt, c->d * c->d);
   A.in = din.get<double>();
   A.out = stress ? dout.get<double>() : nullptr;
   HIP_TRY(c, launch_material(MAT_STRESS, c->et, c->mats[mat].kind, c->stream, A, M));
@@ -2392,12 +2418,13 @@ int akx_material_compute_stress(akx_ctx* c, int mat, const double* grad_u, doubl
 
 int akx_material_compute_all_stresses(akx_ctx* c, int mat, double* grad_u, double* stress) {
   if (!c) return AKX_ERR_ARGUMENT;
-  TempBuf filt;
+  ScratchPool::Use use(c->scratch);
+  const uint32_t* filt = nullptr;
   int64_t cnt = 0;
   MatArgs M;
-  int rc = material_setup(c, mat, filt, &cnt, &M);
+  int rc = material_setup(c, mat, &filt, &cnt, &M);
   if (rc) return rc;
-  FeArgs A = fe_args(c, filt.get<uint32_t>(), cnt, c->d);
+  FeArgs A = fe_args(c, filt, cnt, c->d);
   A.in = c->u;
   HIP_TRY(c, launch_material(MAT_ALL_STRESSES, c->et, c->mats[mat].kind, c->stream, A, M));
   HIP_TRY(c, hipStreamSynchronize(c->stream));
@@ -2420,12 +2447,13 @@ int akx_material_compute_all_stresses(akx_ctx* c, int mat, double* grad_u, doubl
 
 int akx_material_assemble_internal_forces(akx_ctx* c, int mat) {
   if (!c) return AKX_ERR_ARGUMENT;
-  TempBuf filt;
+  ScratchPool::Use use(c->scratch);
+  const uint32_t* filt = nullptr;
   int64_t cnt = 0;
   MatArgs M;
-  int rc = material_setup(c, mat, filt, &cnt, &M);
+  int rc = material_setup(c, mat, &filt, &cnt, &M);
   if (rc) return rc;
-  FeArgs A = fe_args(c, filt.get<uint32_t>(), cnt, c->d);
+  FeArgs A = fe_args(c, filt, cnt, c->d);
   A.out = static_cast<double*>(c->slots);
   HIP_TRY(c, launch_material(MAT_FORCES, c->et, c->mats[mat].kind, c->stream, A, M));
   HIP_TRY(c, launch_material_gather(c->stream, c->N, c->d, c->n, mat, c->csr_off, c->csr_slot,
@@ -2437,10 +2465,11 @@ int akx_material_assemble_internal_forces(akx_ctx* c, int mat) {
 
 int akx_material_potential_energy(akx_ctx* c, int mat, double* value) {
   if (!c || !value) return AKX_ERR_ARGUMENT;
-  TempBuf filt;
+  ScratchPool::Use use(c->scratch);
+  const uint32_t* filt = nullptr;
   int64_t cnt = 0;
   MatArgs M;
-  int rc = material_setup(c, mat, filt, &cnt, &M);
+  int rc = material_setup(c, mat, &filt, &cnt, &M);
   if (rc) return rc;
   if (cnt == 0) {
     *value = 0.;
@@ -2448,7 +2477,7 @@ int akx_material_potential_energy(akx_ctx* c, int mat, double* value) {
   }
   HIP_TRY(c, launch_energy(AKX_ENERGY_POTENTIAL, c->et, c->mats[mat].kind, c->stream, c->N, c->E,
                            c->u, c->v, c->mass, c->fext, c->fint, c->blocked, c->conn_soa, c->B64,
-                           c->J64, c->elem_mat_d, c->mats_d, c->damage, filt.get<uint32_t>(), cnt,
+                           c->J64, c->elem_mat_d, c->mats_d, c->damage, filt, cnt,
                            c->partial, c->partial_blocks, c->scalar + 1));
   double r = 0;
   HIP_TRY(c, hipMemcpyAsync(&r, c->scalar + 1, 8, hipMemcpyDeviceToHost, c->stream));

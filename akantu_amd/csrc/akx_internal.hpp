@@ -8,6 +8,7 @@
 #include <mutex>
 #include <vector>
 
+#include "akx_copy.hpp"
 #include "akx_device.hpp"
 #include "akx_mlp.hpp"
 
@@ -229,6 +230,8 @@ hipError_t launch_energy(int kind_energy, int et, int mat_kind_uniform, hipStrea
 hipError_t launch_point_fields(int et, int kind, hipStream_t s, const ElemArgs& A, double* gradu,
                                double* stress);
 hipError_t launch_add(hipStream_t s, int64_t n, const double* x, const double* y, double* out);
+hipError_t launch_scatter_rows(hipStream_t s, int64_t rows, int width, const uint32_t* inv,
+                               const double* src, double* dst);
 hipError_t launch_snapshot(hipStream_t s, int64_t rows, int dw, int sw, const uint32_t* inv,
                            const void* src, void* dst, int elem_bytes);
 
@@ -320,9 +323,10 @@ struct Surrogate {
                       double yd_shape, uint64_t seed);
   hipError_t train(hipStream_t s, int iterations, int B, double lr, uint64_t seed,
                    double* final_loss);
-  hipError_t gradients(hipStream_t s, int64_t n, const float* x, const float* t, float* grad,
-                       double* loss);
-  hipError_t infer(hipStream_t s, int64_t n, const float* x, float* y);
+  hipError_t gradients(hipStream_t s, int device, HostCopier& copy, int64_t n, const float* x,
+                       const float* t, float* grad, double* loss);
+  hipError_t infer(hipStream_t s, int device, HostCopier& copy, int64_t n, const float* x,
+                   float* y);
   hipError_t set_params(hipStream_t s, const float* host);
   hipError_t get_params(hipStream_t s, float* host);
 };
@@ -443,6 +447,10 @@ struct akx_ctx {
   hipGraphExec_t graph_exec = nullptr;
 
   akx::Surrogate sur;
+
+  // host copies and device scratch of the calls on caller arrays
+  akx::HostCopier copy;
+  akx::ScratchPool scratch;
 
   // asynchronous downloads: a device snapshot taken on `stream`, copied to
   // page-locked host memory on `copy_stream`; slots are recycled once their

@@ -2775,6 +2775,26 @@ __global__ void __launch_bounds__(256) k_snapshot(int64_t rows, int dw, int sw,
   dst[k] = v;
 }
 
+// The other way: rows of `width` doubles in the caller's numbering to the
+// internal one, dst[inv[r]] = src[r].
+__global__ void __launch_bounds__(256) k_scatter_rows(int64_t rows, int width,
+                                                      const uint32_t* __restrict__ inv,
+                                                      const double* __restrict__ src,
+                                                      double* __restrict__ dst) {
+  const int64_t k = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (k >= rows * width) return;
+  const int64_t r = k / width;
+  dst[int64_t(inv[r]) * width + (k - r * width)] = src[k];
+}
+
+hipError_t launch_scatter_rows(hipStream_t s, int64_t rows, int width, const uint32_t* inv,
+                               const double* src, double* dst) {
+  clear_error();
+  if (rows * width == 0) return hipSuccess;
+  k_scatter_rows<<<grid_for(rows * width, 256), 256, 0, s>>>(rows, width, inv, src, dst);
+  return hipGetLastError();
+}
+
 hipError_t launch_snapshot(hipStream_t s, int64_t rows, int dw, int sw, const uint32_t* inv,
                            const void* src, void* dst, int elem_bytes) {
   clear_error();

@@ -838,19 +838,20 @@ hipError_t Surrogate::batch_loss(hipStream_t s, int B, double* loss) {
   return hipSuccess;
 }
 
-hipError_t Surrogate::gradients(hipStream_t s, int64_t n, const float* x_host, const float* t_host,
-                                float* grad_host, double* loss) {
+hipError_t Surrogate::gradients(hipStream_t s, int device, HostCopier& copy, int64_t n,
+                                const float* x_host, const float* t_host, float* grad_host,
+                                double* loss) {
   hipError_t e;
   const int B = int(n);
   if ((e = ensure_params()) || (e = ensure_batch(B)) || (e = ensure_io(n))) return e;
   if ((e = refresh(s))) return e;
   float* tdev = io_y;
-  if ((e = hipMemcpyAsync(io_x, x_host, size_t(n) * 7 * 4, hipMemcpyHostToDevice, s)) ||
-      (e = hipMemcpyAsync(tdev, t_host, size_t(n) * 7 * 4, hipMemcpyHostToDevice, s)))
+  if ((e = copy.to_device(device, s, io_x, x_host, size_t(n) * 7 * 4)) ||
+      (e = copy.to_device(device, s, tdev, t_host, size_t(n) * 7 * 4)))
     return e;
   if ((e = run_pass(s, io_x, tdev, n, B, 0, -1, true, true)) || (e = apply(s, B, true, 0.f)))
     return e;
-  if ((e = hipMemcpyAsync(grad_host, grad, NPARAM * 4, hipMemcpyDeviceToHost, s))) return e;
+  if ((e = copy.to_host(device, s, grad_host, grad, NPARAM * 4))) return e;
   return batch_loss(s, B, loss);
 }
 
@@ -864,13 +865,13 @@ hipError_t Surrogate::ensure_io(int64_t n) {
   return hipSuccess;
 }
 
-hipError_t Surrogate::infer(hipStream_t s, int64_t n, const float* x_host, float* y_host) {
+hipError_t Surrogate::infer(hipStream_t s, int device, HostCopier& copy, int64_t n,
+                            const float* x_host, float* y_host) {
   hipError_t e;
   if ((e = ensure_params()) || (e = ensure_io(n))) return e;
-  if ((e = hipMemcpyAsync(io_x, x_host, size_t(n) * 7 * 4, hipMemcpyHostToDevice, s))) return e;
+  if ((e = copy.to_device(device, s, io_x, x_host, size_t(n) * 7 * 4))) return e;
   if ((e = launch_sur_mlp(s, img, imgb, infer_bf16, n, io_x, 7, io_y, 7))) return e;
-  if ((e = hipMemcpyAsync(y_host, io_y, size_t(n) * 7 * 4, hipMemcpyDeviceToHost, s))) return e;
-  return hipStreamSynchronize(s);
+  return copy.to_host(device, s, y_host, io_y, size_t(n) * 7 * 4);
 }
 
 hipError_t launch_sur_mlp(hipStream_t s, const void* img, const float* imgb, bool bf16,

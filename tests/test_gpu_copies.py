@@ -1,0 +1,47 @@
+"""Copies between a caller's arrays and the device through the page-locked
+slots: sizes at the edges of a slot and of two (1, 2 MB) and of the one- and
+four-thread copies (8 MB), renumbered and not."""
+import numpy as np
+import pytest
+
+from akantu_amd import akx
+from akantu_amd import mesh as akm
+
+pytestmark = pytest.mark.gpu
+
+
+# nodes of 16 bytes each: 1 MB, a little more, 2 MB, more, 8 MB, more
+@pytest.mark.parametrize("grid", [(2, 2), (256, 256), (257, 256), (512, 256), (513, 257),
+                                  (1024, 512), (1025, 513)])
+@pytest.mark.parametrize("keep", [False, True])
+def test_nodal_fields_round_trip(grid, keep):
+    m = akm.rectangle_quad4(grid[0] - 1, grid[1] - 1, 1.0, 1.0)
+    model = akx.SolidMechanicsModel(m, keep_numbering=keep)
+    model.add_material(E=210e9, nu=0.3, rho=7800.0)
+    model.init_full()
+    rng = np.random.default_rng(grid[0])
+    u, v = rng.normal(size=(2, m.nb_nodes, 2))
+    model.set("displacement", u)
+    model.set("velocity", v)
+    assert np.array_equal(model.get("displacement"), u)
+    assert np.array_equal(model.get("velocity"), v)
+    assert np.array_equal(model.get("current_position"), m.nodes + u)
+    # the mass of a regular grid: one value per node, reported per component
+    mass = model.get("mass")
+    assert np.array_equal(mass[:, 0], mass[:, 1])
+    assert mass[:, 0].sum() == pytest.approx(7800.0, rel=1e-12)
+
+
+@pytest.mark.parametrize("n", [1, 37449, 37450, 74899, 299594, 299595])
+def test_network_outputs_do_not_depend_on_the_copy(n):
+    """28 bytes per point: 37,449.1 points per MB."""
+    m = akm.box_tet4(1, 1, 1)
+    model = akx.SolidMechanicsModel(m)
+    model.add_material(kind=akx.NEOHOOKEAN_DAMAGE, E=1e9, nu=0.3, rho=1200.0, Sd=5e6,
+                       Yd=np.full(m.nb_elements, 1e6))
+    model.init_full()
+    model.surrogate_setup(0, 0.05)
+    x = np.random.default_rng(4).uniform(-1, 1, size=(n, 7)).astype(np.float32)
+    y = model.surrogate_infer(x)
+    parts = [model.surrogate_infer(x[k:k + 30000]) for k in range(0, n, 30000)]
+    assert np.array_equal(y, np.concatenate(parts))
