@@ -339,6 +339,7 @@ ElemArgs elem_args(akx_ctx* c, const KindGroup& g, int precision) {
   A.slots = c->slots;
   A.elem_mat = c->elem_mat_d;
   A.mats = c->mats_d;
+  A.mat0 = c->mat0;
   A.damage = c->damage;
   A.Yd = c->Yd;
   A.xcd_remap = c->xcd_remap;
@@ -351,6 +352,7 @@ ElemArgs elem_args(akx_ctx* c, const KindGroup& g, int precision) {
   A.partials = (A.patch && uses_partials(c, precision)) ? (lay == 3 ? 1 : 2) : 0;
   A.part_pos = (A.partials && lay >= 5) ? c->ppos : nullptr;
   A.patch_max_nodes = c->patch_max_nodes;
+  A.nodal_bytes = c->N * c->d * 8;
   A.patch_lds = c->patch_lds;
   A.patch_blocks = c->patch_blocks;
   A.pnode_cnt = c->pnode_cnt;
@@ -360,6 +362,7 @@ ElemArgs elem_args(akx_ctx* c, const KindGroup& g, int precision) {
   A.lconn = c->lconn;
   A.lrank = c->lrank;
   A.lcr = c->lcr;
+  A.lcr_shift = c->lcr_shift;
   A.tabf = c->tabf;
   A.tab64 = c->tab64_d;
   A.sur_img = nullptr;
@@ -544,15 +547,20 @@ int build_patches(akx_ctx* c, const std::vector<uint32_t>& slot2) {
   HIP_TRY(c, dalloc(&c->pnode_ids, pids_p.size()));
   HIP_TRY(c, dalloc(&c->run_start, rstart_p.size()));
   HIP_TRY(c, dalloc(&c->run_base, rbase_p.size()));
-  // patch-local node and rank packed in 16 bits per (e, a) when every patch
-  // has at most 256 nodes: one vector load per element
-  if (maxm <= 256) {
+  // patch-local node and rank packed in 16 bits per (e, a) when they fit: one
+  // vector load per element.  At least 8 bits for the node, so that meshes of
+  // tetrahedra and triangles share one shift.
+  int shift = 8, rank_max = 0;
+  while ((1 << shift) < maxm) ++shift;
+  for (uint8_t r : lrank) rank_max = std::max(rank_max, int(r));
+  c->lcr_shift = shift;
+  if (shift < 16 && rank_max < (1 << (16 - shift))) {
     const int np = n == 3 ? 4 : n;
     std::vector<uint16_t> lcr(size_t(E) * np, 0);
     for (int64_t e = 0; e < E; ++e)
       for (int a = 0; a < n; ++a)
-        lcr[size_t(e) * np + a] =
-            uint16_t(lconn[size_t(a) * E + e] | (uint16_t(lrank[size_t(a) * E + e]) << 8));
+        lcr[size_t(e) * np + a] = uint16_t(lconn[size_t(a) * E + e] |
+                                           (uint32_t(lrank[size_t(a) * E + e]) << shift));
     HIP_TRY(c, dalloc(&c->lcr, lcr.size()));
     HIP_TRY(c, hipMemcpy(c->lcr, lcr.data(), lcr.size() * 2, hipMemcpyHostToDevice));
   } else {
@@ -1186,6 +1194,7 @@ int akx_init(akx_ctx* c) {
         return fail(c, AKX_ERR_STATE, "damage material without thresholds (akx_material_damage)");
     }
   }
+  c->mat0 = mp[0];
   HIP_TRY(c, dalloc(&c->mats_d, nm));
   HIP_TRY(c, hipMemcpy(c->mats_d, mp.data(), nm * sizeof(MatParams), hipMemcpyHostToDevice));
   if (nm > 1) {

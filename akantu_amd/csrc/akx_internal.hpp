@@ -41,6 +41,7 @@ struct ElemArgs {
   void* slots;               // [e][dn], double or float
   const uint16_t* elem_mat;  // nullptr = material 0
   const MatParams* mats;
+  MatParams mat0;            // mats[0]: what every element has without elem_mat
   double* damage;            // [e*Q + q]
   const double* Yd;          // [e*Q + q]
   int xcd_remap;
@@ -52,6 +53,7 @@ struct ElemArgs {
   int patch;                 // 1: use it
   int partials;              // write one sum per (patch, node) instead of the runs: 1 FP64, 2 FP32
   const uint32_t* part_pos;  // [b * S + k] node-major position of the partial, nullptr = b * S + k
+  int64_t nodal_bytes;       // size of u and X
   int patch_max_nodes;       // most distinct nodes of one patch = stride S of the lists
   int patch_lds;             // dynamic LDS bytes per block
   int64_t patch_blocks;      // number of patches
@@ -59,9 +61,10 @@ struct ElemArgs {
   const uint32_t* pnode_ids; // [b * S + k] patch nodes (internal ids, ascending; padded)
   const uint32_t* run_start; // [b * S + k] first mixed-CSR position of the node's run
   const uint16_t* run_base;  // [b * (S + 1) + k] prefix of run lengths (padded)
-  // patch-local node | rank << 8 per (e, a), element-major with stride
-  // lcr_stride (n, 4 for 3-node elements); nullptr: lconn / lrank instead
+  // patch-local node | rank << lcr_shift per (e, a), element-major with stride
+  // n (4 for 3-node elements); nullptr: lconn / lrank instead
   const uint16_t* lcr;
+  int lcr_shift;
   const uint16_t* lconn;     // [a][E] patch-local node index
   const uint8_t* lrank;      // [a][E] rank of (e, a) inside the node's run
   ElemTablesF tabf;
@@ -366,6 +369,7 @@ struct akx_ctx {
   uint32_t *mass_off = nullptr, *mass_slot = nullptr;  // element-ascending order
   void* slots = nullptr;
   uint16_t* elem_mat_d = nullptr;
+  akx::MatParams mat0{};               // the first material
   akx::MatParams* mats_d = nullptr;
   double* damage = nullptr;
   double* Yd = nullptr;
@@ -401,6 +405,7 @@ struct akx_ctx {
   uint32_t *pnode_cnt = nullptr, *pnode_ids = nullptr, *run_start = nullptr;
   uint16_t *run_base = nullptr, *lconn = nullptr, *lcr = nullptr;
   uint8_t* lrank = nullptr;
+  int lcr_shift = 8;
   // node -> entries of the per-patch partial sums (slot layout 3)
   uint32_t *pcsr_off = nullptr, *pentry = nullptr, *ppos = nullptr;
   // fused FP64 step (slot layout 6)

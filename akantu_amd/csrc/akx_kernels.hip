@@ -1212,16 +1212,30 @@ __device__ __forceinline__ bool sur_strain_from_differences(const ElemArgs& A, i
 // At least 4 waves per SIMD: the 8-point hexahedron with finite strain would
 // otherwise take 151 VGPRs (3 waves); capped at 128 it spills a few values and
 // runs 6 % faster.  The other instantiations are far below the cap.
-template <int ET, int KIND>
+// HALVES > 0: packed patch indices (one 16-bit word per element and node),
+// fewer than 256 HALVES nodes per patch, nodal arrays below 4 GB and FP32
+// partials at their node-major place (layout 5, what the mixed path runs).
+// Every load that does not depend on another is issued at once -- indices,
+// node ids, partials' places, runs' bases -- then the nodes' u and X: two round
+// trips before the block works.  Lanes past the patch's nodes repeat the last
+// one's loads instead of branching round them: a branch ends in a wait.  With
+// the forms chosen at run time (HALVES 0) the compiler waited for the indices
+// before it asked for the node ids, and for places and bases after u and X.
+// 6 million tetrahedra (elastic): 66.6 -> 57.8 us for the element kernel, 91.3
+// -> 83.7 us for the step; 2.1 million hexahedra (neo-Hookean, 405 nodes per
+// patch, now packed) 146 -> 137 us; 1.6 million triangles 19.4 -> 15.2 us.  What
+// is left is bound by FP32 and FP64 issue at 8 waves per SIMD.
+template <int ET, int KIND, int HALVES>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8)))
 k_element_patch(ElemArgs A) {
   using T = Elem<ET>;
   constexpr int d = T::d, n = T::n, dn = d * n;
+  constexpr bool FAST = HALVES > 0;
   extern __shared__ __align__(16) unsigned char smem[];
   const int64_t b = logical_block(A.xcd_remap);
-  const int64_t e0 = b * int64_t(blockDim.x);
+  const int64_t e0 = b * 256;
   if (e0 >= A.count) return;  // uniform over the block
-  const int ne = int(min<int64_t>(blockDim.x, A.count - e0));
+  const int ne = int(min<int64_t>(256, A.count - e0));
   // per-patch lists are padded to a fixed stride S (the largest patch), so
   // that no load waits for the patch's offset; padding repeats a valid node
   const int S = A.patch_max_nodes;
@@ -1232,13 +1246,33 @@ k_element_patch(ElemArgs A) {
   uint32_t* s_rs = reinterpret_cast<uint32_t*>(s_ux + size_t(S) * 2 * d);
   uint16_t* s_rb = reinterpret_cast<uint16_t*>(s_rs + S);
   float* s_f = reinterpret_cast<float*>(smem + patch_force_offset(S, d));
-  // the element's own indices do not depend on the staged nodes: issue their
-  // loads first so that both latency chains overlap
   const int t = threadIdx.x;
   const int64_t e = e0 + min(t, ne - 1);
+  const uint32_t m_nodes = A.pnode_cnt[b];
+  // node values relative to the patch's first node, formed in FP64 and then
+  // rounded: the element differences below stay accurate in FP32
+  const uint32_t ref = A.pnode_ids[k0];
+  double uref[d], xref[d];
+#pragma unroll
+  for (int i = 0; i < d; ++i) {
+    uref[i] = A.u[int64_t(ref) * d + i];
+    xref[i] = A.X[int64_t(ref) * d + i];
+  }
+  auto stage = [&](int k, const double* u, const double* X) {
+    float v[2 * d];
+#pragma unroll
+    for (int i = 0; i < d; ++i) {
+      v[i] = float(u[i] - uref[i]);
+      v[d + i] = float(X[i] - xref[i]);
+    }
+    float2* dst = reinterpret_cast<float2*>(s_ux + size_t(k) * 2 * d);
+#pragma unroll
+    for (int j = 0; j < d; ++j) dst[j] = make_float2(v[2 * j], v[2 * j + 1]);
+  };
   int ln[n], rk[n];
-  if (A.lcr) {
-    // packed: patch-local node | rank << 8, one 8- or 16-byte load per element
+  MatParams m = A.mat0;
+  uint32_t pos[FAST ? HALVES : 1];  // FAST: where the partials of nodes t, t + 256 go
+  if constexpr (FAST) {
     constexpr int np = n == 3 ? 4 : n;
     uint32_t w[np / 2];
     if constexpr (np == 4) {
@@ -1249,53 +1283,85 @@ k_element_patch(ElemArgs A) {
       const uint4 v = reinterpret_cast<const uint4*>(A.lcr)[e];
       w[0] = v.x; w[1] = v.y; w[2] = v.z; w[3] = v.w;
     }
+    constexpr bool runs = KIND != SUR_STRAIN;
+    const int mn = int(m_nodes);
+    uint32_t id[HALVES], rb[HALVES];
+#pragma unroll
+    for (int h = 0; h < HALVES; ++h) {
+      const int k = min(t + 256 * h, mn - 1);
+      id[h] = A.pnode_ids[k0 + k];
+      if constexpr (runs) {
+        pos[h] = A.part_pos[k0 + k];
+        // one base more than nodes: the end of the last run
+        rb[h] = A.run_base[b * int64_t(S + 1) + min(t + 256 * h, mn)];
+      }
+    }
+    double u[HALVES][d], X[HALVES][d];
+#pragma unroll
+    for (int h = 0; h < HALVES; ++h) {
+      const uint32_t at = id[h] * uint32_t(d * 8);
+      const double* pu = reinterpret_cast<const double*>(reinterpret_cast<const char*>(A.u) + at);
+      const double* px = reinterpret_cast<const double*>(reinterpret_cast<const char*>(A.X) + at);
+#pragma unroll
+      for (int i = 0; i < d; ++i) {
+        u[h][i] = pu[i];
+        X[h][i] = px[i];
+      }
+    }
+    if (A.elem_mat) m = A.mats[A.elem_mat[e]];
+#pragma unroll
+    for (int h = 0; h < HALVES; ++h) {
+      const int k = t + 256 * h;
+      if (k < mn) stage(k, u[h], X[h]);
+      if (runs && k <= mn) s_rb[k] = uint16_t(rb[h]);
+    }
+    const int shift = A.lcr_shift;
+    const uint32_t low = (1u << shift) - 1u;
 #pragma unroll
     for (int a = 0; a < n; ++a) {
       const uint32_t h = (w[a >> 1] >> (16 * (a & 1))) & 0xffffu;
-      ln[a] = int(h & 0xffu);
-      rk[a] = int(h >> 8);
+      ln[a] = int(h & low);
+      rk[a] = int(h >> shift);
     }
   } else {
+    if (A.lcr) {
+      constexpr int np = n == 3 ? 4 : n;
+      const int shift = A.lcr_shift;
 #pragma unroll
-    for (int a = 0; a < n; ++a) {
-      ln[a] = A.lconn[a * A.E + e];
-      rk[a] = A.lrank[a * A.E + e];
+      for (int a = 0; a < n; ++a) {
+        const uint32_t h = A.lcr[e * np + a];
+        ln[a] = int(h & ((1u << shift) - 1u));
+        rk[a] = int(h >> shift);
+      }
+    } else {
+#pragma unroll
+      for (int a = 0; a < n; ++a) {
+        ln[a] = A.lconn[a * A.E + e];
+        rk[a] = A.lrank[a * A.E + e];
+      }
     }
-  }
-  const int mat = A.elem_mat ? A.elem_mat[e] : 0;
-  const uint32_t m_nodes = A.pnode_cnt[b];
-  // node values relative to the patch's first node, formed in FP64 and then
-  // rounded: the element differences below stay accurate in FP32
-  const int64_t ref = A.pnode_ids[k0];
-  double uref[d], xref[d];
+    if (A.elem_mat) m = A.mats[A.elem_mat[e]];
+    for (int k = t; k < S; k += 256) {
+      const int64_t node = A.pnode_ids[k0 + k];
+      double u[d], X[d];
 #pragma unroll
-  for (int i = 0; i < d; ++i) {
-    uref[i] = A.u[ref * d + i];
-    xref[i] = A.X[ref * d + i];
-  }
-  for (int k = threadIdx.x; k < S; k += blockDim.x) {
-    const int64_t node = A.pnode_ids[k0 + k];
-    float v[2 * d];
-#pragma unroll
-    for (int i = 0; i < d; ++i) {
-      v[i] = float(A.u[node * d + i] - uref[i]);
-      v[d + i] = float(A.X[node * d + i] - xref[i]);
+      for (int i = 0; i < d; ++i) {
+        u[i] = A.u[node * d + i];
+        X[i] = A.X[node * d + i];
+      }
+      stage(k, u, X);
+      if constexpr (KIND != SUR_STRAIN) {
+        // run start (layout 2) or the partial's node-major position (layout 5)
+        if (!A.partials) s_rs[k] = A.run_start[k0 + k];
+        else if (A.part_pos) s_rs[k] = A.part_pos[k0 + k];
+        s_rb[k] = A.run_base[b * int64_t(S + 1) + k];
+      }
     }
-    float2* dst = reinterpret_cast<float2*>(s_ux + size_t(k) * 2 * d);
-#pragma unroll
-    for (int j = 0; j < d; ++j) dst[j] = make_float2(v[2 * j], v[2 * j + 1]);
-    if constexpr (KIND != SUR_STRAIN) {
-      // run start (layout 2) or the partial's node-major position (layout 5)
-      if (!A.partials) s_rs[k] = A.run_start[k0 + k];
-      else if (A.part_pos) s_rs[k] = A.part_pos[k0 + k];
-      s_rb[k] = A.run_base[b * int64_t(S + 1) + k];
-    }
+    if (KIND != SUR_STRAIN && t == 0) s_rb[S] = A.run_base[b * int64_t(S + 1) + S];
   }
-  if (KIND != SUR_STRAIN && threadIdx.x == 0) s_rb[S] = A.run_base[b * int64_t(S + 1) + S];
   __syncthreads();
   bool outside = false;  // surrogate strain pass: point outside the envelope
   if (t < ne) {
-    const MatParams m = A.mats[mat];
     auto node_ux = [&](int k, float* v) {
       const float2* src = reinterpret_cast<const float2*>(s_ux + size_t(k) * 2 * d);
 #pragma unroll
@@ -1341,17 +1407,17 @@ k_element_patch(ElemArgs A) {
     return;
   }
   __syncthreads();
-  if (A.partials) {
+  if (FAST || A.partials) {
     // one sum per patch node, its run summed in element order in FP64 and
     // stored in FP64 (partials 1) or rounded once to FP32 (partials 2)
-    for (uint32_t k = threadIdx.x; k < m_nodes; k += blockDim.x) {
+    for (uint32_t k = threadIdx.x; k < m_nodes; k += 256) {
       double f[d];
 #pragma unroll
       for (int i = 0; i < d; ++i) f[i] = 0.;
       // chunks of RUNCHUNK entries: a chunk's LDS reads are issued together.
-      // Full chunks add unmasked; the last, partial chunk reads into the
-      // force area's RUNCHUNK - 1 entries of padding and its entries past
-      // the run add +0, so the sum is the sequential one.  Patch-local nodes
+      // Full chunks add unmasked; the last, partial chunk (of at most
+      // RUNCHUNK - 1 entries) reads into the force area's padding and its
+      // entries past the run add +0, so the sum is the sequential one.  Patch-local nodes
       // are numbered by decreasing run length, so the lanes of a wavefront
       // run about the same number of chunks.
       const int q1 = s_rb[k + 1];
@@ -1366,16 +1432,20 @@ k_element_patch(ElemArgs A) {
           for (int i = 0; i < d; ++i) f[i] += double(v[j * d + i]);
       }
       if (q < q1) {
-        float v[RUNCHUNK * d];
+        float v[(RUNCHUNK - 1) * d];
 #pragma unroll
-        for (int j = 0; j < RUNCHUNK * d; ++j) v[j] = s_f[q * d + j];
+        for (int j = 0; j < (RUNCHUNK - 1) * d; ++j) v[j] = s_f[q * d + j];
 #pragma unroll
-        for (int j = 0; j < RUNCHUNK; ++j)
+        for (int j = 0; j < RUNCHUNK - 1; ++j)
 #pragma unroll
-          for (int i = 0; i < d; ++i) f[i] += double(q + j < q1 ? v[j * d + i] : 0.f);
+          for (int i = 0; i < d; ++i) {
+            // masked by bits, so that the select is one on the 32-bit value
+            const uint32_t keep = j == 0 || q + j < q1 ? ~0u : 0u;
+            f[i] += double(__uint_as_float(__float_as_uint(v[j * d + i]) & keep));
+          }
       }
-      const int64_t at = A.part_pos ? int64_t(s_rs[k]) : k0 + k;
-      if (A.partials == 2) {
+      const int64_t at = FAST ? int64_t(pos[HALVES > 1 ? k >> 8 : 0]) : A.part_pos ? int64_t(s_rs[k]) : k0 + k;
+      if (FAST || A.partials == 2) {
         float* __restrict__ part = static_cast<float*>(A.slots);
 #pragma unroll
         for (int i = 0; i < d; ++i) part[at * d + i] = float(f[i]);
@@ -1390,7 +1460,7 @@ k_element_patch(ElemArgs A) {
   // contiguous runs: output q belongs to the node k with rb[k] <= q < rb[k+1]
   float* __restrict__ out = static_cast<float*>(A.slots);
   const int total = ne * n;
-  for (int q = threadIdx.x; q < total; q += blockDim.x) {
+  for (int q = threadIdx.x; q < total; q += 256) {
     int lo = 0, hi = int(m_nodes);  // s_rb[lo] <= q < s_rb[hi]
     while (hi - lo > 1) {
       const int mid = (lo + hi) >> 1;
@@ -2296,6 +2366,19 @@ hipError_t launch_mass(int et, hipStream_t s, int64_t N, int64_t E, const uint32
   return hipGetLastError();
 }
 
+// one block per patch of 256 elements (the patches are built for that size)
+template <int ET, int KIND>
+static void launch_patch(hipStream_t s, const ElemArgs& A) {
+  const unsigned g = unsigned(A.patch_blocks);
+  const bool fast = A.lcr && A.partials == 2 && A.part_pos && A.nodal_bytes < (int64_t(1) << 32);
+  if (fast && A.patch_max_nodes < 256)
+    k_element_patch<ET, KIND, 1><<<g, 256, A.patch_lds, s>>>(A);
+  else if (fast && A.patch_max_nodes < 512)
+    k_element_patch<ET, KIND, 2><<<g, 256, A.patch_lds, s>>>(A);
+  else
+    k_element_patch<ET, KIND, 0><<<g, 256, A.patch_lds, s>>>(A);
+}
+
 template <int ET>
 static hipError_t launch_element_et(int kind, int precision, hipStream_t s, const ElemArgs& A,
                                     int block) {
@@ -2333,8 +2416,7 @@ static hipError_t launch_element_et(int kind, int precision, hipStream_t s, cons
     if constexpr (ET == TET4) {
       if (kind != NH_DAMAGE) return hipErrorInvalidValue;
       const unsigned ge = grid_for(A.count, 256);
-      if (A.patch)
-        k_element_patch<TET4, SUR_STRAIN><<<unsigned(A.patch_blocks), 256, A.patch_lds, s>>>(A);
+      if (A.patch) launch_patch<TET4, SUR_STRAIN>(s, A);
       else
         k_sur_strain<<<ge, 256, 0, s>>>(A);
       hipError_t err = hipGetLastError();
@@ -2343,20 +2425,17 @@ static hipError_t launch_element_et(int kind, int precision, hipStream_t s, cons
       err = launch_sur_mlp(s, A.sur_img, A.sur_b, A.sur_bf16, A.count, A.sur_x, 8, A.sur_y, 8);
       if (err != hipSuccess) return err;
       if (A.net_ev1) (void)hipEventRecord(A.net_ev1, s);
-      if (A.patch)
-        k_element_patch<TET4, NH_DAMAGE_SUR><<<unsigned(A.patch_blocks), 256, A.patch_lds, s>>>(A);
+      if (A.patch) launch_patch<TET4, NH_DAMAGE_SUR>(s, A);
       else
         k_sur_forces<<<ge, 256, 0, s>>>(A);
     } else {
       return hipErrorInvalidValue;
     }
   } else if (A.patch) {
-    // one block per patch of 256 elements (the patches are built for that size)
-    const unsigned gp = unsigned(A.patch_blocks);
     switch (kind) {
-    case ELASTIC: k_element_patch<ET, ELASTIC><<<gp, 256, A.patch_lds, s>>>(A); break;
-    case NEOHOOKEAN: k_element_patch<ET, NEOHOOKEAN><<<gp, 256, A.patch_lds, s>>>(A); break;
-    case NH_DAMAGE: k_element_patch<ET, NH_DAMAGE><<<gp, 256, A.patch_lds, s>>>(A); break;
+    case ELASTIC: launch_patch<ET, ELASTIC>(s, A); break;
+    case NEOHOOKEAN: launch_patch<ET, NEOHOOKEAN>(s, A); break;
+    case NH_DAMAGE: launch_patch<ET, NH_DAMAGE>(s, A); break;
     default: return hipErrorInvalidValue;
     }
   } else {
