@@ -75,7 +75,7 @@ void free_derived(akx_ctx* c) {
   dfree(c->node_inv_d); dfree(c->elem_inv_d);
   dfree(c->fel_off); dfree(c->fel); dfree(c->flslot); dfree(c->fch_off); dfree(c->fcbase);
   dfree(c->fblk); dfree(c->fhalo_off); dfree(c->fhalo); dfree(c->fsrec); dfree(c->fsmat);
-  dfree(c->u_alt); dfree(c->pcoef); dfree(c->frec);
+  dfree(c->u_alt); dfree(c->pcoef);
   c->fused_ok = false;
   c->fused_default = false;
   c->patch_ok = false;
@@ -645,7 +645,7 @@ int build_fused(akx_ctx* c, const std::vector<uint32_t>& order, const std::vecto
   // block-local number of a node, valid for the list that stamped it
   std::vector<uint32_t> loc(N), seen(N, 0);
   uint32_t stamp = 0;
-  size_t lds_max = 0;
+  size_t lds_max = 0, lds_mixed = 0, lds_max_mixed = 0;
   // Elements (by rank) of the nodes [n0, n1), where each node's run of each
   // chunk starts, and the LDS the block takes with its nodes staged.
   auto list = [&](int64_t n0, int64_t n1) -> size_t {
@@ -682,7 +682,9 @@ int build_fused(akx_ctx* c, const std::vector<uint32_t>& order, const std::vecto
           loc[v[a]] = own ? uint32_t(v[a] - n0) : uint32_t(n1 - n0) + others++;
         }
     }
-    return ((size_t(n1 - n0) + others) * 2 + slots) * size_t(d) * 8;
+    const size_t nodes = (size_t(n1 - n0) + others) * 2;
+    lds_mixed = (nodes * 8 + slots * 4) * size_t(d);
+    return (nodes + slots) * size_t(d) * 8;
   };
   // Small meshes take smaller blocks: a block's chunks follow one another, so
   // that few large blocks leave most of the chip idle for the longest time
@@ -712,6 +714,7 @@ int build_fused(akx_ctx* c, const std::vector<uint32_t>& order, const std::vecto
     }
     next = std::min(most, n1 - n0 + 16);
     lds_max = std::max(lds_max, lds);
+    lds_max_mixed = std::max(lds_max_mixed, lds_mixed);
     blk.push_back(uint32_t(n1));
     el_off.push_back(uint32_t(el.size()));
     ch_off.push_back(uint32_t(cbase.size() / (FUSED_NB + 1)));
@@ -773,7 +776,8 @@ int build_fused(akx_ctx* c, const std::vector<uint32_t>& order, const std::vecto
   HIP_TRY(c, hipMemcpy(c->fcbase, cbase.data(), cbase.size() * 2, hipMemcpyHostToDevice));
   c->fused_blocks = nblk;
   c->fused_elements = int64_t(el.size());
-  c->fused_lds = FUSED_CH * n * d * 4;  // the mixed step's FP32 contributions
+  // the mixed step: FP32 contributions, behind the nodes if they are staged
+  c->fused_lds = staged ? int(lds_max_mixed) : FUSED_CH * n * d * 4;
   if (staged) {
     HIP_TRY(c, dalloc(&c->fhalo_off, halo_off.size()));
     HIP_TRY(c, dalloc(&c->fhalo, halo.size()));
@@ -1207,24 +1211,6 @@ int akx_init(akx_ctx* c) {
   // (position form), the fused step's output
   if (!c->u_alt) HIP_TRY(c, dalloc(&c->u_alt, size_t(N) * d));
   HIP_TRY(c, dalloc(&c->pcoef, size_t(N)));
-  // the fused mixed step on triangles streams one 32-byte record per
-  // evaluation (built here, after the material indices it carries are on
-  // the device; X is fixed after akx_init): node ids in 23 bits and material
-  // indices in 17, else it gathers through element ids
-  if (c->fused_ok && c->et == AKX_TRIANGLE_3 && N <= FUSED_REC_MAX_NODES &&
-      int64_t(nm) <= FUSED_REC_MAX_MATERIALS) {
-    HIP_TRY(c, dalloc(&c->frec, size_t(c->fused_elements) * 2));
-    float* geo = nullptr;  // per element, only to build the records
-    HIP_TRY(c, dalloc(&geo, size_t(E) * fused_geo_stride(n, d)));
-    hipError_t er = launch_fused_geometry(c->et, c->stream, E, c->X, c->conn_soa, geo);
-    if (er == hipSuccess)
-      er = launch_fused_records(c->stream, c->fused_elements, E, c->fel, c->conn_soa, geo,
-                                c->flslot, c->elem_mat_d, c->frec);
-    const hipError_t es = hipStreamSynchronize(c->stream);
-    dfree(geo);
-    HIP_TRY(c, er);
-    HIP_TRY(c, es);
-  }
   if (any_damage) {
     std::vector<double> yd(size_t(E) * Q, 0.), ydi(size_t(E) * Q);
     for (int64_t e = 0; e < E; ++e) {
@@ -1608,10 +1594,6 @@ int enqueue_steps(akx_ctx* c, int nsteps, int precision, bool timing) {
       F.ch_off = c->fch_off;
       F.cbase = c->fcbase;
       F.u_out = unext;
-      // B rebuilt from the streamed records (mixed_recompute 1) or from
-      // coordinates gathered through element ids (0): the same forces bit
-      // for bit
-      F.rec = c->mixed_recompute ? c->frec : nullptr;
       F.blk = c->fblk;
       F.halo_off = c->fhalo_off;
       F.halo = c->fhalo;
@@ -1864,7 +1846,7 @@ int akx_query(akx_ctx* c, const char* key, double* value) {
   else if (k == "fused_available") *value = c->fused_ok ? 1. : 0.;
   else if (k == "fused_blocks") *value = double(c->fused_ok ? c->fused_blocks : 0);
   else if (k == "fused_staged_lds") *value = double(c->fsrec ? c->fused_staged_lds : 0);
-  else if (k == "fused_records") *value = c->frec ? 1. : 0.;
+  else if (k == "fused_records") *value = c->fsrec ? 1. : 0.;
   else if (k == "fused_elements") *value = double(c->fused_ok ? c->fused_elements : 0);
   else if (k == "element_block") *value = c->elem_block;
   else if (k == "node_block") *value = c->node_block;
@@ -2081,12 +2063,9 @@ int akx_autotune(akx_ctx* c, int precision, int nsteps, int* chosen, double* bes
               cand.push_back(Shape{eb, nb, x, rcmp, lay, stage});
             }
           }
-  // the fused step (layout 6) has its own block shapes and rebuilds B; on the
-  // mixed path from per-evaluation records (mixed_recompute 1, triangles)
-  // or from coordinates gathered through element ids (0)
+  // the fused step (layout 6) has its own block shapes and rebuilds B
   if (c->fused_ok)
-    for (int rcmp = (precision == AKX_MIXED && c->frec ? 0 : 1); rcmp < 2; ++rcmp)
-      for (int x = 0; x < 2; ++x) cand.push_back(Shape{256, 256, x, rcmp, 6, 0});
+    for (int x = 0; x < 2; ++x) cand.push_back(Shape{256, 256, x, 1, 6, 0});
   for (const Shape& sh : cand) {
           const int eb = sh.eb, nb = sh.nb, x = sh.x, lay = sh.lay;
           c->elem_block = eb; c->node_block = nb; c->xcd_remap = x; c->node_ordered = lay;

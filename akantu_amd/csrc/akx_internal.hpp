@@ -119,15 +119,11 @@ struct FusedArgs {
   const uint32_t* ch_off;  // [nblk + 1] first chunk table of each block
   const uint16_t* cbase;   // [chunk * (FUSED_NB + 1) + k] first slot of block node k in the chunk
   double* u_out;           // displacement written by the step (read from NodeArgs::u)
-  // mixed path on triangles: per evaluation j (entry of el), everything the
-  // element needs but u, 32 bytes read as a stream (nullptr: element ids and
-  // gathers instead): rec[2 j] = the element's coordinate differences
-  // x_a - x_0, a = 1, 2 (4 FP32); rec[2 j + 1] = fused_record_ids(...)
-  const uint4* rec;
-  // FP64 path, nodes staged in LDS: the nodes beyond its own that a block's
-  // elements touch, and per evaluation one word per node, block-local number (own nodes first, then the halo) |
-  // LDS slot << 16 (0xFFFF: not a block node); the fourth word of a triangle
-  // is its material, larger elements have it in smat (several materials)
+  // nodes staged in LDS (srec nullptr: not): the nodes beyond its own that a
+  // block's elements touch, and per evaluation one word per node, block-local
+  // number (own nodes first, then the halo) | LDS slot << 16 (0xFFFF: not a
+  // block node); the fourth word of a triangle is its material, larger
+  // elements have it in smat (several materials)
   const uint32_t* halo_off;  // [nblk + 1] offsets into halo
   const uint32_t* halo;
   const uint4* srec;
@@ -140,26 +136,6 @@ struct FusedArgs {
 // elements, runs on slots).
 constexpr size_t FUSED_STAGED_LDS = 40 * 1024 - 512;
 constexpr int64_t FUSED_NB_MIN = 32;
-
-// Second word of a fused triangle record: the three node ids in the low 23
-// bits of x, y, z; LDS slots 0 and 1 in w (16 bits each, 0xFFFF: not a block
-// node); LDS slot 2 in 10 bits (0x3FF: not a block node) and the material in
-// 17 bits spread over the high 9 bits of x, y, z.
-constexpr int FUSED_REC_NODE_BITS = 23;
-constexpr int64_t FUSED_REC_MAX_NODES = int64_t(1) << FUSED_REC_NODE_BITS;
-constexpr int FUSED_REC_MAX_MATERIALS = 1 << 17;
-constexpr uint32_t FUSED_REC_SLOT2_NONE = 0x3FFu;
-__host__ __device__ inline uint4 fused_record_ids(uint32_t n0, uint32_t n1, uint32_t n2,
-                                                  uint32_t s0, uint32_t s1, uint32_t s2,
-                                                  uint32_t mat) {
-  const uint32_t q = s2 == 0xFFFFu ? FUSED_REC_SLOT2_NONE : s2;
-  return make_uint4(n0 | (q & 0x1FFu) << 23, n1 | (q >> 9) << 23 | (mat & 0xFFu) << 24,
-                    n2 | (mat >> 8) << 23, s0 | s1 << 16);
-}
-
-// Floats per element of the fused mixed step's geometry record: (n - 1) d
-// coordinate differences, padded to whole 16-byte vectors.
-constexpr int fused_geo_stride(int n, int d) { return ((n - 1) * d + 3) & ~3; }
 
 enum NodeMode {
   NODE_CORRECT = 1,     // gather forces, residual, lumped solve, corrector
@@ -210,11 +186,6 @@ hipError_t launch_fused(int et, int kind, int precision, bool has_fext, hipStrea
                         const ElemArgs& EA, const NodeArgs& NA, const FusedArgs& F, int lds);
 hipError_t launch_node(int d, int precision, bool has_fext, hipStream_t s, const NodeArgs& A,
                        int block);
-hipError_t launch_fused_records(hipStream_t s, int64_t J, int64_t E, const uint32_t* el,
-                                const uint32_t* conn_soa, const float* geo, const uint16_t* lslot,
-                                const uint16_t* elem_mat, uint4* rec);
-hipError_t launch_fused_geometry(int et, hipStream_t s, int64_t E, const double* X,
-                                 const uint32_t* conn_soa, float* geo);
 hipError_t launch_stable_dt(int et, hipStream_t s, int64_t E, const double* X, const double* u,
                             const uint32_t* conn_soa, const uint16_t* elem_mat,
                             const MatParams* mats, double* partial, int nblocks_max,
@@ -423,7 +394,6 @@ struct akx_ctx {
   uint16_t* fsmat = nullptr;
   double* u_alt = nullptr;  // second displacement buffer (position form, fused step)
   double* pcoef = nullptr;  // position form: dt^2 / M per node
-  uint4* frec = nullptr;     // per-evaluation records of the fused mixed step (triangles)
   akx::ElemTablesF tabf;
   akx::ElemTables* tab64_d = nullptr;
   // internal numbering: perm[internal] = caller id, inv[caller id] = internal

@@ -1879,6 +1879,53 @@ __global__ void __launch_bounds__(256) k_node(NodeArgs A) {
 //   much as fewer repeated elements: 240 us with 54 KB of LDS a block (9.8 M
 //   evaluations), 183 with 40 KB (10.3 M), 199 with 32 KB (11.2 M).
 // ===========================================================================
+// Place of pair i of (u, X) of staged node k in LDS.  In 2D u and X lie in an
+// array each, 16 bytes a node: one after the other, the nodes' u would use
+// every other group of four banks only.  In 3D a node's 48 bytes spread over
+// the banks by themselves.
+template <int d>
+__device__ __forceinline__ int staged_pair(int k, int i, int total) {
+  return d == 2 ? i * total + k : k * d + i;
+}
+
+// u and X of a block's own nodes n0, n0 + 1, ... (cnt <= 256 of them) and of its
+// halo into LDS.  The halo's node ids are asked for before the own nodes'
+// values, and those are not waited for before the halo's are under way; the
+// halo starts at the last thread, so that a small block's wavefronts have one
+// or the other.
+template <int d>
+__device__ __forceinline__ void stage_nodes(const double* __restrict__ u,
+                                            const double* __restrict__ X, int64_t n0, int cnt,
+                                            const uint32_t* __restrict__ halo, int total,
+                                            double2* s_n) {
+  const int t = threadIdx.x, r = 255 - t, H = total - cnt;
+  uint32_t id = 0;
+  if (r < H) id = halo[r];
+  double v[2 * d];
+  if (t < cnt)
+#pragma unroll
+    for (int i = 0; i < d; ++i) {
+      v[i] = u[(n0 + t) * d + i];
+      v[d + i] = X[(n0 + t) * d + i];
+    }
+  for (int k = r; k < H; k += 256) {
+    double w[2 * d];
+#pragma unroll
+    for (int i = 0; i < d; ++i) {
+      w[i] = u[int64_t(id) * d + i];
+      w[d + i] = X[int64_t(id) * d + i];
+    }
+    if (k + 256 < H) id = halo[k + 256];
+#pragma unroll
+    for (int i = 0; i < d; ++i)
+      s_n[staged_pair<d>(cnt + k, i, total)] = make_double2(w[2 * i], w[2 * i + 1]);
+  }
+  if (t < cnt)
+#pragma unroll
+    for (int i = 0; i < d; ++i)
+      s_n[staged_pair<d>(t, i, total)] = make_double2(v[2 * i], v[2 * i + 1]);
+}
+
 template <int ET, int KIND, bool HAS_FEXT>
 __global__ void __launch_bounds__(256) k_step_fused(ElemArgs EA, NodeArgs NA, FusedArgs F) {
   static_assert(KIND != NH_DAMAGE, "the fused step recomputes elements: stateless laws only");
@@ -1906,20 +1953,9 @@ __global__ void __launch_bounds__(256) k_step_fused(ElemArgs EA, NodeArgs NA, Fu
   const int total = cnt + int(F.halo_off[b + 1] - h0);
   // u and X of the staged nodes, 2 d doubles each, then the contributions of
   // a chunk, d each
-  double* s_n = reinterpret_cast<double*>(smem);
-  double* s_f = s_n + size_t(total) * 2 * d;
-  for (int k = t; k < total; k += 256) {
-    const int64_t nd = k < cnt ? n0 + k : int64_t(F.halo[h0 + uint32_t(k - cnt)]);
-    double v[2 * d];
-#pragma unroll
-    for (int i = 0; i < d; ++i) {
-      v[i] = u_in[nd * d + i];
-      v[d + i] = EA.X[nd * d + i];
-    }
-    double2* dst = reinterpret_cast<double2*>(s_n + size_t(k) * 2 * d);
-#pragma unroll
-    for (int i = 0; i < d; ++i) dst[i] = make_double2(v[2 * i], v[2 * i + 1]);
-  }
+  double2* s_n = reinterpret_cast<double2*>(smem);
+  double* s_f = reinterpret_cast<double*>(s_n + size_t(total) * d);
+  stage_nodes<d>(u_in, EA.X, n0, cnt, F.halo + h0, total, s_n);
   __syncthreads();
   uint32_t c = 0;
   for (uint32_t jc = j0; jc < j1; jc += FUSED_CH, ++c) {
@@ -1943,11 +1979,10 @@ __global__ void __launch_bounds__(256) k_step_fused(ElemArgs EA, NodeArgs NA, Fu
 #pragma unroll
       for (int a = 0; a < n; ++a) {
         ls[a] = w[a] >> 16;
-        const double2* src = reinterpret_cast<const double2*>(s_n + (w[a] & 0xFFFFu) * (2 * d));
         double v[2 * d];
 #pragma unroll
         for (int i = 0; i < d; ++i) {
-          const double2 p = src[i];
+          const double2 p = s_n[staged_pair<d>(int(w[a] & 0xFFFFu), i, total)];
           v[2 * i] = p.x;
           v[2 * i + 1] = p.y;
         }
@@ -1992,7 +2027,8 @@ __global__ void __launch_bounds__(256) k_step_fused(ElemArgs EA, NodeArgs NA, Fu
   uint8_t bl[d];
 #pragma unroll
   for (int i = 0; i < d; ++i) {
-    u[i] = s_n[t * 2 * d + i];
+    const double2 p = s_n[staged_pair<d>(t, i / 2, total)];
+    u[i] = i & 1 ? p.y : p.x;
     v[i] = NA.v[node * d + i];
     acc[i] = NA.a[node * d + i];
     bl[i] = NA.blocked[node * d + i];
@@ -2495,16 +2531,26 @@ static hipError_t launch_node_d(int precision, bool has_fext, hipStream_t s, con
 // arithmetic), contributions in LDS in FP32, each node's run summed in FP64,
 // the node update in the position form of the mixed path.  Its
 // sums follow the FP64 path's assembly order (any fixed order will do here).
-// RECORD (triangles): the element data come from F.rec.
-template <int ET, int KIND, bool HAS_FEXT, bool RECORD>
+// STAGED: u and X of the block's nodes copied into LDS in FP64 and an element
+// read as a 16-byte record of local numbers, as in the FP64 step; else (a node
+// in so many elements that no block holds its nodes) through element ids, with
+// the same forces bit for bit.
+// Against gathering u through L2 (for triangles with 32-byte records that held
+// the coordinate differences): 4,000 triangles 5.3 -> 3.5 us per step, 1.6 M
+// 20.9 -> 20.5, 2.5 M in 128 specimens of a material each 30.5 -> 29.1;
+// 800,000 quadrangles 24.2 -> 23.1, 1.3 M tetrahedra 52 -> 35.  On 1.6 M
+// triangles the vector units are busy for about half of the time; LDS was for
+// 40 %, over half of that in bank conflicts, before u and X had an array each
+// (staged_pair: 21.6 -> 21.0 us).  Blocks of 224 nodes, whose elements fill two
+// chunks instead of 2.25, gain nothing, and the node's own data asked for ahead
+// of the elements' cost 1 us.
+template <int ET, int KIND, bool HAS_FEXT, bool STAGED>
 __global__ void __launch_bounds__(256) k_step_fused_mixed(ElemArgs EA, NodeArgs NA, FusedArgs F) {
-  static_assert(!RECORD || ET == TRI3, "per-evaluation records exist for triangles only");
   static_assert(KIND != NH_DAMAGE, "the fused step recomputes elements: stateless laws only");
   static_assert(FUSED_NB <= 256 && FUSED_CH == 256, "one node and one element per thread of 256");
   using T = Elem<ET>;
   constexpr int d = T::d, n = T::n, dn = d * n;
   extern __shared__ __align__(16) unsigned char smem[];
-  float* s_f = reinterpret_cast<float*>(smem);  // FUSED_CH * n contributions, d each
   const int64_t b = logical_block(NA.xcd_remap);
   if (b >= F.nblk) return;  // uniform over the block
   const int t = threadIdx.x;
@@ -2519,79 +2565,99 @@ __global__ void __launch_bounds__(256) k_step_fused_mixed(ElemArgs EA, NodeArgs 
   for (int i = 0; i < d; ++i) f[i] = 0.;
   const uint32_t j0 = F.el_off[b], j1 = F.el_off[b + 1];
   const uint32_t c0 = F.ch_off[b];
+  // STAGED: u and X of the nodes, then the contributions of a chunk
+  double2* s_n = reinterpret_cast<double2*>(smem);
+  float* s_f = reinterpret_cast<float*>(smem);
+  int total = 0;  // nodes staged
+  uint4 rec = make_uint4(0, 0, 0, 0);
+  if constexpr (STAGED) {
+    // the first elements' records travel with the nodes
+    if (j0 + uint32_t(t) < j1) rec = F.srec[j0 + uint32_t(t)];
+    const uint32_t h0 = F.halo_off[b];
+    total = cnt + int(F.halo_off[b + 1] - h0);
+    s_f = reinterpret_cast<float*>(s_n + size_t(total) * d);
+    stage_nodes<d>(u_in, EA.X, n0, cnt, F.halo + h0, total, s_n);
+    __syncthreads();
+  }
   uint32_t c = 0;
   for (uint32_t jc = j0; jc < j1; jc += FUSED_CH, ++c) {
     const uint32_t j = jc + uint32_t(t);
+    // where the node's run of this chunk lies, needed after the barrier
+    int q0 = 0, q1 = 0;
+    if (owner) {
+      const uint16_t* cb = F.cbase + size_t(c0 + c) * (FUSED_NB + 1);
+      q0 = cb[t];
+      q1 = cb[t + 1];
+    }
     if (j < j1) {
-      // Triangles with records read one 32-byte record per evaluation, in
-      // the block's evaluation order: the coordinate differences (the same
-      // values k_fused_geometry formed from X), the node ids, the LDS slots
-      // and the material, streamed instead of an element id and its
-      // dependent gathers of connectivity, geometry and material; both forms
-      // give the same forces bit for bit.  Larger elements share their
-      // nodes among more elements and gather X (cached) faster than they
-      // would read a record.
-      constexpr int G = RECORD ? 4 : 1;
-      static_assert(FUSED_CH * 3 < int(FUSED_REC_SLOT2_NONE), "LDS slots fit the records");
-      int64_t e = 0;  // element id (not needed with a record)
+      int64_t e = 0;  // element id (not needed with records)
       int mat = 0;
-      int64_t nd[n];
       uint32_t lsl[n];
-      float gx[G];
-      if constexpr (RECORD) {
-        const uint4 r0 = F.rec[size_t(j) * 2], r1 = F.rec[size_t(j) * 2 + 1];
-        constexpr uint32_t LOW = (1u << FUSED_REC_NODE_BITS) - 1u;
-        gx[0] = __uint_as_float(r0.x);
-        gx[1] = __uint_as_float(r0.y);
-        gx[2] = __uint_as_float(r0.z);
-        gx[3] = __uint_as_float(r0.w);
-        nd[0] = r1.x & LOW;
-        nd[1] = r1.y & LOW;
-        nd[2] = r1.z & LOW;
-        lsl[0] = r1.w & 0xFFFFu;
-        lsl[1] = r1.w >> 16;
-        const uint32_t s2 = (r1.x >> 23) | ((r1.y >> 23) & 1u) << 9;
-        lsl[2] = s2 == FUSED_REC_SLOT2_NONE ? 0xFFFFu : s2;
-        mat = int((r1.y >> 24) | (r1.z >> 23) << 8);
+      // differences to node 0 formed in FP64, then rounded
+      float du[dn], dX[dn];
+      auto differences = [&](int a, const double* u0, const double* x0, const double* u,
+                             const double* x) {
+#pragma unroll
+        for (int i = 0; i < d; ++i) {
+          du[i + a * d] = a ? float(u[i] - u0[i]) : 0.f;
+          dX[i + a * d] = a ? float(x[i] - x0[i]) : 0.f;
+        }
+      };
+      if constexpr (STAGED) {
+        const uint32_t w[4] = {rec.x, rec.y, rec.z, rec.w};
+        // triangles carry their material in the fourth word
+        if (n == 3) mat = int(rec.w);
+        else if (EA.elem_mat) mat = F.smat[j];
+        if (j + FUSED_CH < j1) rec = F.srec[j + FUSED_CH];
+        double v0[2 * d];
+#pragma unroll
+        for (int a = 0; a < n; ++a) {
+          lsl[a] = w[a] >> 16;
+          double v[2 * d];
+#pragma unroll
+          for (int i = 0; i < d; ++i) {
+            const double2 p = s_n[staged_pair<d>(int(w[a] & 0xFFFFu), i, total)];
+            v[2 * i] = p.x;
+            v[2 * i + 1] = p.y;
+          }
+          if (a == 0)
+#pragma unroll
+            for (int i = 0; i < 2 * d; ++i) v0[i] = v[i];
+          differences(a, v0, v0 + d, v, v + d);
+        }
       } else {
         e = F.el[j];
         mat = EA.elem_mat ? EA.elem_mat[e] : 0;
+        const int64_t first = EA.conn[e];
 #pragma unroll
-        for (int a = 0; a < n; ++a) nd[a] = EA.conn[a * E + e];
-#pragma unroll
-        for (int a = 0; a < n; ++a) lsl[a] = F.lslot[size_t(j) * n + a];
-      }
-      const MatParams m = EA.mats[mat];
-      // differences to node 0 formed in FP64, then rounded
-      float du[dn], dX[dn];
-#pragma unroll
-      for (int i = 0; i < d; ++i) {
-        const double u0 = u_in[nd[0] * d + i];
-        const double x0 = RECORD ? 0. : EA.X[nd[0] * d + i];
-        du[i] = 0.f;
-        dX[i] = 0.f;
-#pragma unroll
-        for (int a = 1; a < n; ++a) {
-          du[i + a * d] = float(u_in[nd[a] * d + i] - u0);
-          if constexpr (RECORD) dX[i + a * d] = gx[(a - 1) * d + i];
-          else dX[i + a * d] = float(EA.X[nd[a] * d + i] - x0);
+        for (int a = 0; a < n; ++a) {
+          const int64_t nd = EA.conn[a * E + e];
+          lsl[a] = F.lslot[size_t(j) * n + a];
+          differences(a, u_in + first * d, EA.X + first * d, u_in + nd * d, EA.X + nd * d);
         }
       }
+      const MatParams m = EA.mats[mat];
       float fe[dn];
       mixed_element_forces<ET, KIND, true>(EA, e, m, du, dX, fe);
 #pragma unroll
-      for (int a = 0; a < n; ++a) {
-        const uint32_t ls = lsl[a];
-        if (ls != 0xFFFFu)
+      for (int a = 0; a < n; ++a)
+        if (lsl[a] != 0xFFFFu)
 #pragma unroll
-          for (int i = 0; i < d; ++i) s_f[ls * d + i] = fe[i + a * d];
-      }
+          for (int i = 0; i < d; ++i) s_f[lsl[a] * d + i] = fe[i + a * d];
     }
     __syncthreads();
     if (owner) {
-      const uint16_t* cb = F.cbase + size_t(c0 + c) * (FUSED_NB + 1);
-      const int q0 = cb[t], q1 = cb[t + 1];
-      for (int q = q0; q < q1; ++q)
+      int q = q0;
+      for (; q + 4 <= q1; q += 4) {
+        float x[4 * d];
+#pragma unroll
+        for (int k = 0; k < 4 * d; ++k) x[k] = s_f[q * d + k];
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+#pragma unroll
+          for (int i = 0; i < d; ++i) f[i] += -1. * double(x[k * d + i]);
+      }
+      for (; q < q1; ++q)
 #pragma unroll
         for (int i = 0; i < d; ++i) f[i] += -1. * double(s_f[q * d + i]);
     }
@@ -2608,7 +2674,12 @@ __global__ void __launch_bounds__(256) k_step_fused_mixed(ElemArgs EA, NodeArgs 
   uint8_t bl[d];
 #pragma unroll
   for (int i = 0; i < d; ++i) {
-    u[i] = u_in[node * d + i];
+    if constexpr (STAGED) {
+      const double2 p = s_n[staged_pair<d>(t, i / 2, total)];
+      u[i] = i & 1 ? p.y : p.x;
+    } else {
+      u[i] = u_in[node * d + i];
+    }
     up[i] = F.u_out[node * d + i];
     v[i] = mid ? 0. : NA.v[node * d + i];
     acc[i] = mid ? 0. : NA.a[node * d + i];
@@ -2626,71 +2697,6 @@ __global__ void __launch_bounds__(256) k_step_fused_mixed(ElemArgs EA, NodeArgs 
   }
 }
 
-// Geometry records of the mixed fused step on triangles: per element,
-// x_a - x_0 for a > 0 formed in FP64 and rounded to FP32 (the arithmetic the
-// element kernels use on the fly), zero-padded to fused_geo_stride floats.
-template <int ET>
-__global__ void __launch_bounds__(256) k_fused_geometry(int64_t E, const double* __restrict__ X,
-                                                        const uint32_t* __restrict__ conn,
-                                                        float* __restrict__ geo) {
-  using T = Elem<ET>;
-  constexpr int d = T::d, n = T::n, G = fused_geo_stride(n, d);
-  const int64_t e = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (e >= E) return;
-  const int64_t n0 = conn[e];
-  float r[G];
-#pragma unroll
-  for (int k = 0; k < G; ++k) r[k] = 0.f;
-#pragma unroll
-  for (int a = 1; a < n; ++a) {
-    const int64_t na = conn[a * E + e];
-#pragma unroll
-    for (int i = 0; i < d; ++i) r[(a - 1) * d + i] = float(X[na * d + i] - X[n0 * d + i]);
-  }
-#pragma unroll
-  for (int k = 0; k < G; ++k) geo[e * G + k] = r[k];
-}
-
-// Per-evaluation records of the fused mixed step on triangles (FusedArgs::rec,
-// recx), one thread per evaluation j of the blocks' element lists.
-__global__ void __launch_bounds__(256) k_fused_records(int64_t J, int64_t E,
-                                                       const uint32_t* __restrict__ el,
-                                                       const uint32_t* __restrict__ conn,
-                                                       const float* __restrict__ geo,
-                                                       const uint16_t* __restrict__ lslot,
-                                                       const uint16_t* __restrict__ elem_mat,
-                                                       uint4* __restrict__ rec) {
-  const int64_t j = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (j >= J) return;
-  const int64_t e = el[j];
-  const float4 g = reinterpret_cast<const float4*>(geo)[e];
-  rec[j * 2] = make_uint4(__float_as_uint(g.x), __float_as_uint(g.y), __float_as_uint(g.z),
-                          __float_as_uint(g.w));
-  const uint32_t mat = elem_mat ? uint32_t(elem_mat[e]) : 0u;
-  rec[j * 2 + 1] = fused_record_ids(conn[e], conn[E + e], conn[2 * E + e], lslot[j * 3],
-                                    lslot[j * 3 + 1], lslot[j * 3 + 2], mat);
-}
-
-hipError_t launch_fused_records(hipStream_t s, int64_t J, int64_t E, const uint32_t* el,
-                                const uint32_t* conn_soa, const float* geo, const uint16_t* lslot,
-                                const uint16_t* elem_mat, uint4* rec) {
-  clear_error();
-  if (J == 0) return hipSuccess;
-  k_fused_records<<<unsigned((J + 255) / 256), 256, 0, s>>>(J, E, el, conn_soa, geo, lslot,
-                                                             elem_mat, rec);
-  return hipGetLastError();
-}
-
-hipError_t launch_fused_geometry(int et, hipStream_t s, int64_t E, const double* X,
-                                 const uint32_t* conn_soa, float* geo) {
-  clear_error();
-  if (E == 0) return hipSuccess;
-  const unsigned g = unsigned((E + 255) / 256);
-  if (et != TRI3) return hipErrorInvalidValue;
-  k_fused_geometry<TRI3><<<g, 256, 0, s>>>(E, X, conn_soa, geo);
-  return hipGetLastError();
-}
-
 template <int ET, int KIND>
 static hipError_t launch_fused_et(bool has_fext, hipStream_t s, const ElemArgs& EA,
                                   const NodeArgs& NA, const FusedArgs& F, int lds) {
@@ -2704,15 +2710,13 @@ template <int ET, int KIND>
 static hipError_t launch_fused_mixed_et(bool has_fext, hipStream_t s, const ElemArgs& EA,
                                         const NodeArgs& NA, const FusedArgs& F, int lds) {
   const unsigned g = unsigned(F.nblk);
-  if constexpr (ET == TRI3) {
-    if (F.rec) {
-      if (has_fext) k_step_fused_mixed<ET, KIND, true, true><<<g, 256, lds, s>>>(EA, NA, F);
-      else k_step_fused_mixed<ET, KIND, false, true><<<g, 256, lds, s>>>(EA, NA, F);
-      return hipGetLastError();
-    }
+  if (F.srec) {
+    if (has_fext) k_step_fused_mixed<ET, KIND, true, true><<<g, 256, lds, s>>>(EA, NA, F);
+    else k_step_fused_mixed<ET, KIND, false, true><<<g, 256, lds, s>>>(EA, NA, F);
+  } else {
+    if (has_fext) k_step_fused_mixed<ET, KIND, true, false><<<g, 256, lds, s>>>(EA, NA, F);
+    else k_step_fused_mixed<ET, KIND, false, false><<<g, 256, lds, s>>>(EA, NA, F);
   }
-  if (has_fext) k_step_fused_mixed<ET, KIND, true, false><<<g, 256, lds, s>>>(EA, NA, F);
-  else k_step_fused_mixed<ET, KIND, false, false><<<g, 256, lds, s>>>(EA, NA, F);
   return hipGetLastError();
 }
 

@@ -124,18 +124,22 @@ def fused_bytes(E, N, n, d, evaluations, nblk, node_block=256, chunk=256, staged
 
 
 def fused_mixed_bytes(E, N, n, d, evaluations, nblk, dt_per_node=False, node_block=256,
-                      chunk=256, records=True):
+                      chunk=256, records=True, staged=False):
     """Compulsory HBM bytes of one fused mixed step (slot layout 6 on the mixed
     path): as the FP64 one, but within a run the node update is the position
     form (the previous displacement read from the output buffer before it is
     overwritten; neither v nor a; dt^2 / M per node in place of the mass and
     the per-node time step), and triangles with
-    records (mixed_recompute 1) stream one 32-byte record per evaluation
+    records stream one 32-byte record per evaluation
     (coordinate differences, node ids, LDS slots, material) instead of the
-    element list, LDS slots, connectivity and coordinates."""
+    element list, LDS slots, connectivity and coordinates.  staged (what the
+    library runs): one 16-byte record per evaluation and the coordinates
+    once, as in the FP64 step."""
     chunks = evaluations / chunk + nblk
     tables = chunks * (node_block + 1) * 2 + (nblk + 1) * 8
-    if n == 3 and records:
+    if staged:
+        elements = evaluations * 16 + N * d * 8
+    elif n == 3 and records:
         elements = evaluations * 32
     else:
         elements = evaluations * (4 + 2 * n) + E * n * 4 + N * d * 8
@@ -389,7 +393,7 @@ def bench_cube(args, akx):
         (args.error_steps, rel_u, rel_e))
 
     def elem_kernel(patch, rc):
-        return ("void akx::k_element_patch<2, 0>(akx::ElemArgs)" if patch else
+        return ("void akx::k_element_patch<2, 0, 1>(akx::ElemArgs)" if patch else
                 "void akx::k_element_mixed<2, 0, %s>(akx::ElemArgs)" % ("true" if rc else "false"))
     kname, kbytes, kms, achieved, eb, nb, step_gbs = dominant(
         res, shapes, model, elem_kernel, "void akx::k_node<3, 1, false>(akx::NodeArgs)",
@@ -527,7 +531,7 @@ def bench_hex8(args, akx):
         log("CPU: %.3f s/step" % sec)
 
     def elem_kernel(patch, rc):
-        return ("void akx::k_element_patch<3, 1>(akx::ElemArgs)" if patch else
+        return ("void akx::k_element_patch<3, 1, 2>(akx::ElemArgs)" if patch else
                 "void akx::k_element_mixed<3, 1, %s>(akx::ElemArgs)" % ("true" if rc else "false"))
     kname, kbytes, kms, achieved, eb, nb, step_gbs = dominant(
         res, shapes, model, elem_kernel, "void akx::k_node<3, 1, false>(akx::NodeArgs)",
@@ -637,7 +641,7 @@ def bench_ensemble(args, akx):
         "median %.3e" % (err_amp.max(), np.median(err_amp), err_end.max(), np.median(err_end)))
 
     def elem_kernel(patch, rc):
-        return ("void akx::k_element_patch<0, 0>(akx::ElemArgs)" if patch else
+        return ("void akx::k_element_patch<0, 0, 1>(akx::ElemArgs)" if patch else
                 "void akx::k_element_mixed<0, 0, %s>(akx::ElemArgs)" % ("true" if rc else "false"))
     fused = model.query("fused_available") == 1
     nblk = model.query("fused_blocks")
@@ -647,12 +651,11 @@ def bench_ensemble(args, akx):
                                      staged=model.query("fused_staged_lds") > 0)
     if fused and shapes["mixed"]["slot_layout"] == 6:
         # one kernel per step: its roofline is the step's
-        records = (shapes["mixed"]["mixed_recompute"] == 1 and
-                   model.query("fused_records") == 1)
+        staged = model.query("fused_records") == 1
         kname = ("void akx::k_step_fused_mixed<0, 0, false, %s>"
-                 "(akx::ElemArgs, akx::NodeArgs, akx::FusedArgs)" % ("true" if records else "false"))
+                 "(akx::ElemArgs, akx::NodeArgs, akx::FusedArgs)" % ("true" if staged else "false"))
         kbytes = fused_mixed_bytes(E, N, n, d, model.query("fused_elements"), nblk,
-                                   dt_per_node=True, records=records)
+                                   dt_per_node=True, records=False, staged=staged)
         kms = res["mixed"]["element_ms"]
         achieved = kbytes / (kms * 1e-3) / 1e9
         eb, nb = kbytes, 0

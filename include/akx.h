@@ -242,11 +242,7 @@ int akx_last_step_timing(akx_ctx* ctx, double* element_ms, double* node_ms);
  * (patch-relative FP32 node values, partial sums), and so do the tables and
  * the rebuilt geometry (for hexahedron_8 rebuilt in the Walsh basis of the
  * trilinear shape functions, without B).  The mixed fused step (6) always
- * rebuilds B; on triangle_3 with mixed_recompute 1 from one 32-byte record
- * per element evaluation streamed in the blocks' order (coordinate
- * differences, node ids, LDS slots, material; meshes of up to 2^23 nodes
- * and 2^17 materials), with 0 from coordinates gathered through element ids:
- * the same result bit for bit. */
+ * rebuilds B: mixed_recompute does not matter to it. */
 int akx_set_launch(akx_ctx* ctx, int element_block, int node_block, int xcd_remap,
                    int mixed_recompute, int slot_layout, int node_stage);
 
@@ -258,7 +254,7 @@ int akx_set_launch(akx_ctx* ctx, int element_block, int node_block, int xcd_rema
  *   "fused_elements" (element evaluations of one fused step), "fused_blocks",
  *   "fused_staged_lds" (LDS bytes of a block of the fused FP64 step, 0: nodes
  *   not staged),
- *   "fused_records" (1/0: per-evaluation records of the mixed fused step),
+ *   "fused_records" (1/0: the fused steps read one record per evaluation),
  *   "element_block", "node_block", "xcd_remap", "mixed_recompute", "slot_layout". */
 int akx_query(akx_ctx* ctx, const char* key, double* value);
 

@@ -106,3 +106,34 @@ def test_layout_set_and_unset_capture_apart():
             p.gpu.solve_step_graph(n, akx.FP64)
             p.cpu.solve_step(n)
             assert np.array_equal(p.gpu.get_displacement(), p.cpu.nodal("u")), (layout, n)
+
+
+@pytest.mark.parametrize("name", ["tri_one", "tri_64", "tri_65", "tri_large", "quad", "tet",
+                                  "tet_large", "fan"])
+def test_mixed_step_staged_and_not(name):
+    """The mixed fused step with its nodes staged in LDS, on several materials,
+    and on a fan whose nodes no block holds.  Differences are formed in FP64
+    and rounded once (2^-24): 1e-5 covers the sums over an element; the fan's
+    triangles are 477 times as long as wide, and their area as much less exact."""
+    fan = name == "fan"
+    if fan:
+        t = np.linspace(0, 2 * np.pi, 3000, endpoint=False)
+        X = np.concatenate([[[0.0, 0.0]], np.stack([np.cos(t), np.sin(t)], axis=1)])
+        i = np.arange(3000)
+        m = akm.Mesh(akx.TRIANGLE_3, X, np.stack([0 * i, 1 + i, 1 + (i + 1) % 3000], axis=1))
+    else:
+        m = MESHES[name]()
+    mats = [STEEL, dict(E=70e9, nu=0.33, rho=2700.0), dict(E=3e9, nu=0.4, rho=1200.0)]
+    rng = np.random.default_rng(5)
+    p = gh.Pair(m, mats, rng.integers(0, 3, size=m.nb_elements))
+    p.set_nodal("displacement", 1e-5 * rng.normal(size=m.nodes.shape))
+    p.set_nodal("velocity", rng.normal(size=m.nodes.shape))
+    p.set_nodal("external_force", rng.normal(size=m.nodes.shape))
+    p.set_time_step(0.5 * p.cpu.stable_time_step())
+    p.gpu.set_launch(slot_layout=6)
+    assert p.gpu.query("fused_records") == (0 if fan else 1)
+    for n in (1, 3):
+        p.step(n, akx.MIXED)
+        for field, oname in (("displacement", "u"), ("velocity", "v"), ("internal_force", "f_int")):
+            assert gh.rel(p.gpu.get(field), p.cpu.nodal(oname)) <= 1e-5 * (477 if fan else 1), \
+                (field, n)
