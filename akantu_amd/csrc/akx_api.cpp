@@ -683,14 +683,23 @@ int build_fused(akx_ctx* c, const std::vector<uint32_t>& order, const std::vecto
         }
     }
     const size_t nodes = (size_t(n1 - n0) + others) * 2;
+    slots += 2;  // read behind the last run
     lds_mixed = (nodes * 8 + slots * 4) * size_t(d);
     return (nodes + slots) * size_t(d) * 8;
   };
-  // Small meshes take smaller blocks: a block's chunks follow one another, so
-  // that few large blocks leave most of the chip idle for the longest time
-  // (bar of 4,000 triangles: 7.1 us per step in 9 blocks of 256 nodes, 4.4 in
-  // 34 of 64).
-  const int64_t most = std::min<int64_t>(FUSED_NB, std::max<int64_t>(64, (N / 512 + 63) / 64 * 64));
+  // A mesh that does not fill the chip several times over is cut into as many
+  // blocks per CU as run on it at a time, and no more: a block's chunks follow
+  // one another, and one block more than a multiple of 256 costs a CU a whole
+  // further block.  Triangles run 8 at a time, tetrahedra 4.  Quadrangles take
+  // 2 while those hold their nodes (less than a chunk of elements per block
+  // leaves lanes idle), else 4.  FP64, us per step, against 512 blocks in
+  // multiples of 64 nodes: 97,000 triangles 5.5 -> 4.4, 320,000 9.0 -> 7.9,
+  // 720,000 15.5 -> 14.6; 216,000 tetrahedra 16.5 -> 13.7, 384,000 21.4 -> 19.2,
+  // 664,000 31.5 -> 28.2; 160,000 quadrangles 12.9 -> 10.5 (3 per CU 12.9);
+  // 90,000 in 515 blocks 8.3, in 472 7.4.
+  const int per_cu = n == 3 ? 8 : d == 3 || N > int64_t(512) * FUSED_NB ? 4 : 2;
+  const int64_t share = (N + 256 * per_cu - 1) / (256 * per_cu);
+  const int64_t most = std::min<int64_t>(FUSED_NB, std::max<int64_t>(64, (share + 7) / 8 * 8));
   bool staged = true;
   int64_t next = most;  // what the last block took and a little more
   for (int64_t n0 = 0; n0 < N;) {
@@ -777,7 +786,7 @@ int build_fused(akx_ctx* c, const std::vector<uint32_t>& order, const std::vecto
   c->fused_blocks = nblk;
   c->fused_elements = int64_t(el.size());
   // the mixed step: FP32 contributions, behind the nodes if they are staged
-  c->fused_lds = staged ? int(lds_max_mixed) : FUSED_CH * n * d * 4;
+  c->fused_lds = staged ? int(lds_max_mixed) : (FUSED_CH * n + 2) * d * 4;
   if (staged) {
     HIP_TRY(c, dalloc(&c->fhalo_off, halo_off.size()));
     HIP_TRY(c, dalloc(&c->fhalo, halo.size()));

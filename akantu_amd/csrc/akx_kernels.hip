@@ -2015,9 +2015,20 @@ __global__ void __launch_bounds__(256) k_step_fused(ElemArgs EA, NodeArgs NA, Fu
 #pragma unroll
           for (int i = 0; i < d; ++i) f[i] -= x[k * d + i];
       }
-      for (; q < q1; ++q)
+      if (q < q1) {
+        // one to three left, read together (behind the run: padding at the
+        // end) and past the run masked to +0, which leaves f as it is
+        double x[3 * d];
 #pragma unroll
-        for (int i = 0; i < d; ++i) f[i] -= s_f[q * d + i];
+        for (int k = 0; k < 3 * d; ++k) x[k] = s_f[q * d + k];
+#pragma unroll
+        for (int k = 0; k < 3; ++k)
+#pragma unroll
+          for (int i = 0; i < d; ++i) {
+            const int64_t keep = k == 0 || q + k < q1 ? -1 : 0;
+            f[i] -= __longlong_as_double(__double_as_longlong(x[k * d + i]) & keep);
+          }
+      }
     }
     __syncthreads();
   }
@@ -2537,7 +2548,7 @@ static hipError_t launch_node_d(int precision, bool has_fext, hipStream_t s, con
 // the same forces bit for bit.
 // Against gathering u through L2 (for triangles with 32-byte records that held
 // the coordinate differences): 4,000 triangles 5.3 -> 3.5 us per step, 1.6 M
-// 20.9 -> 20.5, 2.5 M in 128 specimens of a material each 30.5 -> 29.1;
+// 20.9 -> 20.2, 2.5 M in 128 specimens of a material each 30.5 -> 28.4;
 // 800,000 quadrangles 24.2 -> 23.1, 1.3 M tetrahedra 52 -> 35.  On 1.6 M
 // triangles the vector units are busy for about half of the time; LDS was for
 // 40 %, over half of that in bank conflicts, before u and X had an array each
@@ -2657,9 +2668,18 @@ __global__ void __launch_bounds__(256) k_step_fused_mixed(ElemArgs EA, NodeArgs 
 #pragma unroll
           for (int i = 0; i < d; ++i) f[i] += -1. * double(x[k * d + i]);
       }
-      for (; q < q1; ++q)
+      if (q < q1) {
+        float x[3 * d];
 #pragma unroll
-        for (int i = 0; i < d; ++i) f[i] += -1. * double(s_f[q * d + i]);
+        for (int k = 0; k < 3 * d; ++k) x[k] = s_f[q * d + k];
+#pragma unroll
+        for (int k = 0; k < 3; ++k)
+#pragma unroll
+          for (int i = 0; i < d; ++i) {
+            const uint32_t keep = k == 0 || q + k < q1 ? ~0u : 0u;
+            f[i] -= double(__uint_as_float(__float_as_uint(x[k * d + i]) & keep));
+          }
+      }
     }
     __syncthreads();
   }
