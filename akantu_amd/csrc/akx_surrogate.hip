@@ -550,13 +550,13 @@ __global__ void __launch_bounds__(256) k_sur_refresh(const float* __restrict__ P
 }
 
 // evaluation of the network on n points (scaled inputs, sx floats per point
-// -> outputs, sy floats per point); persistent blocks of 8 waves, the image
+// -> outputs, sy floats per point); persistent blocks of 8 or 12 waves, the image
 // staged in LDS once per block.  With 8 floats per point on both sides (the
 // explicit step's buffers) the points move as two 16-byte words and the 8th
 // input float, the strain pass's envelope flag, is copied to the 8th output
 // float, where the force pass reads it with the outputs.
 template <class F>
-__global__ void __launch_bounds__(512) k_sur_infer(const typename F::x8* __restrict__ img,
+__global__ void __launch_bounds__(768) k_sur_infer(const typename F::x8* __restrict__ img,
                                                    const float* __restrict__ imgb, int64_t n,
                                                    const float* __restrict__ X, int sx, float* Y,
                                                    int sy) {
@@ -878,16 +878,23 @@ hipError_t launch_sur_mlp(hipStream_t s, const void* img, const float* imgb, boo
                           int64_t n, const float* x, int sx, float* y, int sy) {
   (void)hipGetLastError();
   if (n <= 0) return hipSuccess;
-  // one block of 8 waves per CU (the weight image fills most of the LDS):
-  // two waves per SIMD, so one wave's activations overlap the other's MFMAs
+  // One block per CU (the weight image fills most of the LDS), so that one
+  // wave's activations overlap another's MFMAs: 8 waves, or 12 where they take
+  // less than three quarters as many rounds of a tile per wave (a round of 12
+  // takes about 4/3 of one of 8).  Step of a plate with the network, 8 / 12
+  // waves: 77,568 points 32.1 / 28.6 us (2 rounds, 1), 112,752 34.0 / 37.8 (2,
+  // 2), 160,320 42.9 / 40.7 (3, 2), 4.03 M 587 / 578 (62, 42), where 12 reach
+  // 1.04 PFLOP/s.
   const int64_t tiles = (n + 31) / 32;
-  const unsigned g = unsigned(std::min<int64_t>(256, (tiles + 7) / 8));
+  auto rounds = [&](int waves) { return (tiles + 256 * waves - 1) / (256 * waves); };
+  const int waves = rounds(12) * 4 < rounds(8) * 3 ? 12 : 8;
+  const unsigned g = unsigned(std::min<int64_t>(256, (tiles + waves - 1) / waves));
   if (bf16)
-    k_sur_infer<Bf16><<<g, 512, 0, s>>>(static_cast<const Bf16::x8*>(img), imgb, n, x, sx, y,
-                                        sy);
+    k_sur_infer<Bf16><<<g, 64 * waves, 0, s>>>(static_cast<const Bf16::x8*>(img), imgb, n, x, sx,
+                                               y, sy);
   else
-    k_sur_infer<Fp16><<<g, 512, 0, s>>>(static_cast<const Fp16::x8*>(img), imgb, n, x, sx, y,
-                                        sy);
+    k_sur_infer<Fp16><<<g, 64 * waves, 0, s>>>(static_cast<const Fp16::x8*>(img), imgb, n, x, sx,
+                                               y, sy);
   return hipGetLastError();
 }
 

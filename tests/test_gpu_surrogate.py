@@ -84,6 +84,22 @@ def test_bf16_inference_kernel_matches_reference():
     assert model.surrogate_format() == "fp16"
 
 
+@pytest.mark.parametrize("fmt", ["fp16", "bf16"])
+@pytest.mark.parametrize("n", [65536, 65537, 98304, 98305])
+def test_inference_at_the_edges_of_the_wave_count(n, fmt):
+    """Blocks of 8 waves or of 12, by the number of points: a point's outputs
+    do not depend on it (parts of 30,001 points take 8)."""
+    model = _plate_model()
+    rng = np.random.default_rng(n)
+    model.surrogate_format(fmt)
+    model.surrogate_params(rng.normal(size=model.surrogate_params().size).astype(np.float32) * 0.1)
+    x = rng.uniform(-1, 1, size=(n, 7)).astype(np.float32)
+    y = model.surrogate_infer(x)
+    parts = [model.surrogate_infer(x[a:a + 30001]) for a in range(0, n, 30001)]
+    assert np.isfinite(y).all() and np.abs(y).max() > 0
+    assert np.array_equal(y, np.concatenate(parts))
+
+
 def test_training_gradients_match_reference():
     """Forward + backward MFMA kernels (no update) against the CPU reference
     with the same BF16 rounding points, and the loss they report."""
