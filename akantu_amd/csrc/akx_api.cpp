@@ -801,12 +801,12 @@ int build_fused(akx_ctx* c, const std::vector<uint32_t>& order, const std::vecto
     }
     c->fused_staged_lds = int(lds_max);
     // Against slots on layout 0 (us per step, slots / fused): 4,000 triangles
-    // 8.9 / 4.4, 1.6 M 62 / 31; 6,000 tetrahedra 17 / 9.0, 1.3 M 128 / 51,
-    // neo-Hookean 131 / 86, with a shuffled numbering kept (4 evaluations per
-    // element) 267 / 124.  A quadrangle's four points are dear to repeat:
-    // 800,000 take 52 / 44 at 1.19 evaluations per element, a shuffled
-    // 240,000 45 / 56 at 4, hence the line between them at the ratio where
-    // the former would break even.
+    // 8.2 / 4.1, 1.6 M 61 / 28; 6,000 tetrahedra 17 / 8.5, 1.3 M 128 / 46,
+    // neo-Hookean 133 / 77, with a shuffled numbering kept (4 evaluations per
+    // element) 268 / 117.  A quadrangle's four points are dear to repeat:
+    // 800,000 take 53 / 38 at 1.19 evaluations per element, a shuffled
+    // 240,000 45 / 53 at 4, hence the line between them, below the ratio where
+    // the former would break even (1.6).
     c->fused_default = c->Q == 1 || double(el.size()) <= 1.4 * double(E);
   }
   c->fused_ok = true;

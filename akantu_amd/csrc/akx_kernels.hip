@@ -1875,9 +1875,10 @@ __global__ void __launch_bounds__(256) k_node(NodeArgs A) {
 //   instruction and set the step's time.
 //   Bound: FP64 instructions and LDS about equally.  Cube of 6 M tetrahedra,
 //   per step: 288 us gathering, 205 staged, 183 with the quotients by one
-//   divisor (Divisor; 170 in a graph), where two blocks more per CU matter as
-//   much as fewer repeated elements: 240 us with 54 KB of LDS a block (9.8 M
-//   evaluations), 183 with 40 KB (10.3 M), 199 with 32 KB (11.2 M).
+//   divisor (Divisor), where two blocks more per CU matter as much as fewer
+//   repeated elements: 240 us with 54 KB of LDS a block (9.8 M evaluations),
+//   183 with 40 KB (10.3 M), 199 with 32 KB (11.2 M).  165 with the halo's ids
+//   asked for first and the ends of the runs read together.
 // ===========================================================================
 // Place of pair i of (u, X) of staged node k in LDS.  In 2D u and X lie in an
 // array each, 16 bytes a node: one after the other, the nodes' u would use
