@@ -2147,6 +2147,20 @@ hipError_t temp_alloc(akx_ctx* c, TempBuf& b, size_t bytes) {
   return c->scratch.take(std::max<size_t>(bytes, 8), &b.p);
 }
 
+// `count` caller element ids as internal ids on the device, none included.
+int upload_element_ids(akx_ctx* c, const uint32_t* ids, int64_t count, const uint32_t** dev) {
+  std::vector<uint32_t> internal(static_cast<size_t>(count));
+  for (int64_t t = 0; t < count; ++t) {
+    if (int64_t(ids[t]) >= c->E) return fail(c, AKX_ERR_ARGUMENT, "element id out of range");
+    internal[size_t(t)] = c->elem_inv[ids[t]];
+  }
+  TempBuf b;
+  HIP_TRY(c, temp_alloc(c, b, internal.size() * 4));
+  HIP_TRY(c, c->copy.to_device(c->device, c->stream, b.p, internal.data(), internal.size() * 4));
+  *dev = b.get<uint32_t>();
+  return AKX_OK;
+}
+
 // The caller's element list (nullptr: every element, caller order) as
 // internal ids on the device (nullptr: 0 .. count - 1); returns the row count
 // through *count.
@@ -2159,17 +2173,8 @@ int fe_element_list(akx_ctx* c, const uint32_t* ids, int64_t nb, const uint32_t*
     *count = c->E;
     return AKX_OK;
   }
-  std::vector<uint32_t> internal(static_cast<size_t>(nb));
-  for (int64_t t = 0; t < nb; ++t) {
-    if (int64_t(ids[t]) >= c->E) return fail(c, AKX_ERR_ARGUMENT, "element id out of range");
-    internal[size_t(t)] = c->elem_inv[ids[t]];
-  }
-  TempBuf b;
-  HIP_TRY(c, temp_alloc(c, b, internal.size() * 4));
-  HIP_TRY(c, c->copy.to_device(c->device, c->stream, b.p, internal.data(), internal.size() * 4));
-  *dev = b.get<uint32_t>();
   *count = nb;
-  return AKX_OK;
+  return upload_element_ids(c, ids, nb, dev);
 }
 
 FeArgs fe_args(akx_ctx* c, const uint32_t* filt, int64_t count, int nb) {
@@ -2252,9 +2257,10 @@ int material_setup(akx_ctx* c, int mat, const uint32_t** filt, int64_t* cnt, Mat
   if (rc) return rc;
   if (mat < 0 || mat >= int(c->mats.size())) return fail(c, AKX_ERR_ARGUMENT, "no such material");
   (void)hipSetDevice(c->device);
+  // a material may have no elements: its list is empty, never "every element"
   const std::vector<uint32_t> ids = material_filter(c, mat);
-  if ((rc = fe_element_list(c, ids.data(), int64_t(ids.size()), filt, cnt)))
-    return rc;
+  *cnt = int64_t(ids.size());
+  if ((rc = upload_element_ids(c, ids.data(), *cnt, filt))) return rc;
   const size_t ne = size_t(c->E) * c->Q * c->d * c->d;
   if (!c->gradu) {
     HIP_TRY(c, dalloc(&c->gradu, ne));

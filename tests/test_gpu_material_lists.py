@@ -1,0 +1,48 @@
+"""The material operators (akx_material_*) on the rows that belong to a
+material, and no others."""
+import numpy as np
+import pytest
+
+from akantu_amd import akx
+from akantu_amd import mesh as akm
+
+pytestmark = pytest.mark.gpu
+
+MESHES = {"tri": lambda: akm.rectangle_tri3(5, 4, 1.0, 1.0), "hex": lambda: akm.cube_hex8(3)}
+
+
+def _model(mesh, kind, used):
+    """Elastic everywhere, and a second material that `used` elements have."""
+    g = akx.SolidMechanicsModel(mesh)
+    g.add_material(E=210e9, nu=0.3, rho=7800.0)
+    law = dict(kind=kind, E=1e7, nu=0.4, rho=1000.0)
+    if kind == akx.NEOHOOKEAN_DAMAGE:
+        law.update(Sd=1e5, Yd=np.full(mesh.nb_elements * mesh.nb_qp, 1e2))
+    g.add_material(**law)
+    g.assign_materials((np.arange(mesh.nb_elements) < used).astype(np.int32))
+    g.init_full()
+    u = 0.02 * np.random.default_rng(3).standard_normal(mesh.nodes.shape)
+    g.set("displacement", u)
+    return g
+
+
+@pytest.mark.parametrize("kind", [akx.ELASTIC, akx.NEOHOOKEAN, akx.NEOHOOKEAN_DAMAGE])
+@pytest.mark.parametrize("name", list(MESHES))
+def test_material_without_elements(name, kind):
+    """Every operator leaves the mesh alone and returns no rows, no energy."""
+    mesh = MESHES[name]()
+    g = _model(mesh, kind, 0)
+    assert len(g.material_elements(1)) == 0
+    assert g.material_potential_energy(1) == 0.0
+    assert g.material_potential_energy(0) > 0.0
+    damage = g.get("damage") if kind == akx.NEOHOOKEAN_DAMAGE else None
+    f = np.random.default_rng(4).standard_normal(mesh.nodes.shape)
+    g.set("internal_force", f)
+    rows = np.zeros((0, mesh.dim ** 2))
+    assert g.material_compute_stress(1, rows).shape == rows.shape
+    for out in g.material_compute_all_stresses(1):
+        assert out.shape == rows.shape
+    g.material_assemble_internal_forces(1)
+    assert np.array_equal(g.get("internal_force"), f)
+    if damage is not None:
+        assert np.array_equal(g.get("damage"), damage)
