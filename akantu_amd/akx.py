@@ -388,6 +388,10 @@ class SolidMechanicsModel:
         """Material::computeStress on the material's points from given gradients."""
         g = np.ascontiguousarray(grad_u, dtype=np.float64)
         out = np.empty_like(g)
+        n = ctypes.c_int64()
+        self.ctx.check(lib.akx_material_elements(self.ctx.h, int(mat_id), ctypes.byref(n), None))
+        # rows past the material's points are not written
+        out.reshape(-1)[n.value * self.mesh.nb_qp * self.dim ** 2:] = 0.0
         self.ctx.check(lib.akx_material_compute_stress(self.ctx.h, int(mat_id), _ptr(g),
                                                        _ptr(out)))
         return out
@@ -449,6 +453,7 @@ class SolidMechanicsModel:
     def surrogate_infer(self, x):
         x = np.ascontiguousarray(x, dtype=np.float32)
         y = np.empty_like(x)
+        y.reshape(-1)[7 * x.shape[0]:] = 0.0  # 7 values per point are written
         self.ctx.check(lib.akx_surrogate_infer(self.ctx.h, x.shape[0], _ptr(x), _ptr(y)))
         return y
 

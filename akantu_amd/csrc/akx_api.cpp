@@ -2391,9 +2391,11 @@ int akx_fe_assemble_field_lumped(akx_ctx* c, const double* field, int nb_dof, do
 int akx_material_elements(akx_ctx* c, int mat, int64_t* count, uint32_t* ids) {
   if (!c || !count) return AKX_ERR_ARGUMENT;
   if (mat < 0 || mat >= int(c->mats.size())) return fail(c, AKX_ERR_ARGUMENT, "no such material");
-  const std::vector<uint32_t> f = material_filter(c, mat);
-  *count = int64_t(f.size());
-  if (ids) std::copy(f.begin(), f.end(), ids);
+  *count = int64_t(std::count(c->elem_mat.begin(), c->elem_mat.end(), mat));
+  if (ids) {
+    const std::vector<uint32_t> f = material_filter(c, mat);
+    std::copy(f.begin(), f.end(), ids);
+  }
   return AKX_OK;
 }
 

@@ -1,5 +1,6 @@
 """The material operators (akx_material_*) on the rows that belong to a
-material, and no others."""
+material, and no others: a material that no element uses, and arrays longer
+than the material's rows."""
 import numpy as np
 import pytest
 
@@ -46,3 +47,31 @@ def test_material_without_elements(name, kind):
     assert np.array_equal(g.get("internal_force"), f)
     if damage is not None:
         assert np.array_equal(g.get("damage"), damage)
+
+
+@pytest.mark.parametrize("name", list(MESHES))
+def test_rows_past_the_material_are_zero(name, monkeypatch):
+    """A gradient array of every point handed to a material of three elements:
+    its points' stresses first, zeros behind them."""
+    monkeypatch.setattr(np, "empty_like", lambda a, *k, **kw: np.full_like(a, np.nan))
+    mesh = MESHES[name]()
+    g = _model(mesh, akx.ELASTIC, 3)
+    G = 1e-3 * np.random.default_rng(5).standard_normal((mesh.nb_elements * mesh.nb_qp,
+                                                          mesh.dim ** 2))
+    own = 3 * mesh.nb_qp
+    out = g.material_compute_stress(1, G)
+    assert np.array_equal(out[:own], g.material_compute_stress(1, G[:own]))
+    assert np.abs(out[:own]).min() > 0.0 and np.array_equal(out[own:], 0.0 * G[own:])
+
+
+def test_network_outputs_past_the_points_are_zero(monkeypatch):
+    """Seven outputs per point are written; the rest of a wider array is zero."""
+    monkeypatch.setattr(np, "empty_like", lambda a, *k, **kw: np.full_like(a, np.nan))
+    m = akm.box_tet4(1, 1, 1)
+    g = akx.SolidMechanicsModel(m)
+    g.add_material(kind=akx.NEOHOOKEAN_DAMAGE, E=1e9, nu=0.3, rho=1200.0, Sd=5e6,
+                   Yd=np.full(m.nb_elements, 1e6))
+    g.init_full()
+    g.surrogate_setup(0, 0.05)
+    y = g.surrogate_infer(np.zeros((5, 8), dtype=np.float32)).reshape(-1)
+    assert np.isfinite(y).all() and np.array_equal(y[35:], np.zeros(5, dtype=np.float32))
