@@ -285,14 +285,16 @@ void to_internal_points(const akx_ctx* c, const T* src, T* dst, int comp) {
     std::memcpy(dst + size_t(e) * per, src + size_t(c->elem_perm[e]) * per, per * sizeof(T));
 }
 
-// The slot layout a launch takes: the one set, else element-ordered slots on
-// the mixed path (another layout would round differently) and, on the FP64
-// path, where all layouts give the same bits, the fused step (fused_default)
-// or node-ordered slots: the node kernel streams them where it would gather
+// The slot layout a launch takes.  Mixed path: the one set or tuned last, else
+// element-ordered slots (another layout would round differently).  FP64 path,
+// where all layouts give the same bits: the one set or tuned for it -- tuning
+// the mixed path does not touch it --, else the fused step (fused_default) or
+// node-ordered slots: the node kernel streams them where it would gather
 // element-ordered ones (64,000 neo-Hookean hexahedra: 14.4 -> 10.1 us, 1 M
 // 126 -> 69; the element kernel's scattered stores cost 0 and 38 us of that).
 int layout_of(const akx_ctx* c, int precision) {
-  if (c->layout_set || precision == AKX_MIXED) return c->node_ordered;
+  if (precision == AKX_MIXED) return c->node_ordered;
+  if (c->fp64_layout >= 0) return c->fp64_layout;
   return c->fused_default ? 6 : 1;
 }
 
@@ -325,6 +327,16 @@ bool uses_partials(const akx_ctx* c, int precision) {
 // per-patch partials, FP32 otherwise
 int node_precision(const akx_ctx* c, int precision) {
   return uses_partials(c, precision) ? AKX_FP64 : precision;
+}
+
+// The layout a step runs with: layout_of, or what stands in for it where it
+// does not apply to the mesh, its laws or the precision.
+int running_layout(const akx_ctx* c, int precision) {
+  const int lay = layout_of(c, precision);
+  if (lay < 2 || uses_fused(c, precision)) return lay;
+  if (precision == AKX_FP64) return 1;
+  if (uses_partials(c, precision)) return lay == 6 ? 5 : lay;
+  return c->patch_ok && c->groups.size() == 1 && !c->groups[0].filter ? 2 : 1;
 }
 
 ElemArgs elem_args(akx_ctx* c, const KindGroup& g, int precision) {
@@ -1685,7 +1697,7 @@ int akx_solve_step_graph(akx_ctx* c, int nsteps, int precision) {
   akx_ctx::GraphKey k;
   k.nsteps = nsteps; k.precision = precision;
   k.eb = c->elem_block; k.nb = c->node_block; k.x = c->xcd_remap; k.rc = c->mixed_recompute;
-  k.lay = c->layout_set ? c->node_ordered : -1; k.stage = c->node_stage;
+  k.lay = layout_of(c, precision); k.stage = c->node_stage;
   k.fext = c->has_fext; k.bc = c->has_bc_inc; k.dt = c->dt;
   for (int i = 0; i < 3; ++i) k.bc_inc[i] = c->bc_inc[i];
   k.dt_node = c->dt_node;
@@ -1862,6 +1874,8 @@ int akx_query(akx_ctx* c, const char* key, double* value) {
   else if (k == "xcd_remap") *value = c->xcd_remap;
   else if (k == "mixed_recompute") *value = c->mixed_recompute;
   else if (k == "slot_layout") *value = c->node_ordered;
+  else if (k == "slot_layout_fp64") *value = running_layout(c, AKX_FP64);
+  else if (k == "slot_layout_mixed") *value = running_layout(c, AKX_MIXED);
   else if (k == "node_stage") *value = c->node_stage;
   else if (k == "surrogate_eps") *value = c->sur.eps;
   else if (k == "surrogate_stress_scale") *value = c->sur.sS;
@@ -2053,7 +2067,7 @@ int akx_autotune(akx_ctx* c, int precision, int nsteps, int* chosen, double* bes
   float best_t = std::numeric_limits<float>::max();
   const bool was_timing = c->timing;
   c->timing = false;
-  c->layout_set = true;  // each candidate names its layout, and so does the choice
+  const int keep_fp64 = c->fp64_layout;
   // candidates: slot layout x node staging x table/recompute x XCD mapping x block sizes
   struct Shape { int eb, nb, x, rcmp, lay, stage; };
   std::vector<Shape> cand;
@@ -2078,6 +2092,7 @@ int akx_autotune(akx_ctx* c, int precision, int nsteps, int* chosen, double* bes
   for (const Shape& sh : cand) {
           const int eb = sh.eb, nb = sh.nb, x = sh.x, lay = sh.lay;
           c->elem_block = eb; c->node_block = nb; c->xcd_remap = x; c->node_ordered = lay;
+          if (precision == AKX_FP64) c->fp64_layout = lay;
           c->node_stage = sh.stage;
           c->mixed_recompute = sh.rcmp;
           if ((rc = restore())) break;
@@ -2097,6 +2112,9 @@ int akx_autotune(akx_ctx* c, int precision, int nsteps, int* chosen, double* bes
   c->timing = was_timing;
   c->elem_block = best[0]; c->node_block = best[1]; c->xcd_remap = best[2];
   c->mixed_recompute = best[3]; c->node_ordered = best[4]; c->node_stage = best[5];
+  // the FP64 path's own layout: its tuner's choice, if a candidate ran
+  const bool tuned = best_t < std::numeric_limits<float>::max();
+  c->fp64_layout = precision == AKX_FP64 && tuned ? best[4] : keep_fp64;
   int rc2 = restore();
   (void)hipStreamSynchronize(c->stream);
   for (auto& s : saved) dfree(s.second);
@@ -2122,7 +2140,7 @@ int akx_set_launch(akx_ctx* c, int element_block, int node_block, int xcd_remap,
   if (mixed_recompute >= 0) c->mixed_recompute = mixed_recompute ? 1 : 0;
   if (slot_layout >= 0) {
     c->node_ordered = slot_layout;
-    c->layout_set = true;
+    c->fp64_layout = slot_layout;
   }
   if (node_stage >= 0) c->node_stage = node_stage ? 1 : 0;
   return AKX_OK;

@@ -362,8 +362,8 @@ struct akx_ctx {
 
   int elem_block = 256, node_block = 256, xcd_remap = 1, mixed_recompute = 1;
   int node_ordered = 0;             // slot layout (see store_slots)
-  // set by akx_set_launch or the autotuner (until then: layout_of)
-  bool layout_set = false;
+  // the FP64 path's, set by akx_set_launch or its autotuner (-1: layout_of)
+  int fp64_layout = -1;
   int node_stage = 1;               // node kernel copies its slot range to LDS when it fits
   uint32_t span_max[4] = {0, 0, 0, 0};  // largest slot range of a node block of 64, 128, 192, 256
   uint32_t* slot_pos = nullptr;     // [a][E] CSR position of (e, a)

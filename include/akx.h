@@ -233,11 +233,14 @@ int akx_last_step_timing(akx_ctx* ctx, double* element_ms, double* node_ms);
  * path), or no slots at all (6: one fused launch per step over node blocks
  * that recompute the elements around their nodes, on either path; stateless
  * laws of one kind on elements of up to 4 nodes -- elsewhere the FP64 path
- * runs 6 as node-ordered slots and the mixed path as 5; until a layout is set
- * or autotuned, the FP64 path takes 6 or 1, the faster one, and the mixed path
- * 0), and whether the node
- * kernel copies its block's contiguous slot range to LDS first (node_stage
- * 1/0) (-1 keeps).  On the FP64 path none of these changes a result bit; on
+ * runs 6 as node-ordered slots and the mixed path as 5; a layout set here
+ * holds for both paths; until one is set or autotuned in FP64 the FP64 path
+ * takes 6 or 1, the faster one, and until one is set or autotuned the mixed
+ * path takes 0), and whether the node kernel copies its block's contiguous
+ * slot range to LDS first (node_stage 1/0) (-1 keeps).  Hexahedra on the FP64
+ * path always rebuild B, in blocks of 256 threads: element_block and
+ * mixed_recompute do not matter to them.  On the FP64 path none of these
+ * changes a result bit; on
  * the mixed path layouts 0/1, 2, 3 and 4/5 differ in rounding only
  * (patch-relative FP32 node values, partial sums), and so do the tables and
  * the rebuilt geometry (for hexahedron_8 rebuilt in the Walsh basis of the
@@ -255,12 +258,16 @@ int akx_set_launch(akx_ctx* ctx, int element_block, int node_block, int xcd_rema
  *   "fused_staged_lds" (LDS bytes of a block of the fused FP64 step, 0: nodes
  *   not staged),
  *   "fused_records" (1/0: the fused steps read one record per evaluation),
- *   "element_block", "node_block", "xcd_remap", "mixed_recompute", "slot_layout". */
+ *   "element_block", "node_block", "xcd_remap", "mixed_recompute", "node_stage",
+ *   "slot_layout" (set or tuned last, 0 if none was; set again, it becomes the
+ *   layout of both paths), "slot_layout_fp64" and "slot_layout_mixed" (the
+ *   layouts that steps of either precision run with now). */
 int akx_query(akx_ctx* ctx, const char* key, double* value);
 
 /* Autotuner: times every launch shape (element and node block sizes, XCD
  * mapping, mixed-path table/recompute variant, slot layout) over `nsteps`
- * steps of the given precision on the current mesh and keeps the fastest.
+ * steps of the given precision on the current mesh and keeps the fastest (the
+ * slot layout of the FP64 path only when that precision is tuned).
  * The model state (u, v, a, damage, ...) is restored afterwards.  chosen
  * (optional, 6 ints) receives element_block, node_block, xcd_remap,
  * mixed_recompute, slot_layout, node_stage; best_ms (optional) the fastest
