@@ -165,6 +165,11 @@ class ScratchPool {
       if (b.p) (void)hipFree(b.p);
     bufs_.clear();
   }
+  size_t kept() const {  // bytes held now
+    size_t sum = 0;
+    for (const auto& b : bufs_) sum += b.cap;
+    return sum;
+  }
   class Use {
    public:
     explicit Use(ScratchPool& p) : pool_(p) { pool_.next_ = 0; }

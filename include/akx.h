@@ -258,6 +258,7 @@ int akx_set_launch(akx_ctx* ctx, int element_block, int node_block, int xcd_rema
  *   "fused_staged_lds" (LDS bytes of a block of the fused FP64 step, 0: nodes
  *   not staged),
  *   "fused_records" (1/0: the fused steps read one record per evaluation),
+ *   "scratch_bytes" (device memory kept for calls on host arrays),
  *   "element_block", "node_block", "xcd_remap", "mixed_recompute", "node_stage",
  *   "slot_layout" (set or tuned last, 0 if none was; set again, it becomes the
  *   layout of both paths), "slot_layout_fp64" and "slot_layout_mixed" (the

@@ -45,3 +45,37 @@ def test_network_outputs_do_not_depend_on_the_copy(n):
     y = model.surrogate_infer(x)
     parts = [model.surrogate_infer(x[k:k + 30000]) for k in range(0, n, 30000)]
     assert np.array_equal(y, np.concatenate(parts))
+
+
+def _plate(keep):
+    """476,701 nodes, 474,300 quadrangles of four points."""
+    m = akm.rectangle_quad4(697, 682, 1.0, 1.0)
+    model = akx.SolidMechanicsModel(m, keep_numbering=keep)
+    model.add_material(E=210e9, nu=0.3, rho=7800.0)
+    model.init_full()
+    return m, model
+
+
+def test_renumbered_copies_in_pieces():
+    """Fields of more than 32 MB go to and from the caller's numbering in
+    pieces: the same values as without renumbering, and no more than a piece of
+    device memory beside the field."""
+    rng = np.random.default_rng(6)
+    out = []
+    u = a = f = None
+    for keep in (True, False):
+        m, model = _plate(keep)
+        fe = model.get_fe_engine()
+        if u is None:
+            u = rng.normal(size=(m.nb_nodes, 2))
+            a = rng.normal(size=(m.nb_nodes, 9))         # 34 MB
+            f = rng.normal(size=(m.nb_elements * 4, 9))  # 137 MB
+        model.set("displacement", u)
+        stress = model.get("stress")                     # 61 MB
+        kept = model.query("scratch_bytes")
+        assert kept <= 32 << 20
+        out.append((stress, fe.interpolate_on_integration_points(a, 9),
+                    fe.assemble_field_lumped(f, a.copy())))
+        del model, fe
+    for x, y in zip(*out):
+        assert np.array_equal(x, y)
