@@ -154,8 +154,9 @@ class HostCopier {
 };
 
 // Device buffers that the operator calls of one context reuse, taken in order
-// by a call and returned at its end (the calls are synchronous).  Buffers
-// above KEEP are given back when the call ends.
+// by a call and returned at its end (the calls are synchronous).  KEEP bytes
+// at most stay allocated between calls: at the end of a call, buffers that
+// would take the sum above it are given back.
 class ScratchPool {
  public:
   static constexpr size_t KEEP = size_t(256) << 20;
@@ -174,10 +175,13 @@ class ScratchPool {
    public:
     explicit Use(ScratchPool& p) : pool_(p) { pool_.next_ = 0; }
     ~Use() {
+      size_t sum = 0;
       for (auto& b : pool_.bufs_)
-        if (b.cap > KEEP) {
+        if (b.cap > KEEP - sum) {
           (void)hipFree(b.p);
           b = Buf();
+        } else {
+          sum += b.cap;
         }
       pool_.next_ = 0;
     }

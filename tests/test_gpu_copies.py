@@ -79,3 +79,17 @@ def test_renumbered_copies_in_pieces():
         del model, fe
     for x, y in zip(*out):
         assert np.array_equal(x, y)
+
+
+def test_scratch_kept_between_calls_is_bounded():
+    """Operand and result of 130 MiB each: a context keeps 256 MiB in all."""
+    m, model = _plate(True)
+    fe = model.get_fe_engine()
+    D = np.random.default_rng(7).normal(size=(m.nb_elements * 4, 18))
+    first = fe.compute_btd(D)                       # 9 rows: 273 MB in, 546 MB out
+    assert model.query("scratch_bytes") <= 256 << 20
+    ones = np.ones((m.nb_elements * 4, 9))
+    assert fe.integrate(ones, 9)[:, 0].sum() == pytest.approx(1.0, rel=1e-9)
+    fe.integrate_on_integration_points(ones, 9)     # 137 MB in, 137 MB out
+    assert model.query("scratch_bytes") <= 256 << 20
+    assert np.array_equal(fe.compute_btd(D[:4 * 1000], np.arange(1000)), first[:4 * 1000])
