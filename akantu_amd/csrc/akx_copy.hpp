@@ -154,12 +154,13 @@ class HostCopier {
 };
 
 // Device buffers that the operator calls of one context reuse, taken in order
-// by a call and returned at its end (the calls are synchronous).  KEEP bytes
-// at most stay allocated between calls: at the end of a call, buffers that
-// would take the sum above it are given back.
+// by a call and returned at its end (the calls are synchronous).  Between calls
+// a buffer of up to KEEP bytes stays allocated while their sum is at most
+// KEEP_ALL, which holds the operand and the result of a call; the others are
+// given back (freeing and allocating 77 + 206 MB costs B^T D 0.95 ms of 11).
 class ScratchPool {
  public:
-  static constexpr size_t KEEP = size_t(256) << 20;
+  static constexpr size_t KEEP = size_t(256) << 20, KEEP_ALL = 2 * KEEP;
   ~ScratchPool() { release(); }
   void release() {
     for (auto& b : bufs_)
@@ -177,7 +178,7 @@ class ScratchPool {
     ~Use() {
       size_t sum = 0;
       for (auto& b : pool_.bufs_)
-        if (b.cap > KEEP - sum) {
+        if (b.cap > KEEP || b.cap > KEEP_ALL - sum) {
           (void)hipFree(b.p);
           b = Buf();
         } else {
