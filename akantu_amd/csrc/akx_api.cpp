@@ -843,10 +843,10 @@ int device_numbering(akx_ctx* c) {
 }
 
 // Scratch for rows of `row_bytes` that go to or from the caller's numbering in
-// pieces: at most ROWS_PIECE bytes (downloads of 48 MB in three pieces take 8 %
-// longer than in one of its size), and less where the card has not that much
-// left, so that a copy needs no room for the whole field.
-constexpr size_t ROWS_PIECE = size_t(32) << 20;
+// pieces: at most ROWS_PIECE bytes (35 MB in two pieces took 1.58 ms to the
+// host, in one 1.45), and less where the card has not that much left, so that a
+// copy needs no room for the whole field.
+constexpr size_t ROWS_PIECE = size_t(128) << 20;
 int take_rows(akx_ctx* c, int64_t rows, size_t row_bytes, void** raw, int64_t* piece) {
   int64_t m = std::min<int64_t>(rows, std::max<int64_t>(1, int64_t(ROWS_PIECE / row_bytes)));
   hipError_t e;
@@ -859,13 +859,33 @@ int take_rows(akx_ctx* c, int64_t rows, size_t row_bytes, void** raw, int64_t* p
   return AKX_OK;
 }
 
+// caller -> internal numbering of a context's rows (dev nullptr: equal)
+struct RowMap {
+  const uint32_t* dev;
+  const uint32_t* host;
+};
+RowMap node_rows(const akx_ctx* c) { return {c->node_inv_d, c->node_inv.data()}; }
+RowMap element_rows(const akx_ctx* c) { return {c->elem_inv_d, c->elem_inv.data()}; }
+
+// Up to HOST_ROWS bytes are renumbered on the host, beside a copy of 12 to 22
+// us, rather than by a launch (a nodal field to the host, host / device: 17 KB
+// 12 / 24 us, 115 KB 22 / 29, 217 KB 32.5 / 32.5; by the device array's size).
+constexpr size_t HOST_ROWS = size_t(128) << 10;
+
 // Rows of `width` doubles between a caller array in its own numbering and a
-// device array in the internal one (inv: caller -> internal, nullptr: equal).
-int upload_numbered(akx_ctx* c, int64_t rows, int width, const uint32_t* inv, const double* host,
+// device array in the internal one.
+int upload_numbered(akx_ctx* c, int64_t rows, int width, RowMap map, const double* host,
                     double* dev) {
-  const size_t row = size_t(width) * 8;
-  if (!inv || rows == 0) {
-    HIP_TRY(c, c->copy.to_device(c->device, c->stream, dev, host, size_t(rows) * row));
+  const size_t row = size_t(width) * 8, bytes = size_t(rows) * row;
+  if (!map.dev || rows == 0) {
+    HIP_TRY(c, c->copy.to_device(c->device, c->stream, dev, host, bytes));
+    return AKX_OK;
+  }
+  if (bytes <= HOST_ROWS) {
+    std::vector<double> t(size_t(rows) * width);
+    for (int64_t r = 0; r < rows; ++r)
+      std::memcpy(&t[size_t(map.host[r]) * width], host + r * width, row);
+    HIP_TRY(c, c->copy.to_device(c->device, c->stream, dev, t.data(), bytes));
     return AKX_OK;
   }
   void* raw = nullptr;
@@ -874,16 +894,26 @@ int upload_numbered(akx_ctx* c, int64_t rows, int width, const uint32_t* inv, co
   for (int64_t r = 0; r < rows; r += piece) {
     const int64_t m = std::min(piece, rows - r);
     HIP_TRY(c, c->copy.to_device(c->device, c->stream, raw, host + r * width, size_t(m) * row));
-    HIP_TRY(c, launch_scatter_rows(c->stream, m, width, inv + r, static_cast<double*>(raw), dev));
+    HIP_TRY(c, launch_scatter_rows(c->stream, m, width, map.dev + r, static_cast<double*>(raw),
+                                   dev));
   }
   return AKX_OK;
 }
 // dw values per row out of rows of sw (sw 1: repeated)
-int download_numbered(akx_ctx* c, int64_t rows, int dw, int sw, const uint32_t* inv,
-                      const double* dev, double* host) {
-  const size_t row = size_t(dw) * 8;
-  if ((!inv && dw == sw) || rows == 0) {
-    HIP_TRY(c, c->copy.to_host(c->device, c->stream, host, dev, size_t(rows) * row));
+int download_numbered(akx_ctx* c, int64_t rows, int dw, int sw, RowMap map, const double* dev,
+                      double* host) {
+  const size_t row = size_t(dw) * 8, bytes = size_t(rows) * row;
+  if ((!map.dev && dw == sw) || rows == 0) {
+    HIP_TRY(c, c->copy.to_host(c->device, c->stream, host, dev, bytes));
+    return AKX_OK;
+  }
+  if (size_t(rows) * sw * 8 <= HOST_ROWS) {
+    std::vector<double> t(size_t(rows) * sw);
+    HIP_TRY(c, c->copy.to_host(c->device, c->stream, t.data(), dev, t.size() * 8));
+    for (int64_t r = 0; r < rows; ++r) {
+      const double* from = &t[size_t(map.dev ? map.host[r] : r) * sw];
+      for (int i = 0; i < dw; ++i) host[r * dw + i] = from[sw == 1 ? 0 : i];
+    }
     return AKX_OK;
   }
   void* raw = nullptr;
@@ -891,8 +921,8 @@ int download_numbered(akx_ctx* c, int64_t rows, int dw, int sw, const uint32_t* 
   if (int rc = take_rows(c, rows, row, &raw, &piece)) return rc;
   for (int64_t r = 0; r < rows; r += piece) {
     const int64_t m = std::min(piece, rows - r);
-    HIP_TRY(c, launch_snapshot(c->stream, m, dw, sw, inv ? inv + r : nullptr,
-                               inv ? dev : dev + r * sw, raw, 8));
+    HIP_TRY(c, launch_snapshot(c->stream, m, dw, sw, map.dev ? map.dev + r : nullptr,
+                               map.dev ? dev : dev + r * sw, raw, 8));
     HIP_TRY(c, c->copy.to_host(c->device, c->stream, host + r * dw, raw, size_t(m) * row));
   }
   return AKX_OK;
@@ -901,8 +931,7 @@ int download_numbered(akx_ctx* c, int64_t rows, int dw, int sw, const uint32_t* 
 int read_blocked(akx_ctx* c, std::vector<uint8_t>& internal) {
   const size_t nd = size_t(c->N) * c->d;
   internal.resize(nd);
-  HIP_TRY(c, hipMemcpyAsync(internal.data(), c->blocked, nd, hipMemcpyDeviceToHost, c->stream));
-  HIP_TRY(c, hipStreamSynchronize(c->stream));
+  HIP_TRY(c, c->copy.to_host(c->device, c->stream, internal.data(), c->blocked, nd));
   return AKX_OK;
 }
 
@@ -1320,7 +1349,8 @@ int akx_field_upload(akx_ctx* c, int field, const void* host, size_t bytes) {
     to_internal_nodal(c, static_cast<const uint8_t*>(host), h.data());
     // bit0: blocked; bit1 (per-step Dirichlet increment) survives on DOFs that stay blocked
     for (size_t k = 0; k < nd; ++k) cur[k] = uint8_t(h[k] ? (1 | (cur[k] & 2)) : 0);
-    HIP_TRY(c, hipMemcpy(c->blocked, cur.data(), nd, hipMemcpyHostToDevice));
+    HIP_TRY(c, c->copy.to_device(c->device, c->stream, c->blocked, cur.data(), nd));
+    HIP_TRY(c, hipStreamSynchronize(c->stream));
     return AKX_OK;
   }
   if (field == AKX_DAMAGE) {
@@ -1328,7 +1358,7 @@ int akx_field_upload(akx_ctx* c, int field, const void* host, size_t bytes) {
     if (bytes != size_t(c->E) * c->Q * 8) return fail(c, AKX_ERR_ARGUMENT, "damage: size mismatch");
     if (int rc = device_numbering(c)) return rc;
     ScratchPool::Use use(c->scratch);
-    if (int rc = upload_numbered(c, c->E, c->Q, c->elem_inv_d, static_cast<const double*>(host),
+    if (int rc = upload_numbered(c, c->E, c->Q, element_rows(c), static_cast<const double*>(host),
                                  c->damage))
       return rc;
     HIP_TRY(c, hipStreamSynchronize(c->stream));
@@ -1343,7 +1373,7 @@ int akx_field_upload(akx_ctx* c, int field, const void* host, size_t bytes) {
   if (int rc = device_numbering(c)) return rc;
   const double* h = static_cast<const double*>(host);
   ScratchPool::Use use(c->scratch);
-  if (int rc = upload_numbered(c, c->N, c->d, c->node_inv_d, h, p)) return rc;
+  if (int rc = upload_numbered(c, c->N, c->d, node_rows(c), h, p)) return rc;
   if (field == AKX_EXTERNAL_FORCE) {
     c->has_fext = false;
     for (size_t k = 0; k < nd && !c->has_fext; ++k) c->has_fext = (h[k] != 0.);
@@ -1371,7 +1401,7 @@ int akx_field_download(akx_ctx* c, int field, void* host, size_t bytes) {
   if (bytes != ne * 8) return fail(c, AKX_ERR_ARGUMENT, "size mismatch");
   double* h = static_cast<double*>(host);
   if (int rc = device_numbering(c)) return rc;
-  const uint32_t *ninv = c->node_inv_d, *einv = c->elem_inv_d;
+  const RowMap ninv = node_rows(c), einv = element_rows(c);
   ScratchPool::Use use(c->scratch);
   if (field == AKX_MASS) {
     if (!c->initialized) return fail(c, AKX_ERR_STATE, "akx_init has not been called");
@@ -2242,7 +2272,7 @@ FeArgs fe_args(akx_ctx* c, const uint32_t* filt, int64_t count, int nb) {
 int upload_nodal(akx_ctx* c, const double* host, int nb, TempBuf& dev) {
   if (int rc = device_numbering(c)) return rc;
   HIP_TRY(c, temp_alloc(c, dev, size_t(c->N) * nb * 8));
-  return upload_numbered(c, c->N, nb, c->node_inv_d, host, dev.get<double>());
+  return upload_numbered(c, c->N, nb, node_rows(c), host, dev.get<double>());
 }
 
 int upload_rows(akx_ctx* c, const double* host, size_t n, TempBuf& dev) {
@@ -2421,7 +2451,7 @@ int akx_fe_assemble_field_lumped(akx_ctx* c, const double* field, int nb_dof, do
   ScratchPool::Use use(c->scratch);
   TempBuf din, integ, dl;
   HIP_TRY(c, temp_alloc(c, din, size_t(E) * Q * nb_dof * 8));
-  if ((rc = upload_numbered(c, E, Q * nb_dof, c->elem_inv_d, field, din.get<double>()))) return rc;
+  if ((rc = upload_numbered(c, E, Q * nb_dof, element_rows(c), field, din.get<double>()))) return rc;
   if ((rc = upload_nodal(c, lumped, nb_dof, dl))) return rc;
   HIP_TRY(c, temp_alloc(c, integ, size_t(E) * n * nb_dof * 8));
   FeArgs A = fe_args(c, nullptr, E, nb_dof);
@@ -2430,7 +2460,7 @@ int akx_fe_assemble_field_lumped(akx_ctx* c, const double* field, int nb_dof, do
   HIP_TRY(c, launch_fe(FE_LUMPED_ELEMENTS, c->et, c->stream, A));
   HIP_TRY(c, launch_fe_lumped_nodes(c->stream, N, nb_dof, n, c->mass_off, c->mass_slot,
                                     integ.get<double>(), dl.get<double>()));
-  return download_numbered(c, N, nb_dof, nb_dof, c->node_inv_d, dl.get<double>(), lumped);
+  return download_numbered(c, N, nb_dof, nb_dof, node_rows(c), dl.get<double>(), lumped);
 }
 
 int akx_material_elements(akx_ctx* c, int mat, int64_t* count, uint32_t* ids) {

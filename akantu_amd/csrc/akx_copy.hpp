@@ -1,13 +1,17 @@
 // akx_copy.hpp -- copies between a caller's pageable host arrays and the
 // device for the calls that return or take host data.
 //
-// The runtime's own pageable copies reach 18 GB/s to the host and 30 GB/s to
-// the device on a card whose link carries 57: it stages or pins them on the
-// calling thread, in turn with the transfer, and a caller's fresh array is
-// mapped page by page on the way.  Here the data pass through small
-// page-locked slots, two per helper thread: a slot travels while the other is
-// copied, and large copies use several threads, since one thread alone fills
-// fresh pages at 13 GB/s (41 MB into a fresh array: 4.2 ms by hipMemcpy).
+// To the host, the runtime's own pageable copies reach 18 GB/s on a card whose
+// link carries 57: it stages or pins the pages on the calling thread, in turn
+// with the transfer, and a caller's fresh array is mapped page by page on the
+// way.  Here the data pass through small page-locked slots, two per helper
+// thread: a slot travels while the other is copied, and large copies use
+// several threads, since one thread alone fills fresh pages at 13 GB/s (41 MB
+// into a fresh array: 4.2 ms by hipMemcpy).  To the device the runtime's copy
+// is the faster one between 1 and 24 MB (16 MB: 0.47 ms, 0.61 through slots);
+// below, one slot spares the pinning of the caller's pages (256 KB: 26 us, 28
+// to 130), and above, the threads gain (B^T D with an operand of 18 MB 2.37 ms
+// by the runtime's copy, 2.46 by slots; 35 MB 4.84 and 4.71).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -27,37 +31,62 @@ class HostCopier {
   void release() {
     for (auto& lane : lanes_)
       for (auto& s : lane) {
-        if (s.done) (void)hipEventSynchronize(s.done);
+        (void)idle(s);
         if (s.done) (void)hipEventDestroy(s.done);
         if (s.mem) (void)hipHostFree(s.mem);
         s = Slot();
       }
   }
 
-  // Copies that are complete when the call returns (to_host: after the work
-  // queued on the stream).  to_device returns when the host array has been
-  // read; the device copy is ordered before later work on the stream.
+  // Copies that are complete when the call returns, after the work queued on
+  // the stream.
   hipError_t to_host(int device, hipStream_t s, void* host, const void* dev, size_t bytes) {
-    return run(device, bytes, [=](int lane, int lanes, size_t chunks) -> hipError_t {
-      return fetch(lane, lanes, chunks, s, static_cast<char*>(host),
-                   static_cast<const char*>(dev), bytes);
-    });
+    if (bytes == 0) return hipSuccess;
+    if (bytes > SLOT)
+      return run(device, bytes, [=](int lane, int lanes, size_t chunks) -> hipError_t {
+        return fetch(lane, lanes, chunks, s, static_cast<char*>(host),
+                     static_cast<const char*>(dev), bytes);
+      });
+    // one slot: the stream is waited for, which is 7 us less than an event
+    Slot& slot = lanes_[0][0];
+    hipError_t e = fillable(slot, s);
+    if (e == hipSuccess) e = hipMemcpyAsync(slot.mem, dev, bytes, hipMemcpyDeviceToHost, s);
+    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    if (e != hipSuccess) return e;
+    std::memcpy(host, slot.mem, bytes);
+    for (auto& up : lanes_[0])
+      if (up.upload == s) up.upload = nullptr;
+    return hipSuccess;
   }
+  // Returns when the host array has been read; the device copy is ordered
+  // before later work on the stream.
   hipError_t to_device(int device, hipStream_t s, void* dev, const void* host, size_t bytes) {
-    return run(device, bytes, [=](int lane, int lanes, size_t chunks) -> hipError_t {
-      return send(lane, lanes, chunks, s, static_cast<char*>(dev),
-                  static_cast<const char*>(host), bytes);
-    });
+    if (bytes == 0) return hipSuccess;
+    if (bytes > LARGE_UPLOAD)
+      return run(device, bytes, [=](int lane, int lanes, size_t chunks) -> hipError_t {
+        return send(lane, lanes, chunks, s, static_cast<char*>(dev),
+                    static_cast<const char*>(host), bytes);
+      });
+    if (bytes > SLOT) {
+      const hipError_t e = hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, s);
+      return e == hipSuccess ? hipStreamSynchronize(s) : e;
+    }
+    // an event costs 5 us, as much as the transfer of a small array
+    return send_slot(lanes_[0][turn_ ^= 1], s, dev, host, bytes, bytes > SMALL);
   }
 
  private:
   static constexpr size_t SLOT = size_t(1) << 20;
+  static constexpr size_t SMALL = size_t(128) << 10;
+  static constexpr size_t LARGE_UPLOAD = size_t(24) << 20;
   static constexpr int LANES = 4;
   struct Slot {
     void* mem = nullptr;
-    hipEvent_t done = nullptr;  // the slot's last transfer
+    hipEvent_t done = nullptr;     // the last transfer of a longer copy
+    hipStream_t upload = nullptr;  // a small upload may be reading the slot
   };
   Slot lanes_[LANES][2];
+  int turn_ = 0;  // slot of the next upload
 
   // One lane up to 8 MB: inference of 200,003 points (5.6 MB each way) takes
   // 0.66 ms with one or two, and starting threads costs a first call 0.4 ms.
@@ -65,34 +94,48 @@ class HostCopier {
   // 41 MB) take 5.9 ms with one lane, 4.7 with two, 3.8 with four or eight.
   static int lanes_for(size_t bytes) { return bytes <= (size_t(8) << 20) ? 1 : LANES; }
 
-  static hipError_t ready(Slot& s) {
-    if (!s.mem) {
-      hipError_t e = hipHostMalloc(&s.mem, SLOT, hipHostMallocDefault);
-      if (e != hipSuccess) {
-        s.mem = nullptr;
-        return e;
-      }
-    }
-    if (!s.done) {
-      hipError_t e = hipEventCreateWithFlags(&s.done, hipEventDisableTiming);
-      if (e != hipSuccess) {
-        s.done = nullptr;
-        return e;
-      }
-      return hipSuccess;
-    }
-    return hipEventSynchronize(s.done);
+  // waits until nothing reads or fills the slot
+  static hipError_t idle(Slot& s) {
+    hipError_t e = hipSuccess;
+    if (s.upload) e = hipStreamSynchronize(s.upload);
+    s.upload = nullptr;
+    if (s.done && e == hipSuccess) e = hipEventSynchronize(s.done);
+    return e;
+  }
+  static hipError_t allocated(Slot& s) {
+    if (s.mem) return hipSuccess;
+    const hipError_t e = hipHostMalloc(&s.mem, SLOT, hipHostMallocDefault);
+    if (e != hipSuccess) s.mem = nullptr;
+    return e;
+  }
+  static hipError_t with_event(Slot& s) {
+    if (s.done) return hipSuccess;
+    const hipError_t e = hipEventCreateWithFlags(&s.done, hipEventDisableTiming);
+    if (e != hipSuccess) s.done = nullptr;
+    return e;
+  }
+  // the slot takes a transfer on stream s, which follows an upload on s
+  static hipError_t fillable(Slot& slot, hipStream_t s) {
+    if (slot.upload && slot.upload != s)
+      if (hipError_t e = idle(slot)) return e;
+    return allocated(slot);
   }
 
   template <typename F>
   hipError_t run(int device, size_t bytes, F&& lane_copy) {
-    if (bytes == 0) return hipSuccess;
     const size_t chunks = (bytes + SLOT - 1) / SLOT;
     const int lanes = lanes_for(bytes);
     std::atomic<int> first{int(hipSuccess)};
     auto work = [&](int lane) {
-      if (lane > 0) (void)hipSetDevice(device);
-      const hipError_t e = lane_copy(lane, lanes, chunks);
+      hipError_t e = hipSuccess;
+      // uploads of the same call first: queued behind them and the kernels that
+      // read them, the transfers start up to 30 us late (gradient of 8,000
+      // hexahedra, 4.4 MB: 219 us, 243 without the wait)
+      if (lane == 0)
+        for (auto& up : lanes_[0]) e = e == hipSuccess ? idle(up) : e;
+      else
+        (void)hipSetDevice(device);
+      if (e == hipSuccess) e = lane_copy(lane, lanes, chunks);
       if (e != hipSuccess) {
         int none = int(hipSuccess);
         first.compare_exchange_strong(none, int(e));
@@ -116,7 +159,8 @@ class HostCopier {
                    const char* dev, size_t bytes) {
     auto size = [&](size_t k) { return k + 1 < chunks ? SLOT : bytes - k * SLOT; };
     auto start = [&](size_t k, Slot& slot) -> hipError_t {
-      hipError_t e = ready(slot);
+      hipError_t e = fillable(slot, s);
+      if (e == hipSuccess) e = with_event(slot);
       if (e == hipSuccess)
         e = hipMemcpyAsync(slot.mem, dev + k * SLOT, size(k), hipMemcpyDeviceToHost, s);
       return e == hipSuccess ? hipEventRecord(slot.done, s) : e;
@@ -137,17 +181,26 @@ class HostCopier {
     return hipSuccess;
   }
 
+  // from the host array through a slot; without an event the stream tells
+  static hipError_t send_slot(Slot& slot, hipStream_t s, void* dev, const void* host,
+                              size_t bytes, bool event) {
+    hipError_t e = idle(slot);
+    if (e == hipSuccess) e = allocated(slot);
+    if (e == hipSuccess && event) e = with_event(slot);
+    if (e != hipSuccess) return e;
+    std::memcpy(slot.mem, host, bytes);
+    if ((e = hipMemcpyAsync(dev, slot.mem, bytes, hipMemcpyHostToDevice, s))) return e;
+    slot.upload = s;
+    if (event && (e = hipEventRecord(slot.done, s)) == hipSuccess) slot.upload = nullptr;
+    return e;
+  }
   hipError_t send(int lane, int lanes, size_t chunks, hipStream_t s, char* dev, const char* host,
                   size_t bytes) {
     int j = 0;
     for (size_t k = size_t(lane); k < chunks; k += size_t(lanes), j ^= 1) {
-      Slot& slot = lanes_[lane][j];
       const size_t n = k + 1 < chunks ? SLOT : bytes - k * SLOT;
-      hipError_t e = ready(slot);
-      if (e != hipSuccess) return e;
-      std::memcpy(slot.mem, host + k * SLOT, n);
-      if ((e = hipMemcpyAsync(dev + k * SLOT, slot.mem, n, hipMemcpyHostToDevice, s))) return e;
-      if ((e = hipEventRecord(slot.done, s))) return e;
+      if (hipError_t e = send_slot(lanes_[lane][j], s, dev + k * SLOT, host + k * SLOT, n, true))
+        return e;
     }
     return hipSuccess;
   }

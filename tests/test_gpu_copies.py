@@ -57,7 +57,7 @@ def _plate(keep):
 
 
 def test_renumbered_copies_in_pieces():
-    """Fields of more than 32 MB go to and from the caller's numbering in
+    """Fields of more than 128 MiB go to and from the caller's numbering in
     pieces: the same values as without renumbering, and no more than a piece of
     device memory beside the field."""
     rng = np.random.default_rng(6)
@@ -68,14 +68,13 @@ def test_renumbered_copies_in_pieces():
         fe = model.get_fe_engine()
         if u is None:
             u = rng.normal(size=(m.nb_nodes, 2))
-            a = rng.normal(size=(m.nb_nodes, 4))         # 34 MB
+            a = rng.normal(size=(m.nb_nodes, 2))
             f = rng.normal(size=(m.nb_elements * 4, 4))  # 137 MB
         model.set("displacement", u)
         stress = model.get("stress")                     # 137 MB
-        kept = model.query("scratch_bytes")
-        assert kept <= 32 << 20
-        out.append((stress, fe.interpolate_on_integration_points(a, 4),
-                    fe.assemble_field_lumped(f, a.copy())))
+        assert model.query("scratch_bytes") <= 128 << 20
+        out.append((stress, fe.interpolate_on_integration_points(a, 2),
+                    fe.assemble_field_lumped(f, np.tile(a, 2))))
         del model, fe
     for x, y in zip(*out):
         assert np.array_equal(x, y)
@@ -97,3 +96,35 @@ def test_scratch_kept_between_calls_is_bounded():
     first = fe.compute_btd(g)                       # 274 MB of results
     assert model.query("scratch_bytes") <= 512 << 20
     assert np.array_equal(fe.compute_btd(g[:4000], np.arange(1000)), first[:4000])
+
+
+@pytest.mark.parametrize("kb", [1, 17, 126, 131, 520, 1020, 1030, 2600])
+@pytest.mark.parametrize("keep", [False, True])
+def test_successive_copies_share_the_slots(kb, keep):
+    """Operands and results around the sizes where the copies change (128 KiB:
+    host renumbering and uploads without an event, 1 MiB: one slot), several in
+    a row without a wait of the caller's own."""
+    n = max(2, int(round((kb * 1024 / 16) ** 0.5)))
+    m = akm.rectangle_quad4(n - 1, n - 1, 1.0, 1.0)
+    model = akx.SolidMechanicsModel(m, keep_numbering=keep)
+    model.add_material(E=210e9, nu=0.3, rho=7800.0)
+    model.init_full()
+    fe = model.get_fe_engine()
+    rng = np.random.default_rng(n)
+    u, v = rng.normal(size=(2, m.nb_nodes, 2))
+    blocked = rng.random(m.nodes.shape) < 0.3
+    for k in range(3):
+        model.set("displacement", u + k)
+        model.set("velocity", v - k)
+        model.set("blocked_dofs", np.roll(blocked, k))
+        ids = rng.permutation(m.nb_elements).astype(np.uint32)
+        g = fe.gradient_on_integration_points(u + k, 2, ids)
+        assert np.array_equal(model.get("displacement"), u + k)
+        assert np.array_equal(model.get("velocity"), v - k)
+        assert np.array_equal(model.get("current_position"), m.nodes + (u + k))
+        assert np.array_equal(model.get("blocked_dofs"), np.roll(blocked, k))
+        whole = fe.gradient_on_integration_points(u + k, 2)
+        rows = (ids[:, None].astype(np.int64) * 4 + np.arange(4)).reshape(-1)
+        assert np.array_equal(g, whole[rows])
+        mass = model.get("mass")
+        assert np.array_equal(mass[:, 0], mass[:, 1]) and mass.min() > 0
