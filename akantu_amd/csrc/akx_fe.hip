@@ -78,28 +78,29 @@ __global__ void __launch_bounds__(256) k_fe_gradient(FeArgs A) {
   constexpr int d = T::d, n = T::n, Q = T::Q;
   __shared__ PointTables s_p;
   stage_points<ET>(s_p, A.tab64);
-  const int64_t r = int64_t(blockIdx.x) * 256 + threadIdx.x;
-  if (r >= A.count * Q) return;
-  const int64_t t = r / Q;
-  const int64_t e = elem_of(A, t);
-  const int nb = A.nb;
-  double B[d * n];
-  point_b<ET>(A, s_p.dnds[r - t * Q], e, B);
-  int64_t node[n];
+  const int64_t end = A.count * Q;
+  for (int64_t r = int64_t(blockIdx.x) * 256 + threadIdx.x; r < end; r += int64_t(gridDim.x) * 256) {
+    const int64_t t = r / Q;
+    const int64_t e = elem_of(A, t);
+    const int nb = A.nb;
+    double B[d * n];
+    point_b<ET>(A, s_p.dnds[r - t * Q], e, B);
+    int64_t node[n];
 #pragma unroll
-  for (int a = 0; a < n; ++a) node[a] = A.conn[a * A.E + e];
-  // nabla_u (nb x d) = u_e (nb x n) * B^T, B (d x n)
-  double* o = A.out + r * nb * d;
-  for (int i = 0; i < nb; ++i) {
-    double u[n];
+    for (int a = 0; a < n; ++a) node[a] = A.conn[a * A.E + e];
+    // nabla_u (nb x d) = u_e (nb x n) * B^T, B (d x n)
+    double* o = A.out + r * nb * d;
+    for (int i = 0; i < nb; ++i) {
+      double u[n];
 #pragma unroll
-    for (int a = 0; a < n; ++a) u[a] = A.in[node[a] * nb + i];
+      for (int a = 0; a < n; ++a) u[a] = A.in[node[a] * nb + i];
 #pragma unroll
-    for (int j = 0; j < d; ++j) {
-      double s = 0.;
+      for (int j = 0; j < d; ++j) {
+        double s = 0.;
 #pragma unroll
-      for (int l = 0; l < n; ++l) s += u[l] * B[j + l * d];
-      o[i + j * nb] = s;
+        for (int l = 0; l < n; ++l) s += u[l] * B[j + l * d];
+        o[i + j * nb] = s;
+      }
     }
   }
 }
@@ -133,39 +134,40 @@ __global__ void __launch_bounds__(256) k_fe_btd(FeArgs A) {
   constexpr int d = T::d, n = T::n, Q = T::Q;
   __shared__ PointTables s_p;
   stage_points<ET>(s_p, A.tab64);
-  const int64_t r = int64_t(blockIdx.x) * 256 + threadIdx.x;
-  if (r >= A.count * Q) return;
-  const int64_t t = r / Q;
-  double B[d * n];
-  point_b<ET>(A, s_p.dnds[r - t * Q], elem_of(A, t), B);
-  const int rows = ROWS ? ROWS : A.nb;
-  const double* D = A.in + r * rows * d;
-  double* o = A.out + r * rows * n;
-  // Bt_D (rows x n) = D (rows x d) * B (d x n)
-  if constexpr (ROWS > 0) {
-    double R[ROWS * n], Dr[ROWS * d];
+  const int64_t end = A.count * Q;
+  for (int64_t r = int64_t(blockIdx.x) * 256 + threadIdx.x; r < end; r += int64_t(gridDim.x) * 256) {
+    const int64_t t = r / Q;
+    double B[d * n];
+    point_b<ET>(A, s_p.dnds[r - t * Q], elem_of(A, t), B);
+    const int rows = ROWS ? ROWS : A.nb;
+    const double* D = A.in + r * rows * d;
+    double* o = A.out + r * rows * n;
+    // Bt_D (rows x n) = D (rows x d) * B (d x n)
+    if constexpr (ROWS > 0) {
+      double R[ROWS * n], Dr[ROWS * d];
 #pragma unroll
-    for (int k = 0; k < ROWS * d; ++k) Dr[k] = D[k];
-    matrix_matrix<ROWS, n, d>(Dr, B, R);
-    if constexpr (ROWS * n % 2 == 0) {
+      for (int k = 0; k < ROWS * d; ++k) Dr[k] = D[k];
+      matrix_matrix<ROWS, n, d>(Dr, B, R);
+      if constexpr (ROWS * n % 2 == 0) {
 #pragma unroll
-      for (int k = 0; k < ROWS * n / 2; ++k)
-        reinterpret_cast<double2*>(o)[k] = make_double2(R[2 * k], R[2 * k + 1]);
+        for (int k = 0; k < ROWS * n / 2; ++k)
+          reinterpret_cast<double2*>(o)[k] = make_double2(R[2 * k], R[2 * k + 1]);
+      } else {
+#pragma unroll
+        for (int k = 0; k < ROWS * n; ++k) o[k] = R[k];
+      }
     } else {
+      for (int i = 0; i < rows; ++i) {
+        double Di[d];
 #pragma unroll
-      for (int k = 0; k < ROWS * n; ++k) o[k] = R[k];
-    }
-  } else {
-    for (int i = 0; i < rows; ++i) {
-      double Di[d];
+        for (int l = 0; l < d; ++l) Di[l] = D[i + l * rows];
 #pragma unroll
-      for (int l = 0; l < d; ++l) Di[l] = D[i + l * rows];
+        for (int j = 0; j < n; ++j) {
+          double s = 0.;
 #pragma unroll
-      for (int j = 0; j < n; ++j) {
-        double s = 0.;
-#pragma unroll
-        for (int l = 0; l < d; ++l) s += Di[l] * B[l + j * d];
-        o[i + j * rows] = s;
+          for (int l = 0; l < d; ++l) s += Di[l] * B[l + j * d];
+          o[i + j * rows] = s;
+        }
       }
     }
   }
@@ -408,9 +410,10 @@ __global__ void __launch_bounds__(256) k_mat_gather(int64_t N, int d, int n, int
 
 inline void clear_error() { (void)hipGetLastError(); }
 inline unsigned grid_for(int64_t n) { return unsigned((n + 255) / 256); }
-// for kernels whose threads go on with a stride: within a launch's 2^32 threads
+// for kernels whose threads go on with a stride: within a launch's 2^32
+// threads, and many times what the chip runs at a time
 inline unsigned grid_striding(int64_t n) {
-  return unsigned(std::min<int64_t>((n + 255) / 256, 1 << 20));
+  return unsigned(std::min<int64_t>((n + 255) / 256, 1 << 16));
 }
 
 #define AKX_FE_SWITCH(et, F)              \
@@ -429,9 +432,10 @@ hipError_t launch_fe(int op, int et, hipStream_t s, const FeArgs& A) {
   if (A.count <= 0 && op != FE_LUMPED_ELEMENTS) return hipSuccess;
   const int n = et == TRI3 ? 3 : et == HEX8 ? 8 : 4;
   const int Q = et == QUAD4 ? 4 : et == HEX8 ? 8 : 1;
+  const unsigned points = grid_striding(A.count * Q);
   switch (op) {
   case FE_GRADIENT:
-#define F(ET) k_fe_gradient<ET><<<grid_for(A.count * Q), 256, 0, s>>>(A)
+#define F(ET) k_fe_gradient<ET><<<points, 256, 0, s>>>(A)
     AKX_FE_SWITCH(et, F)
 #undef F
     break;
@@ -441,12 +445,12 @@ hipError_t launch_fe(int op, int et, hipStream_t s, const FeArgs& A) {
 #undef F
     break;
   case FE_BTD:
-#define F(ET)                                                              \
-  switch (A.nb) {                                                          \
-  case 1: k_fe_btd<ET, 1><<<grid_for(A.count * Q), 256, 0, s>>>(A); break; \
-  case 2: k_fe_btd<ET, 2><<<grid_for(A.count * Q), 256, 0, s>>>(A); break; \
-  case 3: k_fe_btd<ET, 3><<<grid_for(A.count * Q), 256, 0, s>>>(A); break; \
-  default: k_fe_btd<ET, 0><<<grid_for(A.count * Q), 256, 0, s>>>(A);       \
+#define F(ET)                                                          \
+  switch (A.nb) {                                                      \
+  case 1: k_fe_btd<ET, 1><<<points, 256, 0, s>>>(A); break;            \
+  case 2: k_fe_btd<ET, 2><<<points, 256, 0, s>>>(A); break;            \
+  case 3: k_fe_btd<ET, 3><<<points, 256, 0, s>>>(A); break;            \
+  default: k_fe_btd<ET, 0><<<points, 256, 0, s>>>(A);                  \
   }
     AKX_FE_SWITCH(et, F)
 #undef F
