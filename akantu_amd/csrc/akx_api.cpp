@@ -785,14 +785,10 @@ int build_fused(akx_ctx* c, const std::vector<uint32_t>& order, const std::vecto
   HIP_TRY(c, dalloc(&c->fblk, blk.size()));
   HIP_TRY(c, hipMemcpy(c->fblk, blk.data(), blk.size() * 4, hipMemcpyHostToDevice));
   HIP_TRY(c, dalloc(&c->fel_off, el_off.size()));
-  HIP_TRY(c, dalloc(&c->fel, el.size()));
-  HIP_TRY(c, dalloc(&c->flslot, lslot.size()));
   HIP_TRY(c, dalloc(&c->fch_off, ch_off.size()));
   HIP_TRY(c, dalloc(&c->fcbase, cbase.size()));
   HIP_TRY(c, dalloc(&c->u_alt, size_t(N) * d));
   HIP_TRY(c, hipMemcpy(c->fel_off, el_off.data(), el_off.size() * 4, hipMemcpyHostToDevice));
-  HIP_TRY(c, hipMemcpy(c->fel, el.data(), el.size() * 4, hipMemcpyHostToDevice));
-  HIP_TRY(c, hipMemcpy(c->flslot, lslot.data(), lslot.size() * 2, hipMemcpyHostToDevice));
   HIP_TRY(c, hipMemcpy(c->fch_off, ch_off.data(), ch_off.size() * 4, hipMemcpyHostToDevice));
   HIP_TRY(c, hipMemcpy(c->fcbase, cbase.data(), cbase.size() * 2, hipMemcpyHostToDevice));
   c->fused_blocks = nblk;
@@ -820,6 +816,12 @@ int build_fused(akx_ctx* c, const std::vector<uint32_t>& order, const std::vecto
     // 240,000 45 / 53 at 4, hence the line between them, below the ratio where
     // the former would break even (1.6).
     c->fused_default = c->Q == 1 || double(el.size()) <= 1.4 * double(E);
+  } else {
+    // the mixed step through element ids; the records hold both lists
+    HIP_TRY(c, dalloc(&c->fel, el.size()));
+    HIP_TRY(c, dalloc(&c->flslot, lslot.size()));
+    HIP_TRY(c, hipMemcpy(c->fel, el.data(), el.size() * 4, hipMemcpyHostToDevice));
+    HIP_TRY(c, hipMemcpy(c->flslot, lslot.data(), lslot.size() * 2, hipMemcpyHostToDevice));
   }
   c->fused_ok = true;
   return AKX_OK;
