@@ -42,37 +42,41 @@ class HostCopier {
   // the stream.
   hipError_t to_host(int device, hipStream_t s, void* host, const void* dev, size_t bytes) {
     if (bytes == 0) return hipSuccess;
-    if (bytes > SLOT)
-      return run(device, bytes, [=](int lane, int lanes, size_t chunks) -> hipError_t {
+    hipError_t e;
+    if (bytes > SLOT) {
+      e = run(device, bytes, [=](int lane, int lanes, size_t chunks) -> hipError_t {
         return fetch(lane, lanes, chunks, s, static_cast<char*>(host),
                      static_cast<const char*>(dev), bytes);
       });
-    // one slot: the stream is waited for, which is 7 us less than an event
-    Slot& slot = lanes_[0][0];
-    hipError_t e = fillable(slot, s);
-    if (e == hipSuccess) e = hipMemcpyAsync(slot.mem, dev, bytes, hipMemcpyDeviceToHost, s);
-    if (e == hipSuccess) e = hipStreamSynchronize(s);
-    if (e != hipSuccess) return e;
-    std::memcpy(host, slot.mem, bytes);
-    for (auto& up : lanes_[0])
-      if (up.upload == s) up.upload = nullptr;
-    return hipSuccess;
+    } else {
+      // one slot: the stream is waited for, which is 7 us less than an event
+      Slot& slot = lanes_[0][0];
+      e = fillable(slot, s);
+      if (e == hipSuccess) e = hipMemcpyAsync(slot.mem, dev, bytes, hipMemcpyDeviceToHost, s);
+      if (e == hipSuccess) e = hipStreamSynchronize(s);
+      if (e == hipSuccess) {
+        std::memcpy(host, slot.mem, bytes);
+        for (auto& up : lanes_[0])
+          if (up.upload == s) up.upload = nullptr;
+      }
+    }
+    return e == hipErrorOutOfMemory ? plain(s, host, dev, bytes, hipMemcpyDeviceToHost) : e;
   }
   // Returns when the host array has been read; the device copy is ordered
   // before later work on the stream.
   hipError_t to_device(int device, hipStream_t s, void* dev, const void* host, size_t bytes) {
     if (bytes == 0) return hipSuccess;
+    hipError_t e;
     if (bytes > LARGE_UPLOAD)
-      return run(device, bytes, [=](int lane, int lanes, size_t chunks) -> hipError_t {
+      e = run(device, bytes, [=](int lane, int lanes, size_t chunks) -> hipError_t {
         return send(lane, lanes, chunks, s, static_cast<char*>(dev),
                     static_cast<const char*>(host), bytes);
       });
-    if (bytes > SLOT) {
-      const hipError_t e = hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, s);
-      return e == hipSuccess ? hipStreamSynchronize(s) : e;
-    }
-    // an event costs 5 us, as much as the transfer of a small array
-    return send_slot(lanes_[0][turn_ ^= 1], s, dev, host, bytes, bytes > SMALL);
+    else if (bytes > SLOT)
+      return plain(s, dev, host, bytes, hipMemcpyHostToDevice);
+    else  // an event costs 5 us, as much as the transfer of a small array
+      e = send_slot(lanes_[0][turn_ ^= 1], s, dev, host, bytes, bytes > SMALL);
+    return e == hipErrorOutOfMemory ? plain(s, dev, host, bytes, hipMemcpyHostToDevice) : e;
   }
 
  private:
@@ -103,10 +107,18 @@ class HostCopier {
     return e;
   }
   static hipError_t allocated(Slot& s) {
-    if (s.mem) return hipSuccess;
-    const hipError_t e = hipHostMalloc(&s.mem, SLOT, hipHostMallocDefault);
-    if (e != hipSuccess) s.mem = nullptr;
-    return e;
+    if (s.mem || hipHostMalloc(&s.mem, SLOT, hipHostMallocDefault) == hipSuccess)
+      return hipSuccess;
+    s.mem = nullptr;
+    (void)hipGetLastError();
+    return hipErrorOutOfMemory;
+  }
+  // the runtime's own copy: where it is the faster one, and where there is no
+  // page-locked memory to be had
+  static hipError_t plain(hipStream_t s, void* to, const void* from, size_t bytes,
+                          hipMemcpyKind kind) {
+    const hipError_t e = hipMemcpyAsync(to, from, bytes, kind, s);
+    return e == hipSuccess ? hipStreamSynchronize(s) : e;
   }
   static hipError_t with_event(Slot& s) {
     if (s.done) return hipSuccess;
