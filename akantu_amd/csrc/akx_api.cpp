@@ -871,7 +871,7 @@ RowMap element_rows(const akx_ctx* c) { return {c->elem_inv_d, c->elem_inv.data(
 
 // Up to HOST_ROWS bytes are renumbered on the host, beside a copy of 12 to 22
 // us, rather than by a launch (a nodal field to the host, host / device: 17 KB
-// 12 / 24 us, 115 KB 22 / 29, 217 KB 32.5 / 32.5; by the device array's size).
+// 12 / 24 us, 115 KB 22 / 29; by the device array's size).
 constexpr size_t HOST_ROWS = size_t(128) << 10;
 
 // Rows of `width` doubles between a caller array in its own numbering and a

@@ -1,17 +1,17 @@
 // akx_copy.hpp -- copies between a caller's pageable host arrays and the
 // device for the calls that return or take host data.
 //
-// To the host, the runtime's own pageable copies reach 18 GB/s on a card whose
-// link carries 57: it stages or pins the pages on the calling thread, in turn
-// with the transfer, and a caller's fresh array is mapped page by page on the
-// way.  Here the data pass through small page-locked slots, two per helper
-// thread: a slot travels while the other is copied, and large copies use
-// several threads, since one thread alone fills fresh pages at 13 GB/s (41 MB
-// into a fresh array: 4.2 ms by hipMemcpy).  To the device the runtime's copy
-// is the faster one between 1 and 24 MB (16 MB: 0.47 ms, 0.61 through slots);
-// below, one slot spares the pinning of the caller's pages (256 KB: 26 us, 28
-// to 130), and above, the threads gain (B^T D with an operand of 18 MB 2.37 ms
-// by the runtime's copy, 2.46 by slots; 35 MB 4.84 and 4.71).
+// The runtime's own pageable copies reach 18 GB/s to the host and 30 GB/s to
+// the device on a card whose link carries 57: it stages the pages or pins them
+// on the calling thread, in turn with the transfer, and a caller's fresh array
+// is mapped page by page on the way.  Pages that it has pinned also make later
+// calls slow that map or free memory near them: with uploads of 1 to 24 MB
+// taken straight from the caller's arrays a process of many operators paid 1.47
+// ms for a gradient of 9 MB that takes 0.38 through slots.  Here the data pass
+// through small page-locked slots, two per helper thread: a slot travels while
+// the other is copied, and large copies use several threads, since one thread
+// alone fills fresh pages at 13 GB/s (41 MB into a fresh array: 4.2 ms by
+// hipMemcpy).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -49,11 +49,19 @@ class HostCopier {
                      static_cast<const char*>(dev), bytes);
       });
     } else {
-      // one slot: the stream is waited for, which is 7 us less than an event
       Slot& slot = lanes_[0][0];
       e = fillable(slot, s);
+      // An event tells the end, but for small transfers by DMA, where it costs
+      // 8 us (17 KB 12 us with the stream's wait).  Up to BY_KERNEL the stream's
+      // wait is the slower one behind many launches (12: 72 us, 50 by event),
+      // and above SMALL the calls that follow it were (operators on 26,970
+      // hexahedra 3.85 ms, 3.79 by events).
+      const bool event = bytes <= BY_KERNEL || bytes > SMALL;
+      if (e == hipSuccess && event) e = with_event(slot);
+      if (e == hipSuccess && bytes > SMALL) e = hipEventSynchronize(slot.done);  // see run
       if (e == hipSuccess) e = hipMemcpyAsync(slot.mem, dev, bytes, hipMemcpyDeviceToHost, s);
-      if (e == hipSuccess) e = hipStreamSynchronize(s);
+      if (e == hipSuccess && event) e = hipEventRecord(slot.done, s);
+      if (e == hipSuccess) e = event ? hipEventSynchronize(slot.done) : hipStreamSynchronize(s);
       if (e == hipSuccess) {
         std::memcpy(host, slot.mem, bytes);
         for (auto& up : lanes_[0])
@@ -67,13 +75,11 @@ class HostCopier {
   hipError_t to_device(int device, hipStream_t s, void* dev, const void* host, size_t bytes) {
     if (bytes == 0) return hipSuccess;
     hipError_t e;
-    if (bytes > LARGE_UPLOAD)
+    if (bytes > SLOT)
       e = run(device, bytes, [=](int lane, int lanes, size_t chunks) -> hipError_t {
         return send(lane, lanes, chunks, s, static_cast<char*>(dev),
                     static_cast<const char*>(host), bytes);
       });
-    else if (bytes > SLOT)
-      return plain(s, dev, host, bytes, hipMemcpyHostToDevice);
     else  // an event costs 5 us, as much as the transfer of a small array
       e = send_slot(lanes_[0][turn_ ^= 1], s, dev, host, bytes, bytes > SMALL);
     return e == hipErrorOutOfMemory ? plain(s, dev, host, bytes, hipMemcpyHostToDevice) : e;
@@ -82,7 +88,8 @@ class HostCopier {
  private:
   static constexpr size_t SLOT = size_t(1) << 20;
   static constexpr size_t SMALL = size_t(128) << 10;
-  static constexpr size_t LARGE_UPLOAD = size_t(24) << 20;
+  // up to here the runtime fills page-locked memory by a kernel, above by DMA
+  static constexpr size_t BY_KERNEL = size_t(16) << 10;
   static constexpr int LANES = 4;
   struct Slot {
     void* mem = nullptr;
@@ -90,7 +97,7 @@ class HostCopier {
     hipStream_t upload = nullptr;  // a small upload may be reading the slot
   };
   Slot lanes_[LANES][2];
-  int turn_ = 0;  // slot of the next upload
+  int turn_ = 0;  // slot of the last upload
 
   // One lane up to 8 MB: inference of 200,003 points (5.6 MB each way) takes
   // 0.66 ms with one or two, and starting threads costs a first call 0.4 ms.
@@ -113,8 +120,7 @@ class HostCopier {
     (void)hipGetLastError();
     return hipErrorOutOfMemory;
   }
-  // the runtime's own copy: where it is the faster one, and where there is no
-  // page-locked memory to be had
+  // the runtime's own copy, where there is no page-locked memory to be had
   static hipError_t plain(hipStream_t s, void* to, const void* from, size_t bytes,
                           hipMemcpyKind kind) {
     const hipError_t e = hipMemcpyAsync(to, from, bytes, kind, s);
@@ -214,6 +220,7 @@ class HostCopier {
       if (hipError_t e = send_slot(lanes_[lane][j], s, dev + k * SLOT, host + k * SLOT, n, true))
         return e;
     }
+    if (lane == 0) turn_ = j ^ 1;  // the next upload takes the slot used before the last
     return hipSuccess;
   }
 };

@@ -1,6 +1,6 @@
 """The copies between a caller's arrays and the device (akx_copy.hpp) on a host
 stand-in for the runtime whose copies happen as late as they may: sizes at the
-edges of the small, one-slot, direct and threaded copies, several uploads in a
+edges of the small, one-slot, one-lane and threaded copies, several uploads in a
 row, and page-locked memory that runs out at any point."""
 import os
 import subprocess
@@ -9,7 +9,7 @@ import pytest
 
 HERE = os.path.join(os.path.dirname(os.path.abspath(__file__)), "host")
 KB, MB = 1 << 10, 1 << 20
-EDGES = [1, 128 * KB, 128 * KB + 1, MB, MB + 1, 2 * MB + 5, 8 * MB, 8 * MB + 1, 24 * MB + 3]
+EDGES = [1, 16 * KB, 16 * KB + 1, 128 * KB, 128 * KB + 1, MB, MB + 1, 2 * MB + 5, 8 * MB, 8 * MB + 1, 17 * MB + 3]
 
 
 @pytest.fixture(scope="module")
