@@ -710,7 +710,7 @@ int build_fused(akx_ctx* c, const std::vector<uint32_t>& order, const std::vecto
   // 664,000 31.5 -> 28.2; 160,000 quadrangles 12.9 -> 10.5 (3 per CU 12.9);
   // 90,000 in 515 blocks 8.3, in 472 7.4.
   const int per_cu = n == 3 ? 8 : d == 3 || N > int64_t(512) * FUSED_NB ? 4 : 2;
-  const int64_t share = (N + 256 * per_cu - 1) / (256 * per_cu);
+  const int64_t share = (N + CARD_CUS * per_cu - 1) / (CARD_CUS * per_cu);
   const int64_t most = std::min<int64_t>(FUSED_NB, std::max<int64_t>(64, (share + 7) / 8 * 8));
   bool staged = true;
   int64_t next = most;  // what the last block took and a little more

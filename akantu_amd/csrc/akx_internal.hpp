@@ -111,11 +111,17 @@ struct NodeArgs {
 // the nodes [blk[b], blk[b + 1]), at most FUSED_NB, and recomputes the elements
 // around them in chunks of FUSED_CH, in the reference's assembly order.
 constexpr int FUSED_NB = 256, FUSED_CH = 256;
+// CUs of an MI355X that is not partitioned, which the rules for block counts
+// are measured on
+constexpr int CARD_CUS = 256;
 struct FusedArgs {
   const uint32_t* blk;     // [nblk + 1] first node of each block
   const uint32_t* el_off;  // [nblk + 1] offsets into el
-  const uint32_t* el;      // internal element ids of each block, assembly order
-  const uint16_t* lslot;   // [j * n + a] LDS slot of (element j, node a); 0xFFFF: not a block node
+  // read where the nodes are not staged: internal element ids of each block,
+  // assembly order, and [j * n + a] LDS slot of (element j, node a), 0xFFFF: not
+  // a block node
+  const uint32_t* el;
+  const uint16_t* lslot;
   const uint32_t* ch_off;  // [nblk + 1] first chunk table of each block
   const uint16_t* cbase;   // [chunk * (FUSED_NB + 1) + k] first slot of block node k in the chunk
   double* u_out;           // displacement written by the step (read from NodeArgs::u)
@@ -379,14 +385,15 @@ struct akx_ctx {
   int lcr_shift = 8;
   // node -> entries of the per-patch partial sums (slot layout 3)
   uint32_t *pcsr_off = nullptr, *pentry = nullptr, *ppos = nullptr;
-  // fused FP64 step (slot layout 6)
+  // fused steps (slot layout 6)
   bool fused_ok = false;
   int fused_lds = 0;
   int64_t fused_blocks = 0, fused_elements = 0;
   uint32_t *fel_off = nullptr, *fel = nullptr, *fch_off = nullptr;
   uint16_t *flslot = nullptr, *fcbase = nullptr;
-  // its FP64 form: halo nodes and element records (nullptr: too many nodes);
-  // fused_default: the FP64 path takes it when no layout is set
+  // halo nodes and element records of both precisions (nullptr: too many
+  // nodes to stage, the mixed step runs on fel and flslot, FP64 on slots);
+  // fused_default: the FP64 path takes the fused step when no layout is set
   bool fused_default = false;
   int fused_staged_lds = 0;
   uint32_t *fblk = nullptr, *fhalo_off = nullptr, *fhalo = nullptr;

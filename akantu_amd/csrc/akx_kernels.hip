@@ -1223,8 +1223,10 @@ __device__ __forceinline__ bool sur_strain_from_differences(const ElemArgs& A, i
 // before it asked for the node ids, and for places and bases after u and X.
 // 6 million tetrahedra (elastic): 66.6 -> 57.8 us for the element kernel, 91.3
 // -> 83.7 us for the step; 2.1 million hexahedra (neo-Hookean, 405 nodes per
-// patch, now packed) 146 -> 137 us; 1.6 million triangles 19.4 -> 15.2 us.  What
-// is left is bound by FP32 and FP64 issue at 8 waves per SIMD.
+// patch, now packed) 146 -> 137 us; 1.6 million triangles 19.4 -> 15.2 us.  Of
+// the cycles in which a CU has waves, LDS is busy 91 % (over half of it bank
+// conflicts) and the vector pipe 85 % on the tetrahedra: what is left is bound
+// by the two.
 template <int ET, int KIND, int HALVES>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8)))
 k_element_patch(ElemArgs A) {
@@ -1856,12 +1858,13 @@ __global__ void __launch_bounds__(256) k_node(NodeArgs A) {
 
 // ===========================================================================
 // fused FP64 step over node blocks (stateless laws, slot layout 6)
-//   Block b owns FUSED_NB consecutive nodes.  The elements touching them are
-//   listed per block in the reference's assembly order; the block walks that
-//   list in chunks of FUSED_CH elements: every thread computes one element's
-//   forces (element_forces_fp64, the element kernel's arithmetic), writes the
-//   contributions to the block's own nodes into LDS at their place in the
-//   node's run for this chunk, and each node thread adds its run in order --
+//   Block b owns consecutive nodes, at most FUSED_NB and as few as build_fused
+//   cut it to.  The elements touching them are listed per block in the
+//   reference's assembly order; the block walks that list in chunks of FUSED_CH
+//   elements: every thread computes one element's forces (element_forces_fp64,
+//   the element kernel's arithmetic), writes the contributions to the block's
+//   own nodes into LDS at their place in the node's run for this chunk, and
+//   each node thread adds its run in order --
 //   the chunks follow the assembly order, so every node's sum is the same
 //   sequence of additions as the slot path's.  Then each node thread runs the
 //   node kernel's update on its node.  Elements on block boundaries are

@@ -886,9 +886,9 @@ hipError_t launch_sur_mlp(hipStream_t s, const void* img, const float* imgb, boo
   // 2), 160,320 42.9 / 40.7 (3, 2), 4.03 M 587 / 578 (62, 42), where 12 reach
   // 1.04 PFLOP/s.
   const int64_t tiles = (n + 31) / 32;
-  auto rounds = [&](int waves) { return (tiles + 256 * waves - 1) / (256 * waves); };
+  auto rounds = [&](int waves) { return (tiles + CARD_CUS * waves - 1) / (CARD_CUS * waves); };
   const int waves = rounds(12) * 4 < rounds(8) * 3 ? 12 : 8;
-  const unsigned g = unsigned(std::min<int64_t>(256, (tiles + waves - 1) / waves));
+  const unsigned g = unsigned(std::min<int64_t>(CARD_CUS, (tiles + waves - 1) / waves));
   if (bf16)
     k_sur_infer<Bf16><<<g, 64 * waves, 0, s>>>(static_cast<const Bf16::x8*>(img), imgb, n, x, sx,
                                                y, sy);

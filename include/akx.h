@@ -217,7 +217,9 @@ int akx_synchronize(akx_ctx* ctx);
 
 /* Per-kernel timing with HIP events recorded on the context's stream around
  * every element and node kernel of akx_solve_step (off by default).
- * akx_last_step_timing returns the averages over the last akx_solve_step, ms. */
+ * akx_last_step_timing returns the averages over the last akx_solve_step, ms (a
+ * fused step, one launch, is all element time: the node's is the gap between
+ * two events). */
 int akx_enable_timing(akx_ctx* ctx, int on);
 int akx_last_step_timing(akx_ctx* ctx, double* element_ms, double* node_ms);
 
