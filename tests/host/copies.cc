@@ -1,6 +1,7 @@
 // Uploads in a row, each from the same host array that is overwritten as soon as
 // the call returns, then downloads: every device array holds what it was sent.
 // Arguments: page-locked buffers to be had, then sizes in bytes.
+#include <algorithm>
 #include <cstdio>
 
 #include "../../akantu_amd/csrc/akx_copy.hpp"
